@@ -20,24 +20,30 @@
 // the fp32 normalized activations are cast to fp16 once per call
 // (rv_cast_f32_f16) -- the cast autocast's F.linear performs.
 //
-// Tiling: a workgroup of 4 waves (2 x 2) owns a BM x BN tile of C; each wave
-// owns (BM/2) x (BN/2) = TM x TN tiles of 32 x 32 computed with
-// v_mfma_f32_32x32x16_f16.  K advances 64 per stage through two LDS buffers:
-// the next stage's global loads are issued before the current stage's MFMAs
-// and written to the other buffer afterwards; one barrier per stage.
-// Tile sizes 256x256, 128x256, 128x128 and 64x128 are chosen per shape (the
-// largest one that still gives about one workgroup per CU); the choice does
-// not change any result bit, because every output element sums its k blocks
-// in the same order in every tile shape.  Weight gradients over few output
-// tiles may split the token reduction (split-K) into fp32 partials summed by a
-// second kernel in a fixed order.
+// Tiling: a workgroup of 4 (2 x 2) or 8 (2 x 4) waves owns a BM x BN tile of
+// C; each wave owns TM x TN tiles of 32 x 32 computed with
+// v_mfma_f32_32x32x16_f16.  K advances BK (64 or 32) per stage through rings of
+// LDS buffers that direct-to-LDS loads fill one to three stages ahead; one
+// barrier per stage.  The tile shapes (kShapes) are timed per problem (see
+// tune_act); the choice does not change any result bit, because every output
+// element sums its k blocks in the same order in every tile shape.  Weight
+// gradients over few output tiles may split the token reduction (split-K)
+// into fp32 partials summed by a second kernel in a fixed order.
 //
-// LDS layouts (bank-conflict free for the fragment reads):
-//   KC  row stride 72 halves (144 B): the 16 rows a ds_read_b128 pass touches
-//       start at 16 distinct 4-bank groups.
-//   RC  row (= k) stride chosen so that its byte size is 64 mod 256: the four
-//       k rows one 32-lane pass of ds_read_b64_tr_b16 touches fill 4 disjoint
-//       64-byte bank ranges.
+// LDS layouts: XOR swizzles of the 16-byte chunk index inside a row, bank
+// conflict free for the fragment reads in both a 32- and a 64-bank model
+// (f_kc, f_rc).
+//
+// What bounds the main loop (256 x 256 tile, m = 32768, n = 1024, k = 8192, B an
+// RC source; timing copies with one part taken out): MFMA alone 248 us, MFMA
+// and fragment reads 302, the loads alone 253, MFMA and loads 337, all three
+// 429-437, i.e. 1.26-1.28 PFLOP/s; the same with every load an L2 hit: 423.  The
+// LDS carries 64 KB of fragment reads and 32 KB of DMA writes per 32 k (512
+// cycles each at 128 and 64 B/clk) against 1024 MFMA cycles, and with one wave
+// per SIMD a read or a load that finds its queue full holds up the MFMAs
+// behind it.  Before: 64-byte segments of the KC rows per stage, loads and reads
+// in bursts, per-load vector address arithmetic and one wait for all of a k
+// step's reads: 479-487 us.
 //
 // MFMA 32x32x16 lane layout (gfx950): lane l supplies A row / B row (l % 32)
 // with k = (l/32)*8 + 0..7; accumulator value j of lane l is
@@ -55,6 +61,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <utility>
 
 #include "rv_device.h"
 
@@ -67,30 +74,36 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));  // 16-byte staging word
 #define RV_LDS __attribute__((address_space(3)))
 
-constexpr int kThreads = 256;
-constexpr int kBK = 32;             // k per pipeline stage
-#ifndef RV_ST_256x256
-#define RV_ST_256x256 4
-#endif
-#ifndef RV_ST_128x256
-#define RV_ST_128x256 3
-#endif
-#ifndef RV_ST_128x128
-#define RV_ST_128x128 4
-#endif
-#ifndef RV_ST_64x128
-#define RV_ST_64x128 4
-#endif
-// depth of the LDS ring per tile shape
-constexpr int stages_for(int bm, int bn) {
-  return bm == 256 ? RV_ST_256x256 : bn == 256 ? RV_ST_128x256 : bm == 128 ? RV_ST_128x128 : RV_ST_64x128;
-}
+// Tile shapes: BM x BN tile, waves, k per pipeline stage (one or half a
+// 128-byte line of a KC row), depth of the two operands' LDS rings, workgroups
+// per CU that the rings leave room for.  One workgroup per CU has the least
+// LDS and L2 traffic per MFMA; two or three overlap one's epilogue with the
+// others' MFMAs, and small problems need the smaller tiles.  Each is the
+// fastest of the seven somewhere (us, m x d x f): 256 x 256 dx 32768x1024x4096
+// 429 (the others 450-715), with 8 waves up 497 (522-743); 128 x 256 dgate
+// 32768x1024x4096 382 (412-497); 128 x 128 with BK 64 dx 16896x256x1024 27.2
+// (31.8-42), with BK 32 up + u 33.6 (35-47); 64 x 128 at two per CU dx of 51 rows
+// 11.6 (12.6-43), at three proj 16896x256 7.1 (7.5-11).
+struct TileShape {
+  int bm, bn, waves, bk, ra, rb, per_cu;
+};
+// The first kRuleShapes are the ones pick_act's rule and the weight-gradient
+// plan choose from; the tuner also times the rest.
+constexpr int kNumShapes = 7, kRuleShapes = 4;
+constexpr TileShape kShapes[kNumShapes] = {
+    {256, 256, 4, 64, 3, 2, 1}, {128, 256, 4, 32, 3, 3, 2}, {128, 128, 4, 64, 3, 2, 2},
+    {64, 128, 4, 64, 4, 3, 2},  {256, 256, 8, 64, 3, 2, 1}, {128, 128, 4, 32, 3, 3, 3},
+    {64, 128, 4, 64, 2, 2, 3}};
 constexpr int kCUs = 256;           // MI355X compute units (tile-shape choice only)
 constexpr int kRsrcWord3 = 0x00020000;  // raw buffer resource, gfx9 data format
 
 // XOR swizzles of the 16-byte chunk index inside one LDS row (see the layout
 // notes at the top of the file).
-__device__ __forceinline__ int f_kc(int row) { return ((row >> 2) & 3) ^ (row & 2); }
+template <int BK>
+__device__ __forceinline__ int f_kc(int row) {
+  if constexpr (BK == 64) return (row & 7) ^ ((row >> 3) & 1);
+  else return ((row >> 2) & 3) ^ (row & 2);
+}
 template <int ROWS>
 __device__ __forceinline__ int f_rc(int k) {
   return ((ROWS >= 128 ? 0xCA60 : 0x6420) >> ((k & 3) * 4)) & 0xF;
@@ -136,115 +149,155 @@ struct MapGateValue {
   }
 };
 
+// A wave-uniform 64-bit value in scalar registers: a value that reaches a buffer
+// resource through vector registers costs a loop around every load.
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32));
+  return (int64_t)((uint64_t)hi << 32 | lo);
+}
+
 // ---------------------------------------------------------------------------
 // Global -> LDS copies: direct-to-LDS buffer loads (buffer_load_dwordx4 ...
 // lds).  One wave instruction fills 1 KB of LDS, lane L's 16 bytes at byte
 // 16 L; each lane loads the source chunk whose swizzled LDS slot that is.
-// A tile of ROWS rows is ROWS * 64 bytes per stage (kBK = 32 halves per row,
-// or 32 k rows of ROWS halves), i.e. ROWS / 16 wave instructions, ROWS / 64
-// per wave.  Per-lane source offsets are fixed; each stage adds a constant.
+// A tile of ROWS rows is ROWS * 2 BK bytes per stage (BK halves per row, or
+// BK k rows of ROWS halves), i.e. ROWS BK / 512 wave instructions.  A lane's source offsets are fixed for the whole kernel; a
+// stage moves the buffer resource's base instead (scalar arithmetic only), and
+// the resource ends with the operand, so k rows past the end of an RC source
+// read as zero, and a resource of zero bytes (a stage past the end) reads
+// nothing and writes zeros.
 // ---------------------------------------------------------------------------
-template <bool RC, int ROWS, int WAVES>
+template <bool RC, int ROWS, int BK, int WAVES>
 struct Dma {
-  static constexpr int kPerWave = ROWS / 16 / WAVES;
+  static constexpr int kPerWave = ROWS * BK / 512 / WAVES;
+  static constexpr int kChunks = BK / 8;            // 16-byte chunks per KC row
+  static constexpr int kRows = 64 / kChunks;        // KC rows per wave instruction
   uint32_t off[kPerWave];  // byte offset of this lane's chunk at k = 0 of the kernel's range
-  uint32_t kstep;          // bytes per stage
-  __amdgpu_buffer_rsrc_t rsrc;
+  int64_t base;            // address of the kernel's first k
+  int64_t left;            // bytes from base to the operand's end
+  int64_t kstep;           // bytes per stage
 
   // KC source [rows][ld] (k contiguous), tile rows row0..; rows past `rows`
   // are clamped (their results are never stored); map() gathers B rows.
   template <class Map>
-  __device__ __forceinline__ void init_kc(const __half* base, int64_t bytes, int64_t ld,
-                                          const Map& map, int64_t kbeg) {
-    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(base), 0, (int)bytes, kRsrcWord3);
-    kstep = kBK * 2;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __device__ __forceinline__ void init_kc(const __half* p, int64_t bytes, int64_t ld,
+                                          const Map& map, int64_t kbeg, int wave, int lane) {
+    base = uniform(reinterpret_cast<int64_t>(p + kbeg));
+    left = uniform(bytes - kbeg * 2);
+    kstep = BK * 2;
 #pragma unroll
     for (int it = 0; it < kPerWave; ++it) {
-      const int b = (it * WAVES + wave) * 1024 + lane * 16;
-      const int row = b >> 6, chunk = ((b >> 4) & 3) ^ f_kc(row);
-      off[it] = (uint32_t)((map(row) * ld + kbeg + chunk * 8) * 2);
+      const int row = (it * WAVES + wave) * kRows + lane / kChunks;
+      off[it] = (uint32_t)((map(row) * ld + ((lane % kChunks) ^ f_kc<BK>(row)) * 8) * 2);
     }
   }
-  // RC source [k][ld] (tile rows contiguous from row0); k rows past the
-  // resource's end read as zero (the buffer range check).
-  __device__ __forceinline__ void init_rc(const __half* base, int64_t bytes, int64_t ld,
-                                          int64_t row0, int64_t kbeg) {
-    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(base), 0, (int)bytes, kRsrcWord3);
-    kstep = (uint32_t)(kBK * ld * 2);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // RC source [k][ld], tile rows contiguous from row0.
+  __device__ __forceinline__ void init_rc(const __half* p, int64_t bytes, int64_t ld,
+                                          int64_t row0, int64_t kbeg, int wave, int lane) {
+    base = uniform(reinterpret_cast<int64_t>(p + kbeg * ld + row0));
+    left = uniform(bytes - (kbeg * ld + row0) * 2);
+    kstep = BK * ld * 2;
 #pragma unroll
     for (int it = 0; it < kPerWave; ++it) {
       const int b = (it * WAVES + wave) * 1024 + lane * 16;
       const int krow = b / (ROWS * 2), chunk = ((b % (ROWS * 2)) >> 4) ^ f_rc<ROWS>(krow);
-      off[it] = (uint32_t)(((kbeg + krow) * ld + row0 + chunk * 8) * 2);
+      off[it] = (uint32_t)((krow * ld + chunk * 8) * 2);
     }
   }
-  // Issue wave instruction `it` of stage `st` into the tile at `lds`; with
-  // live = false the offset is beyond any buffer's range (2 GiB > the
-  // largest operand the entry points accept): no memory is read and the
-  // lanes write zeros.
-  __device__ __forceinline__ void issue_one(_Float16* lds, int st, int it, bool live) const {
-    const int wave = threadIdx.x >> 6;
-    const uint32_t voff = live ? off[it] + (uint32_t)st * kstep : 0x80000000u;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rsrc, (RV_LDS void*)(lds + (it * WAVES + wave) * 512), 16, voff, 0, 0, 0);
-  }
-  // Issue stage `st` (relative to the kernel's first k) into the tile at `lds`.
-  __device__ __forceinline__ void issue(_Float16* lds, int st) const {
-    const int wave = threadIdx.x >> 6;
+  // A KC row's last stage holds `valid` < BK values of the reduction: chunks
+  // at or past it are sent out of the resource's range (2 GiB > the largest
+  // operand the entry points accept) and read as zero.
+  __device__ __forceinline__ void cut_kc(int valid, int wave, int lane) {
 #pragma unroll
-    for (int it = 0; it < kPerWave; ++it)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc, (RV_LDS void*)(lds + (it * WAVES + wave) * 512), 16, off[it] + (uint32_t)st * kstep,
-          0, 0, 0);
+    for (int it = 0; it < kPerWave; ++it) {
+      const int row = (it * WAVES + wave) * kRows + lane / kChunks;
+      if (((lane % kChunks) ^ f_kc<BK>(row)) * 8 >= valid) off[it] = 0x80000000u;
+    }
+  }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t stage(int st, bool live) const {
+    const int64_t at = (int64_t)st * kstep, n = left - at;
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(base + at), 0,
+                                             live && n > 0 ? (int)n : 0, kRsrcWord3);
+  }
+  // Wave instruction `it` of a stage into the tile at `lds`.
+  __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rsrc, _Float16* lds, int it,
+                                        int wave) const {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rsrc, (RV_LDS void*)(lds + (it * WAVES + wave) * 512), 16, off[it], 0, 0, 0);
   }
 };
 
 // ---------------------------------------------------------------------------
 // MFMA fragments: lane l -> tile row r0 + l%32, k = ks*16 + (l/32)*8 + 0..7.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ f16x8 frag_kc(const _Float16* lds, int r0, int ks, int lane) {
-  const int row = r0 + (lane & 31);
-  const int chunk = ks * 2 + (lane >> 5);
-  return *reinterpret_cast<const f16x8*>(lds + row * kBK + ((chunk ^ f_kc(row)) << 3));
-}
-
-// ds_read_b64_tr_b16 as inline assembly: through the builtin, the compiler
-// cannot tell the read from the in-flight LDS DMA writes and drains every
-// outstanding DMA (vmcnt(0)) before each one.  Its result is therefore not
-// tracked by the compiler's LDS counter: the k-step code waits for it
-// explicitly (lds_ready) before the MFMAs that use it.
-__device__ __forceinline__ i16x4 tr_read(const _Float16* p) {
+// The LDS reads are inline assembly: through the builtin (and ordinary loads)
+// the compiler cannot always tell them from the in-flight LDS DMA writes and
+// drains every outstanding DMA (vmcnt(0)) before them.  Their results are
+// therefore not tracked by the compiler's LDS counter: the k-step code waits
+// for them explicitly (lds_wait) before the MFMAs that use them.
+template <int OFF>
+__device__ __forceinline__ i16x4 tr_read(uint32_t addr) {
+  static_assert(OFF >= 0 && OFF < 65536, "LDS instruction offset");
   i16x4 r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1"
-               : "=v"(r)
-               : "v"((uint32_t)(size_t)(RV_LDS const void*)p));
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
+  return r;
+}
+template <int OFF>
+__device__ __forceinline__ f16x8 b128_read(uint32_t addr) {
+  static_assert(OFF >= 0 && OFF < 65536, "LDS instruction offset");
+  f16x8 r;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
   return r;
 }
 
-template <int ROWS>
-__device__ __forceinline__ f16x8 frag_rc(const _Float16* lds, int r0, int ks, int lane) {
-  const int g = lane >> 4, i = lane & 15;
-  const int m = r0 + (g & 1) * 16 + 4 * (i & 3);
-  const int k = ks * 16 + (g >> 1) * 8 + (i >> 2);
-  const int k4 = k + 4;
-  const i16x4 lo = tr_read(lds + k * ROWS + ((f_rc<ROWS>(k) ^ (m >> 3)) << 3) + (m & 7));
-  const i16x4 hi = tr_read(lds + k4 * ROWS + ((f_rc<ROWS>(k4) ^ (m >> 3)) << 3) + (m & 7));
-  const f16x4 a = __builtin_bit_cast(f16x4, lo), b = __builtin_bit_cast(f16x4, hi);
-  return f16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-}
+// A lane's LDS byte addresses of one operand's fragments inside a stage, for
+// the wave's rows r0 .. r0 + 32 N - 1: everything but the stage's base and the
+// k step.  KC: one address (row r0 + l%32); row block P adds 64 BK P bytes, k
+// step ks flips the bits 32 ks (the chunk index is XOR-swizzled).  RC: one
+// address per row block (the swizzle reaches the row block's bits); k step ks
+// adds 32 ks ROWS bytes, the second half of a fragment (k + 4) 8 ROWS bytes.
+template <bool RC, int ROWS, int BK, int N>
+struct Frags {
+  static constexpr int kReads = RC ? 2 : 1;  // LDS instructions per fragment
+  uint32_t at[RC ? N : 1];
+  __device__ __forceinline__ void init(int r0, int lane) {
+    if constexpr (RC) {
+      const int g = lane >> 4, i = lane & 15;
+      const int k = (g >> 1) * 8 + (i >> 2);
+#pragma unroll
+      for (int p = 0; p < N; ++p) {
+        const int m = r0 + p * 32 + (g & 1) * 16 + 4 * (i & 3);
+        at[p] = (uint32_t)(k * ROWS * 2 + ((f_rc<ROWS>(k) ^ (m >> 3)) << 4) + (m & 7) * 2);
+      }
+    } else {
+      const int row = r0 + (lane & 31);
+      at[0] = (uint32_t)(row * BK * 2 + (((lane >> 5) ^ f_kc<BK>(row)) << 4));
+    }
+  }
+  // Fragment P of k step KS from the operand's tile at LDS byte `tile`.
+  template <int P, int KS>
+  __device__ __forceinline__ f16x8 read(uint32_t tile) const {
+    if constexpr (RC) {
+      const i16x4 lo = tr_read<KS * 32 * ROWS>(tile + at[P]);
+      const i16x4 hi = tr_read<KS * 32 * ROWS + 8 * ROWS>(tile + at[P]);
+      const f16x4 a = __builtin_bit_cast(f16x4, lo), b = __builtin_bit_cast(f16x4, hi);
+      return f16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    } else {
+      return b128_read<P * 64 * BK>((tile + at[0]) ^ (KS * 32));
+    }
+  }
+};
 
-// Wait for every LDS read of this wave, and pass a fragment through an empty
+// Wait until at most N of this wave's LDS instructions are outstanding (they
+// complete in order); wait for all of them; and pass a fragment through an empty
 // asm after that wait so that its users cannot be scheduled before it.
+template <int N>
+__device__ __forceinline__ void lds_wait() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N < 15 ? N : 15) : "memory");
+}
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void after_wait(f16x8& v) { asm volatile("" : "+v"(v)); }
-
-template <bool RC, int ROWS>
-__device__ __forceinline__ f16x8 frag(const _Float16* lds, int r0, int ks, int lane) {
-  if constexpr (RC) return frag_rc<ROWS>(lds, r0, ks, lane);
-  else return frag_kc(lds, r0, ks, lane);
-}
 
 // ---------------------------------------------------------------------------
 // The GEMM kernel.
@@ -258,11 +311,13 @@ enum class Epi {
   PartialF32,     // c fp32 partial [split][m][n] = acc
 };
 
+constexpr int kSplitStep = 64;  // weight gradients: granularity of a split's token range
+
 struct GemmArgs {
   const __half* a; int64_t lda; int64_t a_bytes;   // source, row stride, bytes addressable
   const __half* b; int64_t ldb; int64_t b_bytes;
   int64_t m, n, k;         // C rows, C columns (B rows), reduction length
-  int64_t k_chunk;         // tokens per split (multiple of kBK); == k without split
+  int64_t k_chunk;         // tokens per split (multiple of kSplitStep); == k without split
   int64_t tiles_m, tiles_n;
   void* c; int64_t ldc;
   void* u; int64_t ldu;    // SwiGLU: optional u output; SwiGLUBwd: u input
@@ -286,19 +341,33 @@ __device__ __forceinline__ void tile_of(int64_t t, int64_t tiles_m, int64_t tile
   tn = r / gm;
 }
 
-template <int BM, int BN, bool A_RC, bool B_RC, Epi EPI, int WAVES>
-__global__ __launch_bounds__(WAVES * 64)
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): loops whose
+// index has to be a constant expression.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+template <int SHAPE, bool A_RC, bool B_RC, Epi EPI>
+__global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
+                             kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
 void gemm_kernel(GemmArgs args) {
+  constexpr int BM = kShapes[SHAPE].bm, BN = kShapes[SHAPE].bn, WAVES = kShapes[SHAPE].waves;
+  constexpr int BK = kShapes[SHAPE].bk, RA = kShapes[SHAPE].ra, RB = kShapes[SHAPE].rb;
   // waves: 2 rows x WCOLS columns, each owning a WM x WN block of the tile
   constexpr int WCOLS = WAVES / 2, WM = BM / 2, WN = BN / WCOLS;
   constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int kStages = stages_for(BM, BN);
-  constexpr int kA = BM * kBK, kB = BN * kBK;          // halves per stage and operand
-  constexpr int kRing = kStages * (kA + kB);
+  static_assert(RB >= 2 && (RA == RB || RA == RB + 1), "ring depths");
+  constexpr int kA = BM * BK, kB = BN * BK;      // halves per stage and operand
+  constexpr int kRing = RA * kA + RB * kB;
   constexpr int kStaging = WAVES * WM * (WN + 8);  // fp16 epilogue staging
-  __shared__ __attribute__((aligned(16))) _Float16 lds[kRing > kStaging ? kRing : kStaging];
+  __shared__ __attribute__((aligned(1024))) _Float16 lds[kRing > kStaging ? kRing : kStaging];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WCOLS, wn = wave % WCOLS;
 
   const int64_t tiles = args.tiles_m * args.tiles_n;
@@ -309,16 +378,19 @@ void gemm_kernel(GemmArgs args) {
   const int64_t n0 = (EPI == Epi::SwiGLU) ? tn * (BN / 2) : tn * BN;
   const int64_t kbeg = split * args.k_chunk;
   const int64_t kend = kbeg + args.k_chunk < args.k ? kbeg + args.k_chunk : args.k;
-  const int stages = kend > kbeg ? (int)((kend - kbeg + kBK - 1) / kBK) : 0;
+  const int stages =
+      __builtin_amdgcn_readfirstlane(kend > kbeg ? (int)((kend - kbeg + BK - 1) / BK) : 0);
+  const int ktail = (int)((kend - kbeg) % BK);  // values of a last, partial stage
 
-  Dma<A_RC, BM, WAVES> da;
-  Dma<B_RC, BN, WAVES> db;
-  if constexpr (A_RC) da.init_rc(args.a, args.a_bytes, args.lda, m0, kbeg);
-  else da.init_kc(args.a, args.a_bytes, args.lda, MapDirect{m0, args.m}, kbeg);
-  if constexpr (B_RC) db.init_rc(args.b, args.b_bytes, args.ldb, n0, kbeg);
+  Dma<A_RC, BM, BK, WAVES> da;
+  Dma<B_RC, BN, BK, WAVES> db;
+  if constexpr (A_RC) da.init_rc(args.a, args.a_bytes, args.lda, m0, kbeg, wave, lane);
+  else da.init_kc(args.a, args.a_bytes, args.lda, MapDirect{m0, args.m}, kbeg, wave, lane);
+  if constexpr (B_RC) db.init_rc(args.b, args.b_bytes, args.ldb, n0, kbeg, wave, lane);
   else if constexpr (EPI == Epi::SwiGLU)
-    db.init_kc(args.b, args.b_bytes, args.ldb, MapGateValue<BN, WCOLS>{n0, args.f}, kbeg);
-  else db.init_kc(args.b, args.b_bytes, args.ldb, MapDirect{n0, args.n}, kbeg);
+    db.init_kc(args.b, args.b_bytes, args.ldb, MapGateValue<BN, WCOLS>{n0, args.f}, kbeg, wave,
+               lane);
+  else db.init_kc(args.b, args.b_bytes, args.ldb, MapDirect{n0, args.n}, kbeg, wave, lane);
 
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -328,84 +400,166 @@ void gemm_kernel(GemmArgs args) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  // Ring: stage st lives in buffer st % kStages.  The prologue issues the
-  // DMA groups of stages 0 .. kStages-2 and loads the first k step's
-  // fragments.  Iteration st then
-  //   * waits for its own DMA of stage st + 1 and joins the workgroup, so all
-  //     of stage st + 1 has landed and every wave is done with stage st - 1;
-  //   * runs stage st's two k steps of MFMAs, issuing between them -- at
-  //     fixed points (sched_barrier) -- the DMA group of stage
-  //     st + kStages - 1 into stage st - 1's buffer, the fragments of its
-  //     second k step, and the fragments of stage st + 1's first k step.
-  // A group for a stage past the end is still issued, with an offset beyond
-  // the buffer's range: it reads nothing from memory and writes zeros into a
-  // buffer no later stage uses, and every iteration waits for the same
-  // vmcnt.  Fragments prefetched past the last stage are never used.
-  constexpr int kPerWaveA = Dma<A_RC, BM, WAVES>::kPerWave;
-  constexpr int kPerWave = kPerWaveA + Dma<B_RC, BN, WAVES>::kPerWave;
+  // Rings: operand A's stage st lives in buffer st % RA, B's in st % RB (A may
+  // be one stage deeper: it is the operand that streams from HBM, B a weight
+  // that stays in L2).  A stage is BK / 16 k steps; each k step's fragments
+  // are read during the k step before it.  Before its last k step a stage
+  //   * waits for its own LDS reads (the last k step's fragments), for its own
+  //     DMA of stage st + 1, and joins the workgroup: then all of stage st + 1
+  //     has landed and no wave reads stage st any more;
+  //   * from then on, until its next wait, issues B's stage st + RB and then A's
+  //     stage st + RA into the two buffers just released ("window" st + RB).
+  // A stage past the end is still issued, from a resource of zero bytes: it
+  // reads nothing from memory and writes zeros into a buffer no later stage
+  // uses, and every iteration waits for the same vmcnt.  Fragments prefetched
+  // past the last stage are never used.
+  //
+  // The loop is bound by its waves' issue slots and by the path from L2 to
+  // LDS, not by MFMA: with one wave per SIMD an LDS read or a DMA that finds
+  // its queue full stalls the MFMAs behind it.  So both are spread evenly over
+  // the MFMAs, and each MFMA waits only for its own fragments.
+  constexpr int kPA = Dma<A_RC, BM, BK, WAVES>::kPerWave, kPB = Dma<B_RC, BN, BK, WAVES>::kPerWave;
+  constexpr int kPerWave = kPA + kPB;
+  constexpr int kInFlight = (RB - 2) * kPerWave + (RA - RB) * kPA;  // left at a stage's wait
+  // DMA instructions of a window before its k step 0, 1 and 2 (the first ones
+  // go into the last k step of the stage that released the buffers); with
+  // equal rings of two the whole window has to land within the stage, and its
+  // last k step issues none
+  constexpr int kSteps = BK / 16 - (kInFlight ? 0 : 1);
+  constexpr int kD0 = kPerWave / kSteps, kD1 = kPerWave * 2 / kSteps;
+  constexpr int kD2 = BK == 64 ? kPerWave * 3 / kSteps : kPerWave;
   constexpr int kM = TM * TN, kF = TM + TN;
+  Frags<A_RC, BM, BK, TM> fra;
+  Frags<B_RC, BN, BK, TN> frb;
+  fra.init(wm * WM, lane);
+  frb.init(wn * WN, lane);
+  const uint32_t lds_a = (uint32_t)(size_t)(RV_LDS void*)lds;
+  const uint32_t lds_b = lds_a + RA * kA * 2;
   f16x8 fa[2][TM], fb[2][TN];
+  __amdgpu_buffer_rsrc_t ra, rb;  // the window being issued
+  int ia = 0, ib = 0;             // its buffers
 
-#define RV_FRAG(SLOT, LA, LB, KS, P)                                                        \
-  do {                                                                                      \
-    if ((P) < TM) fa[SLOT][(P)] = frag<A_RC, BM>((LA), wm * WM + (P) * 32, (KS), lane);     \
-    else fb[SLOT][(P) - TM] = frag<B_RC, BN>((LB), wn * WN + ((P) - TM) * 32, (KS), lane);  \
-  } while (0)
-#define RV_DMA(D, BUF, ST, LIVE)                                                            \
-  do {                                                                                      \
-    if ((D) < kPerWaveA) da.issue_one((BUF), (ST), (D), (LIVE));                             \
-    else db.issue_one((BUF) + kA, (ST), (D) - kPerWaveA, (LIVE));                            \
-  } while (0)
-  // MFMAs of fragment slot SLOT; after MFMA q, DMA instruction d goes where
-  // d * kM / kPerWave == q (if DO_DMA) and fragment f of (LA2, LB2, KS2) into
-  // slot SLOT ^ 1 where f * kM / kF == q.
-#define RV_KSTEP(SLOT, DO_DMA, DMABUF, DMAST, LIVE, LA2, LB2, KS2)                           \
-  do {                                                                                      \
-    if constexpr (A_RC || B_RC) {                                                           \
-      lds_wait_all();                                                                       \
-      _Pragma("unroll") for (int i_ = 0; i_ < TM; ++i_) after_wait(fa[SLOT][i_]);           \
-      _Pragma("unroll") for (int j_ = 0; j_ < TN; ++j_) after_wait(fb[SLOT][j_]);           \
-      __builtin_amdgcn_sched_barrier(0);                                                    \
-    }                                                                                       \
-    _Pragma("unroll") for (int q = 0; q < kM; ++q) {                                        \
-      acc[q / TN][q % TN] = __builtin_amdgcn_mfma_f32_32x32x16_f16(                          \
-          fb[SLOT][q % TN], fa[SLOT][q / TN], acc[q / TN][q % TN], 0, 0, 0);                \
-      if (DO_DMA) {                                                                         \
-        _Pragma("unroll") for (int d = 0; d < kPerWave; ++d) if (d * kM / kPerWave == q)    \
-          RV_DMA(d, (DMABUF), (DMAST), (LIVE));                                             \
-      }                                                                                     \
-      _Pragma("unroll") for (int f = 0; f < kF; ++f) if (f * kM / kF == q)                  \
-        RV_FRAG((SLOT) ^ 1, (LA2), (LB2), (KS2), f);                                        \
-      __builtin_amdgcn_sched_barrier(0);                                                    \
-    }                                                                                       \
-  } while (0)
+  auto begin_a = [&](int st, int buf) {
+    if constexpr (!A_RC)
+      if (ktail != 0 && st == stages - 1) da.cut_kc(ktail, wave, lane);
+    ra = da.stage(st, st < stages);
+    ia = buf;
+  };
+  auto begin_b = [&](int st, int buf) {
+    if constexpr (!B_RC)
+      if (ktail != 0 && st == stages - 1) db.cut_kc(ktail, wave, lane);
+    rb = db.stage(st, st < stages);
+    ib = buf;
+  };
+  auto dma = [&](int d) {  // instruction d of a window: B's, then A's
+    if (d < kPB) db.issue(rb, lds + RA * kA + ib * kB, d, wave);
+    else da.issue(ra, lds + ia * kA, d - kPB, wave);
+  };
+  // Fragment reads go in the order the MFMAs need them: B 0, A 0, B 1 .. , A 1 ..
+  auto read = [&](auto slot, auto ks, auto f, uint32_t ta, uint32_t tb) {
+    constexpr int S = decltype(slot)::value, K = decltype(ks)::value, P = decltype(f)::value;
+    if constexpr (P == 0) fb[S][0] = frb.template read<0, K>(tb);
+    else if constexpr (P == 1) fa[S][0] = fra.template read<0, K>(ta);
+    else if constexpr (P <= TN) fb[S][P - 1] = frb.template read<P - 1, K>(tb);
+    else fa[S][P - TN] = fra.template read<P - TN, K>(ta);
+  };
+  constexpr auto reads_of = [](int f) {  // LDS instructions of fragment read f
+    return f == 0 || (f > 1 && f <= TN) ? Frags<B_RC, BN, BK, TN>::kReads
+                                         : Frags<A_RC, BM, BK, TM>::kReads;
+  };
+  // The MFMAs of fragment slot S, with the reads of k step K of the stage at
+  // LDS bytes ta / tb into the other slot, and DMA instructions D0 .. D1 - 1,
+  // spread between them at fixed points.  READY: this slot's reads are known
+  // to be complete.
+  auto kstep = [&](auto slot, auto knext, uint32_t ta, uint32_t tb, auto dfirst, auto dlast,
+                   auto ready) {
+    constexpr int S = decltype(slot)::value;
+    constexpr int D0 = decltype(dfirst)::value, ND = decltype(dlast)::value - D0;
+    constexpr bool READY = decltype(ready)::value;
+    static_for<kM>([&](auto qc) {
+      constexpr int q = decltype(qc)::value, i = q / TN, j = q % TN;
+      if constexpr (!READY && (i == 0 || j == 0)) {
+        // the last read this MFMA needs, and the LDS instructions after it
+        constexpr int need = q == 0 ? 1 : i == 0 ? j + 1 : TN + i;
+        constexpr int after = [&] {
+          int n = 0;
+          for (int f = need + 1; f < kF; ++f) n += reads_of(f);
+          for (int f = 0; f < kF; ++f)
+            if (f * kM / kF < q) n += reads_of(f);
+          return n;
+        }();
+        lds_wait<after>();
+        if constexpr (i == 0) after_wait(fb[S][j]);
+        if constexpr (j == 0) after_wait(fa[S][i]);
+      }
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[S][j], fa[S][i], acc[i][j], 0, 0, 0);
+      static_for<kF>([&](auto fc) {
+        constexpr int f = decltype(fc)::value;
+        if constexpr (f * kM / kF == q)
+          read(std::integral_constant<int, S ^ 1>{}, knext, fc, ta, tb);
+      });
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+        if ((2 * d + 1) * kM / (2 * ND) == q) dma(D0 + d);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> c0{};
+  constexpr integral_constant<int, 1> c1{};
+  constexpr integral_constant<int, 2> c2{};
+  constexpr integral_constant<int, 3> c3{};
+  constexpr integral_constant<int, kD0> d0{};
+  constexpr integral_constant<int, kD1> d1{};
+  constexpr integral_constant<int, kD2> d2{};
+  constexpr integral_constant<int, kPerWave> dn{};
+  constexpr integral_constant<bool, false> pending{};
+  constexpr integral_constant<bool, true> ready{};
 
   if (stages > 0) {
+    if constexpr (RA > RB) {  // A's extra stage
+      begin_a(0, 0);
 #pragma unroll
-    for (int p = 0; p < kStages - 1; ++p) {
-      _Float16* buf = lds + p * (kA + kB);
-#pragma unroll
-      for (int d = 0; d < kPerWave; ++d) RV_DMA(d, buf, p, p < stages);
+      for (int d = kPB; d < kPerWave; ++d) dma(d);
     }
-    wait_vmcnt<(kStages - 2) * kPerWave>();
-    lds_barrier();
 #pragma unroll
-    for (int f = 0; f < kF; ++f) RV_FRAG(0, lds, lds + kA, 0, f);
-  }
-  for (int st = 0; st < stages; ++st) {
-    wait_vmcnt<(kStages - 3) * kPerWave>();
+    for (int p = 0; p < RB; ++p) {  // windows 0 .. RB - 1, the last one's first part
+      begin_b(p, p);
+      begin_a(p + RA - RB, p + RA - RB);
+#pragma unroll
+      for (int d = 0; d < (p < RB - 1 ? kPerWave : kD0); ++d) dma(d);
+    }
+    wait_vmcnt<(RA - RB) * kPA + (RB - 2) * kPerWave + kD0>();
     lds_barrier();
-    const _Float16* la = lds + (st % kStages) * (kA + kB);
-    const _Float16* ln = lds + ((st + 1) % kStages) * (kA + kB);
-    _Float16* dbuf = lds + ((st + kStages - 1) % kStages) * (kA + kB);
-    const int dst = st + kStages - 1;
-    RV_KSTEP(0, true, dbuf, dst, dst < stages, la, la + kA, 1);
-    RV_KSTEP(1, false, dbuf, dst, false, ln, ln + kA, 0);
+    static_for<kF>([&](auto fc) { read(c0, c0, fc, lds_a, lds_b); });
   }
-  wait_vmcnt<0>();  // the trailing groups' zero writes land before the ring is reused
-#undef RV_KSTEP
-#undef RV_DMA
-#undef RV_FRAG
+  int ca = 0, cb = 0;  // the stage's buffers
+  for (int st = 0; st < stages; ++st) {
+    const uint32_t ta = lds_a + ca * (kA * 2), tb = lds_b + cb * (kB * 2);
+    kstep(c0, c1, ta, tb, d0, d1, pending);
+    if constexpr (BK == 64) {
+      kstep(c1, c2, ta, tb, d1, d2, pending);
+      kstep(c0, c3, ta, tb, d2, dn, pending);
+    }
+    lds_wait_all();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) after_wait(fa[1][i]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) after_wait(fb[1][j]);
+    wait_vmcnt<kInFlight>();
+    lds_barrier();
+    begin_b(st + RB, cb);
+    begin_a(st + RA, ca);
+    ca = ca + 1 == RA ? 0 : ca + 1;
+    cb = cb + 1 == RB ? 0 : cb + 1;
+    kstep(c1, c0, lds_a + ca * (kA * 2), lds_b + cb * (kB * 2), c0, d0, ready);
+  }
+  lds_wait_all();  // the last prefetched fragments land before their registers are reused
+#pragma unroll
+  for (int i = 0; i < TM; ++i) after_wait(fa[0][i]);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) after_wait(fb[0][j]);
+  wait_vmcnt<0>();  // the trailing stages' zero writes land before the ring is reused
   __syncthreads();  // every wave is done with the ring before the epilogue reuses it
 
   // ---- epilogue ----
@@ -573,42 +727,19 @@ void gemm_kernel(GemmArgs args) {
 // host dispatch can launch.  Without them this compiler emits the host-side
 // launch stubs of only some of the kernels reached through the dispatch
 // switch, and the library fails to load with undefined symbols.
-template __global__ void gemm_kernel<256, 256, false, false, Epi::SwiGLU, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, false, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, true, Epi::SwiGLUBwd, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, true, Epi::StoreF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, true, true, Epi::AccF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, true, true, Epi::PartialF32, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, false, false, Epi::SwiGLU, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, false, false, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, false, true, Epi::SwiGLUBwd, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, false, true, Epi::StoreF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, true, true, Epi::AccF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, true, true, Epi::PartialF32, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, false, false, Epi::SwiGLU, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, false, false, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, false, true, Epi::SwiGLUBwd, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, false, true, Epi::StoreF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, true, true, Epi::AccF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, true, true, Epi::PartialF32, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, false, false, Epi::SwiGLU, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, false, false, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, false, true, Epi::SwiGLUBwd, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, false, true, Epi::StoreF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, true, true, Epi::AccF32OfF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, true, true, Epi::PartialF32, 4>(GemmArgs);
-
-template __global__ void gemm_kernel<256, 256, false, true, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 256, false, true, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<128, 128, false, true, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<64, 128, false, true, Epi::StoreF16, 4>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, false, Epi::SwiGLU, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, false, Epi::StoreF16, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, true, Epi::SwiGLUBwd, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, true, Epi::StoreF32OfF16, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, true, true, Epi::AccF32OfF16, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, true, true, Epi::PartialF32, 8>(GemmArgs);
-template __global__ void gemm_kernel<256, 256, false, true, Epi::StoreF16, 8>(GemmArgs);
+#define RV_ACT_KERNELS(SHAPE)                                                        \
+  template __global__ void gemm_kernel<SHAPE, false, false, Epi::SwiGLU>(GemmArgs);   \
+  template __global__ void gemm_kernel<SHAPE, false, false, Epi::StoreF16>(GemmArgs); \
+  template __global__ void gemm_kernel<SHAPE, false, true, Epi::SwiGLUBwd>(GemmArgs); \
+  template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF16>(GemmArgs);  \
+  template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF32OfF16>(GemmArgs);
+#define RV_WGRAD_KERNELS(SHAPE)                                                       \
+  template __global__ void gemm_kernel<SHAPE, true, true, Epi::AccF32OfF16>(GemmArgs); \
+  template __global__ void gemm_kernel<SHAPE, true, true, Epi::PartialF32>(GemmArgs);
+RV_ACT_KERNELS(0) RV_ACT_KERNELS(1) RV_ACT_KERNELS(2) RV_ACT_KERNELS(3)
+RV_ACT_KERNELS(4) RV_ACT_KERNELS(5) RV_ACT_KERNELS(6)
+RV_WGRAD_KERNELS(0) RV_WGRAD_KERNELS(1) RV_WGRAD_KERNELS(2) RV_WGRAD_KERNELS(3)
+static_assert(kNumShapes == 7 && kRuleShapes == 4, "instantiations above");
 
 // acc[i] (+)= fp32(fp16(sum_s part[s][i])), splits summed in order.  This is
 // autocast's weight gradient: the fp16 GEMM result, cast to the fp32 weight
@@ -727,26 +858,24 @@ void cast_multi_k(CastTable tab) {
 // ---------------------------------------------------------------------------
 // Host side: tile-shape choice and launches.
 // ---------------------------------------------------------------------------
-struct TileShape {
-  int bm, bn, waves;
-};
-// The first kRuleShapes are the ones pick_act's rule and the weight-gradient
-// plan choose from; the tuner also times the rest (256 x 256 with 8 waves:
-// two waves per SIMD, each owning a 128 x 64 block).
-constexpr int kNumShapes = 5, kRuleShapes = 4;
-constexpr TileShape kShapes[kNumShapes] = {
-    {256, 256, 4}, {128, 256, 4}, {128, 128, 4}, {64, 128, 4}, {256, 256, 8}};
-
 template <bool A_RC, bool B_RC, Epi EPI>
 int launch(int shape, const GemmArgs& a, int64_t splits, hipStream_t s) {
+  constexpr bool kWgrad = A_RC;  // weight gradients use the rule's shapes only
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * splits)), block(kShapes[shape].waves * 64);
+#define RV_LAUNCH(SHAPE) \
+  hipLaunchKernelGGL((gemm_kernel<SHAPE, A_RC, B_RC, EPI>), grid, block, 0, s, a)
   switch (shape) {
-    case 0: hipLaunchKernelGGL((gemm_kernel<256, 256, A_RC, B_RC, EPI, 4>), grid, block, 0, s, a); break;
-    case 1: hipLaunchKernelGGL((gemm_kernel<128, 256, A_RC, B_RC, EPI, 4>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((gemm_kernel<128, 128, A_RC, B_RC, EPI, 4>), grid, block, 0, s, a); break;
-    case 3: hipLaunchKernelGGL((gemm_kernel<64, 128, A_RC, B_RC, EPI, 4>), grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL((gemm_kernel<256, 256, A_RC, B_RC, EPI, 8>), grid, block, 0, s, a); break;
+    case 0: RV_LAUNCH(0); break;
+    case 1: RV_LAUNCH(1); break;
+    case 2: RV_LAUNCH(2); break;
+    case 3: RV_LAUNCH(3); break;
+    default:
+      if constexpr (kWgrad) return RV_ERR_UNSUPPORTED;
+      else if (shape == 4) RV_LAUNCH(4);
+      else if (shape == 5) RV_LAUNCH(5);
+      else RV_LAUNCH(6);
   }
+#undef RV_LAUNCH
   return rv_host::check_launch();
 }
 
@@ -901,12 +1030,12 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
     if (ni % t.bm || nj % t.bn) continue;
     const int64_t tiles = (ni / t.bm) * (nj / t.bn);
     int64_t splits = tiles >= kCUs ? 1 : kCUs / tiles;
-    const int64_t max_splits = (rows + 4 * kBK - 1) / (4 * kBK);  // >= 4 stages per split
+    const int64_t max_splits = (rows + 2 * kSplitStep - 1) / (2 * kSplitStep);
     if (splits > max_splits) splits = max_splits;
     if (splits > 64) splits = 64;
     if (splits < 1) splits = 1;
     int64_t chunk = (rows + splits - 1) / splits;
-    chunk = (chunk + kBK - 1) / kBK * kBK;
+    chunk = (chunk + kSplitStep - 1) / kSplitStep * kSplitStep;
     splits = (rows + chunk - 1) / chunk;
     const int64_t wgs = tiles * splits, rounds = (wgs + kCUs - 1) / kCUs;
     const double fill = (double)wgs / (double)(rounds * kCUs);
@@ -1032,7 +1161,7 @@ int rv_mlp_up_swiglu(const void* x, int64_t ldx, const void* w_up, int64_t rows,
                      int64_t f, void* o, void* u, void* stream) {
   if (!x || !w_up || !o) return RV_ERR_NULL_POINTER;
   if (rows <= 0 || d <= 0 || f <= 0 || ldx < d) return RV_ERR_BAD_SIZE;
-  if (d % kBK || f % 64 || ldx % 8) return RV_ERR_UNSUPPORTED;
+  if (d % 32 || f % 64 || ldx % 8) return RV_ERR_UNSUPPORTED;
   if (!ok16(x) || !ok16(w_up) || !ok16(o) || (u && !ok16(u))) return RV_ERR_UNSUPPORTED;
   if (!fits32(rows * ldx) || !fits32(2 * f * d)) return RV_ERR_UNSUPPORTED;
   GemmArgs a{};
@@ -1047,7 +1176,7 @@ int rv_mlp_down(const void* o, const void* w_down, int64_t rows, int64_t d, int6
                 void* stream) {
   if (!o || !w_down || !y) return RV_ERR_NULL_POINTER;
   if (rows <= 0 || d <= 0 || f <= 0) return RV_ERR_BAD_SIZE;
-  if (f % kBK || d % 128) return RV_ERR_UNSUPPORTED;
+  if (f % 32 || d % 128) return RV_ERR_UNSUPPORTED;
   if (!ok16(o) || !ok16(w_down) || !ok16(y)) return RV_ERR_UNSUPPORTED;
   if (!fits32(rows * f) || !fits32(d * f)) return RV_ERR_UNSUPPORTED;
   GemmArgs a{};
@@ -1062,7 +1191,7 @@ int rv_mlp_dgate(const void* dy, const void* w_down, const void* u, int64_t rows
                  int64_t f, void* du, void* stream) {
   if (!dy || !w_down || !u || !du) return RV_ERR_NULL_POINTER;
   if (rows <= 0 || d <= 0 || f <= 0) return RV_ERR_BAD_SIZE;
-  if (d % kBK || f % 128) return RV_ERR_UNSUPPORTED;
+  if (d % 32 || f % 128) return RV_ERR_UNSUPPORTED;
   if (!ok16(dy) || !ok16(w_down) || !ok16(u) || !ok16(du)) return RV_ERR_UNSUPPORTED;
   if (!fits32(rows * d) || !fits32(d * f)) return RV_ERR_UNSUPPORTED;
   GemmArgs a{};
@@ -1078,7 +1207,7 @@ int rv_mlp_dx(const void* du, const void* w_up, int64_t rows, int64_t d, int64_t
               void* stream) {
   if (!du || !w_up || !dx) return RV_ERR_NULL_POINTER;
   if (rows <= 0 || d <= 0 || f <= 0) return RV_ERR_BAD_SIZE;
-  if ((2 * f) % kBK || d % 128) return RV_ERR_UNSUPPORTED;
+  if ((2 * f) % 32 || d % 128) return RV_ERR_UNSUPPORTED;
   if (!ok16(du) || !ok16(w_up) || !ok16(dx)) return RV_ERR_UNSUPPORTED;
   if (!fits32(rows * 2 * f) || !fits32(2 * f * d)) return RV_ERR_UNSUPPORTED;
   GemmArgs a{};

@@ -269,3 +269,46 @@ def test_first_call_under_graph_capture(cuda_device):
         torch.cuda.synchronize()
         assert torch.equal(y_graph, y_eager)
         mlp.down(o, down16, torch.empty_like(y_eager))  # eager work between replays
+
+
+@pytest.mark.parametrize("rows", [1, 129, 300])
+@pytest.mark.parametrize("d", [32, 64, 96, 160, 352])
+def test_depths_off_the_stage_length(cuda_device, rows, d):
+    """Reductions shorter than, equal to and not a multiple of a pipeline
+    stage (64 or 32 values; the entry points take multiples of 32), on every
+    tile shape that fits: the last stage's missing half reads as zero, also
+    when the operands' neighbouring values are infinite.  Same fp64 bound."""
+    from reversability_amd._hip import _stream, library
+    lib = library()
+    f = 256
+    g = torch.Generator().manual_seed(31)
+    # x's rows sit in a wider buffer whose other columns are inf
+    wide = torch.full((rows, d + 32), float("inf"))
+    wide[:, :d] = torch.randn(rows, d, generator=g)
+    wide = wide.half().to(cuda_device)
+    x = wide[:, :d]
+    up = (0.1 * torch.randn(2 * f, d, generator=g)).half().to(cuda_device)
+    down = (0.1 * torch.randn(d, f, generator=g)).half().to(cuda_device)
+    dy = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    u_in = torch.randn(rows, 2 * f, generator=g).half().to(cuda_device)
+    first = None
+    try:
+        for shape in range(lib.rv_gemm_num_shapes()):
+            assert lib.rv_gemm_force_shape(shape) == 0
+            o = torch.empty(rows, f, device=cuda_device, dtype=torch.float16)
+            u = torch.empty(rows, 2 * f, device=cuda_device, dtype=torch.float16)
+            du = torch.empty_like(u)
+            assert lib.rv_mlp_up_swiglu(wide.data_ptr(), wide.stride(0), up.data_ptr(), rows, d,
+                                        f, o.data_ptr(), u.data_ptr(), _stream(wide)) == 0
+            assert lib.rv_mlp_dgate(dy.data_ptr(), down.data_ptr(), u_in.data_ptr(), rows, d, f,
+                                    du.data_ptr(), _stream(dy)) == 0
+            if first is None:
+                first = (o, u, du)
+                assert within_gemm_bound(u, x, up, d)
+                d_o = (dy.double() @ down.double()).half()
+                ref = torch.from_numpy(oracle.swiglu_bwd(u_in.cpu().numpy(), d_o.cpu().numpy()))
+                assert rel_l2(du.cpu(), ref) < 2e-3
+            else:
+                assert all(torch.equal(a, b) for a, b in zip(first, (o, u, du))), shape
+    finally:
+        lib.rv_gemm_force_shape(-1)
