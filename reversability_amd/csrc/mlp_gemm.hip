@@ -364,7 +364,9 @@ void gemm_kernel(GemmArgs args) {
   static_assert(RB >= 2 && (RA == RB || RA == RB + 1), "ring depths");
   constexpr int kA = BM * BK, kB = BN * BK;      // halves per stage and operand
   constexpr int kRing = RA * kA + RB * kB;
-  constexpr int kStaging = WAVES * WM * (WN + 8);  // fp16 epilogue staging
+  constexpr int kStaging = WAVES * WM * (WN + 8);  // fp16 epilogue staging (the fp32 one is less)
+  static_assert(WAVES * 32 * (WN + 4) * 2 <= (kRing > kStaging ? kRing : kStaging),
+                "fp32 epilogue staging");
   __shared__ __attribute__((aligned(1024))) _Float16 lds[kRing > kStaging ? kRing : kStaging];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -569,36 +571,47 @@ void gemm_kernel(GemmArgs args) {
   const int cq = (lane >> 5) * 4;
   if constexpr (EPI == Epi::PartialF32 || EPI == Epi::StoreF32OfF16 ||
                 EPI == Epi::AccF32OfF16) {
-    // fp32 outputs: 16-byte stores straight from the accumulators.
+    // fp32 outputs: each wave passes its block through LDS 32 rows at a time
+    // (row stride WN + 4 floats: conflict free both ways), so that a store
+    // instruction covers whole rows (512 or 256 contiguous bytes) instead of
+    // 32-byte pieces of 32 rows.
+    constexpr int S = WN + 4, CPR = WN / 4, RPP = 64 / CPR;
+    float* stage = reinterpret_cast<float*>(lds) + wave * (32 * S);
+    const int c = lane % CPR * 4;
+    float* out = static_cast<float*>(args.c) + n0 + wn * WN + c;
+    if constexpr (EPI == Epi::PartialF32) out += split * args.m * args.ldc;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int64_t row = m0 + wm * WM + i * 32 + (lane & 31);
-      if (row >= args.m) continue;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int64_t col = n0 + wn * WN + j * 32 + q * 8 + cq;
-          const float a0 = acc[i][j][q * 4], a1 = acc[i][j][q * 4 + 1];
-          const float a2 = acc[i][j][q * 4 + 2], a3 = acc[i][j][q * 4 + 3];
-          if constexpr (EPI == Epi::PartialF32) {
-            *reinterpret_cast<float4*>(static_cast<float*>(args.c) +
-                                       (split * args.m + row) * args.ldc + col) =
-                make_float4(a0, a1, a2, a3);
-          } else {
-            float4 r = make_float4(rv::round_to<__half>(a0), rv::round_to<__half>(a1),
-                                   rv::round_to<__half>(a2), rv::round_to<__half>(a3));
-            float4* c = reinterpret_cast<float4*>(static_cast<float*>(args.c) + row * args.ldc + col);
-            if constexpr (EPI == Epi::AccF32OfF16) {
-              if (args.accumulate) {
-                const float4 p = *c;
-                r = make_float4(p.x + r.x, p.y + r.y, p.z + r.z, p.w + r.w);
-              }
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(stage + (lane & 31) * S + j * 32 + q * 8 + cq) =
+              make_float4(acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2],
+                          acc[i][j][q * 4 + 3]);
+      lds_wait_all();
+      __builtin_amdgcn_wave_barrier();
+      const int64_t row0 = m0 + wm * WM + i * 32;
+#pragma unroll 8
+      for (int r = lane / CPR; r < 32; r += RPP) {
+        const int64_t row = row0 + r;
+        float4 v = *reinterpret_cast<const float4*>(stage + r * S + c);
+        if (row >= args.m) continue;
+        float4* dst = reinterpret_cast<float4*>(out + row * args.ldc);
+        if constexpr (EPI != Epi::PartialF32) {
+          v = make_float4(rv::round_to<__half>(v.x), rv::round_to<__half>(v.y),
+                          rv::round_to<__half>(v.z), rv::round_to<__half>(v.w));
+          if constexpr (EPI == Epi::AccF32OfF16) {
+            if (args.accumulate) {
+              const float4 p = *dst;
+              v = make_float4(p.x + v.x, p.y + v.y, p.z + v.z, p.w + v.w);
             }
-            *c = r;
           }
         }
+        *dst = v;
       }
+      // the next 32 rows' writes follow these reads in the wave's LDS order
+      __builtin_amdgcn_wave_barrier();
     }
   } else {
     // fp16 outputs: each wave stages fp16(acc) for its WM x WN block in LDS
@@ -1021,8 +1034,12 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
   // per-shape efficiencies measured on the split-K weight gradients (the
   // 128 x 256 tile's 0.55: at C5's attention-projection shape, 1024 x 1024
   // over 32768 tokens, it took 113 us with 8 splits where 256 x 256 with 16
-  // takes 85 us, partial sums and their reduce included)
-  static const double eff[kRuleShapes] = {0.8, 0.55, 0.5, 0.35};
+  // takes 85 us, partial sums and their reduce included; the 64 x 128 tile's
+  // 0.42: with half the splits of 128 x 128 it takes 21.4 us against 24.4 for 768
+  // x 256 over 16896 tokens, 22.0 against 24.8 for 2048 x 256 over 8192, 13.3
+  // against 16.4 for 1536 x 512 over 2331, but 41.2 against 34.7 for 2048 x 256
+  // over 16896)
+  static const double eff[kRuleShapes] = {0.8, 0.55, 0.5, 0.42};
   WgradPlan best{-1, 0, 0, 0, 0};
   double best_cost = 0;
   for (int i = 0; i < kRuleShapes; ++i) {
