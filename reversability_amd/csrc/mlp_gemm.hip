@@ -353,9 +353,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 template <int SHAPE, bool A_RC, bool B_RC, Epi EPI>
-__global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
-                             kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
-void gemm_kernel(GemmArgs args) {
+__device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) {
   constexpr int BM = kShapes[SHAPE].bm, BN = kShapes[SHAPE].bn, WAVES = kShapes[SHAPE].waves;
   constexpr int BK = kShapes[SHAPE].bk, RA = kShapes[SHAPE].ra, RB = kShapes[SHAPE].rb;
   // waves: 2 rows x WCOLS columns, each owning a WM x WN block of the tile
@@ -373,9 +371,9 @@ void gemm_kernel(GemmArgs args) {
   const int wm = wave / WCOLS, wn = wave % WCOLS;
 
   const int64_t tiles = args.tiles_m * args.tiles_n;
-  const int64_t split = blockIdx.x / tiles;
+  const int64_t split = block / tiles;
   int64_t tm, tn;
-  tile_of(blockIdx.x % tiles, args.tiles_m, args.tiles_n, tm, tn);
+  tile_of(block % tiles, args.tiles_m, args.tiles_n, tm, tn);
   const int64_t m0 = tm * BM;
   const int64_t n0 = (EPI == Epi::SwiGLU) ? tn * (BN / 2) : tn * BN;
   const int64_t kbeg = split * args.k_chunk;
@@ -736,6 +734,32 @@ void gemm_kernel(GemmArgs args) {
   }
 }
 
+template <int SHAPE, bool A_RC, bool B_RC, Epi EPI>
+__global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
+                             kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
+void gemm_kernel(GemmArgs args) {
+  gemm_block<SHAPE, A_RC, B_RC, EPI>(args, blockIdx.x);
+}
+
+// Two independent GEMMs in one launch: workgroups [0, first) run g[0], the rest
+// g[1].  An MLP's two weight gradients: alone each is one workgroup per CU,
+// together they fill the second place that the 128 x 128 and 64 x 128 tiles
+// leave, so one's loads and partial sums overlap the other's MFMAs (both
+// gradients and their reduce, us, two launches -> one: 51 x 256 x 1024 8.4 -> 4.7,
+// 2048 x 256 x 1024 21.3 -> 16.8, 16896 x 256 x 1024 60.8 -> 53.8, 1000 x 768 x 3072
+// 34.9 -> 27.7, 3062 x 1024 x 4096 100.7 -> 97.0, 32768 x 1024 x 4096 690 -> 687).
+struct GemmPair {
+  GemmArgs g[2];
+  int64_t first;
+};
+template <int SHAPE, Epi EPI>
+__global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
+                             kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
+void wgrad_pair_kernel(GemmPair pair) {
+  const int second = (int64_t)blockIdx.x >= pair.first;
+  gemm_block<SHAPE, true, true, EPI>(pair.g[second], blockIdx.x - (second ? pair.first : 0));
+}
+
 // Explicit instantiations of every (tile shape, operand layout, epilogue) the
 // host dispatch can launch.  Without them this compiler emits the host-side
 // launch stubs of only some of the kernels reached through the dispatch
@@ -748,7 +772,9 @@ void gemm_kernel(GemmArgs args) {
   template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF32OfF16>(GemmArgs);
 #define RV_WGRAD_KERNELS(SHAPE)                                                       \
   template __global__ void gemm_kernel<SHAPE, true, true, Epi::AccF32OfF16>(GemmArgs); \
-  template __global__ void gemm_kernel<SHAPE, true, true, Epi::PartialF32>(GemmArgs);
+  template __global__ void gemm_kernel<SHAPE, true, true, Epi::PartialF32>(GemmArgs);    \
+  template __global__ void wgrad_pair_kernel<SHAPE, Epi::AccF32OfF16>(GemmPair);         \
+  template __global__ void wgrad_pair_kernel<SHAPE, Epi::PartialF32>(GemmPair);
 RV_ACT_KERNELS(0) RV_ACT_KERNELS(1) RV_ACT_KERNELS(2) RV_ACT_KERNELS(3)
 RV_ACT_KERNELS(4) RV_ACT_KERNELS(5) RV_ACT_KERNELS(6)
 RV_WGRAD_KERNELS(0) RV_WGRAD_KERNELS(1) RV_WGRAD_KERNELS(2) RV_WGRAD_KERNELS(3)
@@ -1030,7 +1056,7 @@ struct WgradPlan {
   int shape;
   int64_t tiles_m, tiles_n, splits, chunk;
 };
-WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
+bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, double& cost) {
   // per-shape efficiencies measured on the split-K weight gradients (the
   // 128 x 256 tile's 0.55: at C5's attention-projection shape, 1024 x 1024
   // over 32768 tokens, it took 113 us with 8 splits where 256 x 256 with 16
@@ -1040,58 +1066,104 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
   // against 16.4 for 1536 x 512 over 2331, but 41.2 against 34.7 for 2048 x 256
   // over 16896)
   static const double eff[kRuleShapes] = {0.8, 0.55, 0.5, 0.42};
-  WgradPlan best{-1, 0, 0, 0, 0};
-  double best_cost = 0;
-  for (int i = 0; i < kRuleShapes; ++i) {
-    const TileShape t = kShapes[i];
-    if (ni % t.bm || nj % t.bn) continue;
-    const int64_t tiles = (ni / t.bm) * (nj / t.bn);
-    int64_t splits = tiles >= kCUs ? 1 : kCUs / tiles;
-    const int64_t max_splits = (rows + 2 * kSplitStep - 1) / (2 * kSplitStep);
-    if (splits > max_splits) splits = max_splits;
-    if (splits > 64) splits = 64;
-    if (splits < 1) splits = 1;
-    int64_t chunk = (rows + splits - 1) / splits;
-    chunk = (chunk + kSplitStep - 1) / kSplitStep * kSplitStep;
-    splits = (rows + chunk - 1) / chunk;
-    const int64_t wgs = tiles * splits, rounds = (wgs + kCUs - 1) / kCUs;
-    const double fill = (double)wgs / (double)(rounds * kCUs);
-    const double flops = 2.0 * rows * ni * nj / (eff[i] * fill);
-    const double bytes = splits > 1 ? 8.0 * splits * ni * nj : 0.0;
-    const double cost = flops + 250.0 * bytes;
-    if (best.shape < 0 || cost < best_cost) {
-      best = WgradPlan{i, ni / t.bm, nj / t.bn, splits, chunk};
+  const TileShape t = kShapes[i];
+  if (ni % t.bm || nj % t.bn) return false;
+  const int64_t tiles = (ni / t.bm) * (nj / t.bn);
+  int64_t splits = tiles >= kCUs ? 1 : kCUs / tiles;
+  const int64_t max_splits = (rows + 2 * kSplitStep - 1) / (2 * kSplitStep);
+  if (splits > max_splits) splits = max_splits;
+  if (splits > 64) splits = 64;
+  if (splits < 1) splits = 1;
+  int64_t chunk = (rows + splits - 1) / splits;
+  chunk = (chunk + kSplitStep - 1) / kSplitStep * kSplitStep;
+  splits = (rows + chunk - 1) / chunk;
+  const int64_t wgs = tiles * splits, rounds = (wgs + kCUs - 1) / kCUs;
+  const double fill = (double)wgs / (double)(rounds * kCUs);
+  const double flops = 2.0 * rows * ni * nj / (eff[i] * fill);
+  const double bytes = splits > 1 ? 8.0 * splits * ni * nj : 0.0;
+  cost = flops + 250.0 * bytes;
+  plan = WgradPlan{i, ni / t.bm, nj / t.bn, splits, chunk};
+  return true;
+}
+WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
+  WgradPlan best{-1, 0, 0, 0, 0}, plan;
+  double best_cost = 0, cost;
+  for (int i = 0; i < kRuleShapes; ++i)
+    if (plan_shape(i, rows, ni, nj, plan, cost) && (best.shape < 0 || cost < best_cost)) {
+      best = plan;
       best_cost = cost;
+    }
+  return best;
+}
+
+// The plans of an MLP's two weight gradients (a: 2f x d, b: d x f).  With one
+// tile shape for both they share a launch (launch_pair): the shape with the
+// least total cost among those whose two plans are both split or both not.
+struct PairPlan {
+  WgradPlan a, b;
+  bool paired;
+};
+PairPlan plan_mlp(int64_t rows, int64_t d, int64_t f) {
+  PairPlan best{plan_wgrad(rows, 2 * f, d), plan_wgrad(rows, d, f), false};
+  double best_cost = 0, ca, cb;
+  WgradPlan a, b;
+  for (int i = 0; i < kRuleShapes; ++i) {
+    if (!plan_shape(i, rows, 2 * f, d, a, ca) || !plan_shape(i, rows, d, f, b, cb)) continue;
+    if ((a.splits > 1) != (b.splits > 1)) continue;
+    if (!best.paired || ca + cb < best_cost) {
+      best = PairPlan{a, b, true};
+      best_cost = ca + cb;
     }
   }
   return best;
 }
 
-// The weight-gradient GEMM.  Unsplit, it writes (or adds) the result itself;
-// split, its fp32 partial sums go to `part` and `seg` describes the reduction
-// still to launch (seg.blocks == 0 otherwise).
-int launch_wgrad(const __half* a, int64_t lda, const __half* b, int64_t ldb, int64_t rows,
-                 int64_t ni, int64_t nj, float* out, int accumulate, float* part,
-                 ReduceSeg& seg, hipStream_t s) {
-  seg = ReduceSeg{nullptr, nullptr, 0, 0, 0};
-  const WgradPlan p = plan_wgrad(rows, ni, nj);
-  if (p.shape < 0) return RV_ERR_UNSUPPORTED;
-  GemmArgs g{};
+// One weight-gradient GEMM, planned: unsplit it writes (or adds) the result
+// itself; split, its fp32 partial sums go to `part` and `seg` describes the
+// reduction still to launch (seg.blocks == 0 otherwise).
+struct WgradJob {
+  WgradPlan plan;
+  GemmArgs g;
+  ReduceSeg seg;
+};
+WgradJob plan_job(const WgradPlan& p, const __half* a, int64_t lda, const __half* b, int64_t ldb,
+                  int64_t rows, int64_t ni, int64_t nj, float* out, int accumulate, float* part) {
+  WgradJob j{p, {}, {nullptr, nullptr, 0, 0, 0}};
+  if (p.shape < 0) return j;
+  GemmArgs& g = j.g;
   g.a = a; g.lda = lda; g.a_bytes = rows * lda * 2;
   g.b = b; g.ldb = ldb; g.b_bytes = rows * ldb * 2;
   g.m = ni; g.n = nj; g.k = rows; g.k_chunk = p.chunk;
   g.tiles_m = p.tiles_m; g.tiles_n = p.tiles_n;
   g.ldc = nj; g.accumulate = accumulate;
-  if (p.splits == 1) {
-    g.c = out;
-    return launch<true, true, Epi::AccF32OfF16>(p.shape, g, 1, s);
+  g.c = p.splits == 1 ? out : part;
+  if (p.splits > 1) {
+    const int64_t n = ni * nj;
+    j.seg = ReduceSeg{part, out, n, (int)p.splits, (n / 4 + 255) / 256};
   }
-  g.c = part;
-  const int st = launch<true, true, Epi::PartialF32>(p.shape, g, p.splits, s);
-  if (st != RV_OK) return st;
-  const int64_t n = ni * nj;
-  seg = ReduceSeg{part, out, n, (int)p.splits, (n / 4 + 255) / 256};
-  return RV_OK;
+  return j;
+}
+int launch_job(const WgradJob& j, hipStream_t s) {
+  if (j.plan.shape < 0) return RV_ERR_UNSUPPORTED;
+  return j.plan.splits == 1 ? launch<true, true, Epi::AccF32OfF16>(j.plan.shape, j.g, 1, s)
+                            : launch<true, true, Epi::PartialF32>(j.plan.shape, j.g, j.plan.splits, s);
+}
+
+template <Epi EPI>
+int launch_pair(const WgradJob& a, const WgradJob& b, hipStream_t s) {
+  GemmPair pair{{a.g, b.g}, a.g.tiles_m * a.g.tiles_n * a.plan.splits};
+  const dim3 grid((unsigned)(pair.first + b.g.tiles_m * b.g.tiles_n * b.plan.splits));
+  const dim3 block(kShapes[a.plan.shape].waves * 64);
+#define RV_LAUNCH(SHAPE) \
+  hipLaunchKernelGGL((wgrad_pair_kernel<SHAPE, EPI>), grid, block, 0, s, pair)
+  switch (a.plan.shape) {
+    case 0: RV_LAUNCH(0); break;
+    case 1: RV_LAUNCH(1); break;
+    case 2: RV_LAUNCH(2); break;
+    default: RV_LAUNCH(3); break;
+  }
+#undef RV_LAUNCH
+  return rv_host::check_launch();
 }
 
 int launch_reduce(const ReduceSeg& a, const ReduceSeg& b, int accumulate, hipStream_t s) {
@@ -1103,15 +1175,14 @@ int launch_reduce(const ReduceSeg& a, const ReduceSeg& b, int accumulate, hipStr
 
 int run_wgrad(const __half* a, int64_t lda, const __half* b, int64_t ldb, int64_t rows,
               int64_t ni, int64_t nj, float* out, int accumulate, float* part, hipStream_t s) {
-  ReduceSeg seg;
-  const int st = launch_wgrad(a, lda, b, ldb, rows, ni, nj, out, accumulate, part, seg, s);
+  const WgradJob j =
+      plan_job(plan_wgrad(rows, ni, nj), a, lda, b, ldb, rows, ni, nj, out, accumulate, part);
+  const int st = launch_job(j, s);
   if (st != RV_OK) return st;
-  return launch_reduce(seg, ReduceSeg{nullptr, nullptr, 0, 0, 0}, accumulate, s);
+  return launch_reduce(j.seg, ReduceSeg{nullptr, nullptr, 0, 0, 0}, accumulate, s);
 }
 
-int64_t wgrad_part_bytes(int64_t rows, int64_t ni, int64_t nj) {
-  const WgradPlan p = plan_wgrad(rows, ni, nj);
-  if (p.shape < 0) return -1;
+int64_t part_bytes(const WgradPlan& p, int64_t ni, int64_t nj) {
   return p.splits > 1 ? p.splits * ni * nj * (int64_t)sizeof(float) : 0;
 }
 
@@ -1272,8 +1343,8 @@ int rv_linear_dx(const void* dy, const void* w, int64_t rows, int64_t in, int64_
 
 int64_t rv_linear_dw_workspace_bytes(int64_t rows, int64_t in, int64_t out) {
   if (rows <= 0 || in <= 0 || out <= 0) return -(int64_t)RV_ERR_BAD_SIZE;
-  const int64_t b = wgrad_part_bytes(rows, out, in);
-  return b < 0 ? -(int64_t)RV_ERR_UNSUPPORTED : b;
+  const WgradPlan p = plan_wgrad(rows, out, in);
+  return p.shape < 0 ? -(int64_t)RV_ERR_UNSUPPORTED : part_bytes(p, out, in);
 }
 
 int rv_linear_dw(const void* dy, const void* x, int64_t ldx, int64_t rows, int64_t in,
@@ -1295,9 +1366,10 @@ int rv_linear_dw(const void* dy, const void* x, int64_t ldx, int64_t rows, int64
 
 int64_t rv_mlp_wgrad_workspace_bytes(int64_t rows, int64_t d, int64_t f) {
   if (rows <= 0 || d <= 0 || f <= 0) return -(int64_t)RV_ERR_BAD_SIZE;
-  const int64_t a = wgrad_part_bytes(rows, d, f), b = wgrad_part_bytes(rows, 2 * f, d);
-  if (a < 0 || b < 0) return -(int64_t)RV_ERR_UNSUPPORTED;
-  return (b > 0 ? align256(a) : a) + b;  // both partial sets at once (one reduction launch)
+  const PairPlan p = plan_mlp(rows, d, f);
+  if (p.a.shape < 0 || p.b.shape < 0) return -(int64_t)RV_ERR_UNSUPPORTED;
+  const int64_t down = part_bytes(p.b, d, f), up = part_bytes(p.a, 2 * f, d);
+  return (up > 0 ? align256(down) : down) + up;  // both at once (one reduction launch)
 }
 
 int rv_mlp_wgrad(const void* dy, const void* o, const void* du, const void* x, int64_t ldx,
@@ -1314,19 +1386,27 @@ int rv_mlp_wgrad(const void* dy, const void* o, const void* du, const void* x, i
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !ok16(workspace)))
     return RV_ERR_WORKSPACE;
   const hipStream_t s = (hipStream_t)stream;
-  // the two GEMMs' partial sums side by side, reduced by one launch
+  // dW_down[d][f] = sum_m dy[m][d] o[m][f]; dW_up[2f][d] = sum_m du[m][j] x16[m][d],
+  // their partial sums side by side, reduced by one launch
+  const PairPlan p = plan_mlp(rows, d, f);
   float* part_down = static_cast<float*>(workspace);
-  float* part_up = part_down + align256(wgrad_part_bytes(rows, d, f)) / (int64_t)sizeof(float);
-  ReduceSeg seg_down, seg_up;
-  // dW_down[d][f] = sum_m dy[m][d] o[m][f]
-  int st = launch_wgrad(static_cast<const __half*>(dy), d, static_cast<const __half*>(o), f, rows,
-                        d, f, ddown, accumulate, part_down, seg_down, s);
+  float* part_up = part_down + align256(part_bytes(p.b, d, f)) / (int64_t)sizeof(float);
+  const WgradJob down =
+      plan_job(p.b, static_cast<const __half*>(dy), d, static_cast<const __half*>(o), f, rows, d,
+               f, ddown, accumulate, part_down);
+  const WgradJob up =
+      plan_job(p.a, static_cast<const __half*>(du), 2 * f, static_cast<const __half*>(x), ldx,
+               rows, 2 * f, d, dup, accumulate, part_up);
+  int st;
+  if (p.paired) {
+    st = p.a.splits > 1 ? launch_pair<Epi::PartialF32>(up, down, s)
+                        : launch_pair<Epi::AccF32OfF16>(up, down, s);
+  } else {
+    st = launch_job(down, s);
+    if (st == RV_OK) st = launch_job(up, s);
+  }
   if (st != RV_OK) return st;
-  // dW_up[2f][d] = sum_m du[m][j] x16[m][d]
-  st = launch_wgrad(static_cast<const __half*>(du), 2 * f, static_cast<const __half*>(x), ldx,
-                    rows, 2 * f, d, dup, accumulate, part_up, seg_up, s);
-  if (st != RV_OK) return st;
-  return launch_reduce(seg_down, seg_up, accumulate, s);
+  return launch_reduce(down.seg, up.seg, accumulate, s);
 }
 
 }  // extern "C"

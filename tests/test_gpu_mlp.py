@@ -312,3 +312,24 @@ def test_depths_off_the_stage_length(cuda_device, rows, d):
                 assert all(torch.equal(a, b) for a, b in zip(first, (o, u, du))), shape
     finally:
         lib.rv_gemm_force_shape(-1)
+
+
+@pytest.mark.parametrize("rows", [1, 64, 129, 300, 1025])
+@pytest.mark.parametrize("d,f", [(128, 128), (384, 1664), (1024, 4096)])
+def test_wgrad_pair_plans(cuda_device, rows, d, f):
+    """Both weight gradients in one launch: split and unsplit plans, uneven
+    tile counts of the two, and token counts around a split's granularity
+    (64); the fp64 bound, and the accumulating call adds the same values."""
+    g = torch.Generator().manual_seed(41)
+    dy = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    o = torch.randn(rows, f, generator=g).half().to(cuda_device)
+    du = (0.3 * torch.randn(rows, 2 * f, generator=g)).half().to(cuda_device)
+    x16 = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    ddown = torch.empty(d, f, device=cuda_device)
+    dup = torch.empty(2 * f, d, device=cuda_device)
+    mlp.wgrad(dy, o, du, x16, ddown, dup, accumulate=False)
+    assert within_gemm_bound(ddown, dy.t(), o.t(), rows)
+    assert within_gemm_bound(dup, du.t(), x16.t(), rows)
+    first = (ddown.clone(), dup.clone())
+    mlp.wgrad(dy, o, du, x16, ddown, dup, accumulate=True)
+    assert torch.equal(ddown, first[0] + first[0]) and torch.equal(dup, first[1] + first[1])
