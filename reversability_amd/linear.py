@@ -27,7 +27,7 @@ from torch.autograd.function import once_differentiable
 
 from . import paths
 from ._hip import RV_F16, RV_F32, _check, _stream, library
-from .mlp import cast_f16, cast_weight
+from .mlp import cast_operands
 
 
 def supported(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
@@ -47,20 +47,20 @@ class FusedLinear(torch.autograd.Function):
         out_f, in_f = weight.shape
         flat = x.reshape(-1, in_f)
         rows = flat.shape[0]
-        x16 = cast_f16(flat.contiguous())
+        x16, w16 = cast_operands(flat.contiguous(), weight)
         y = torch.empty(rows, out_f, device=x.device, dtype=torch.float16)
         if rows:
-            w16 = cast_weight(weight)
             _check(library().rv_linear_fwd(x16.data_ptr(), in_f, w16.data_ptr(), rows, in_f,
                                            out_f, y.data_ptr(), _stream(x)), "rv_linear_fwd")
-        ctx.save_for_backward(x16, weight)
+        # the weight's cast serves the backward too (2 bytes per weight)
+        ctx.save_for_backward(x16, weight, w16)
         ctx.x_dtype, ctx.x_shape = x.dtype, x.shape
         return y.reshape(*x.shape[:-1], out_f)
 
     @staticmethod
     @once_differentiable
     def backward(ctx, gradient):
-        x16, weight = ctx.saved_tensors
+        x16, weight, w16 = ctx.saved_tensors
         out_f, in_f = weight.shape
         dy = gradient.reshape(-1, out_f).to(torch.float16).contiguous()
         rows = dy.shape[0]
@@ -70,7 +70,6 @@ class FusedLinear(torch.autograd.Function):
             return (torch.zeros(ctx.x_shape, device=dy.device, dtype=ctx.x_dtype),
                     torch.zeros_like(weight))
         if ctx.needs_input_grad[0]:
-            w16 = cast_weight(weight)
             dx = torch.empty(rows, in_f, device=dy.device, dtype=ctx.x_dtype)
             code = RV_F32 if ctx.x_dtype == torch.float32 else RV_F16
             _check(lib.rv_linear_dx(dy.data_ptr(), w16.data_ptr(), rows, in_f, out_f,

@@ -49,6 +49,37 @@ def cast_f16(t: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _cast_group(group: list, outs: list) -> None:
+    """fp16 casts of fp32 tensors into ``outs`` (all contiguous, 16-byte
+    aligned, at most rv_cast_f32_f16_max_tensors() of them) in one launch."""
+    n = len(group)
+    src = (ctypes.c_void_p * n)(*[w.data_ptr() for w in group])
+    dst = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
+    numel = (ctypes.c_int64 * n)(*[w.numel() for w in group])
+    _check(library().rv_cast_f32_f16_multi(n, src, dst, numel, _stream(group[0])),
+           "rv_cast_f32_f16_multi")
+
+
+def cast_operands(x: torch.Tensor, *weights: torch.Tensor) -> list:
+    """``[cast_f16(x), cast_weight(w) ...]`` with the casts that are still to
+    be made (x if it is fp32, weights outside a ``weight_cast_cache`` block) in
+    one launch."""
+    if _weight_cache is not None:
+        return [cast_f16(x), *(cast_weight(w) for w in weights)]
+    group, outs = [], []
+    for t in (x, *weights):
+        if t.dtype != torch.float32 or not t.is_contiguous():
+            outs.append(cast_f16(t))
+            continue
+        out = torch.empty(t.shape, device=t.device, dtype=torch.float16)
+        outs.append(out)
+        if t.numel():
+            group.append((t, out))
+    if group:
+        _cast_group([t for t, _ in group], [o for _, o in group])
+    return outs
+
+
 # Call-scoped cache of fp16 weight casts (see weight_cast_cache).
 _weight_cache: dict | None = None
 
@@ -141,12 +172,7 @@ def prefetch_casts(weights) -> None:
         for w, size in zip(group, sizes):
             outs.append(flat[offset:offset + w.numel()].view(w.shape))
             offset += size
-        n = len(group)
-        src = (ctypes.c_void_p * n)(*[w.data_ptr() for w in group])
-        dst = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        numel = (ctypes.c_int64 * n)(*[w.numel() for w in group])
-        _check(lib.rv_cast_f32_f16_multi(n, src, dst, numel, _stream(group[0])),
-               "rv_cast_f32_f16_multi")
+        _cast_group(group, outs)
         for w, o in zip(group, outs):
             cache[id(w)] = (w, o)
 

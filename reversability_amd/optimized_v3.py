@@ -134,8 +134,7 @@ class TiledMLP(torch.autograd.Function):
             from . import mlp
             # autocast's casts, once per call: the same fp16 values F.linear
             # would produce on every tile
-            x16 = mlp.cast_f16(flat.contiguous())
-            up16, down16 = mlp.cast_weight(up), mlp.cast_weight(down)
+            x16, up16, down16 = mlp.cast_operands(flat.contiguous(), up, down)
             tiles = [] if keep_tiles else None
             for start in range(0, flat.shape[0], tokens):
                 o, u = mlp.up_swiglu(x16[start:start + tokens], up16, keep_u=keep_tiles)
@@ -144,8 +143,9 @@ class TiledMLP(torch.autograd.Function):
                 if keep_tiles:
                     tiles.append((o, u))
             ctx.tiles = tiles
-            del x16, up16, down16
-            ctx.save_for_backward(x, up, down)
+            del x16
+            # the weights' casts serve the backward too (2 bytes per weight)
+            ctx.save_for_backward(x, up, down, up16, down16)
             return output.reshape(*x.shape[:-1], down.shape[0])
         with torch.autocast(ctx.device, enabled=False):
             # autocast's F.linear casts the weights on every call; one cast per
@@ -162,15 +162,18 @@ class TiledMLP(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, gradient):
-        x, up, down = ctx.saved_tensors
+        x, up, down, *cast = ctx.saved_tensors
         cdt = _compute_dtype(x, ctx.amp, ctx.dtype)
         flat = x.reshape(-1, x.shape[-1])
         dy = gradient.reshape(-1, gradient.shape[-1]).to(cdt)
         dx = torch.empty_like(flat)
         if _use_mfma(flat, up, down, ctx.fused, cdt):
             from . import mlp
-            x16, dy = mlp.cast_f16(flat.contiguous()), dy.contiguous()
-            up16, down16 = mlp.cast_weight(up), mlp.cast_weight(down)
+            dy = dy.contiguous()
+            if cast:
+                x16, (up16, down16) = mlp.cast_f16(flat.contiguous()), cast
+            else:  # the forward computed nothing (need_output=False)
+                x16, up16, down16 = mlp.cast_operands(flat.contiguous(), up, down)
             dup, ddown = torch.empty_like(up), torch.empty_like(down)
             tiles, ctx.tiles = ctx.tiles, None
             for i, start in enumerate(range(0, flat.shape[0], ctx.tokens)):
