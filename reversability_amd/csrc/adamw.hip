@@ -74,15 +74,60 @@ __device__ __forceinline__ void update1(float& p, float g, float& m, float& v, c
   p = __builtin_fmaf(-s.step_size, m / denom, p);     // addcdiv
 }
 
+// Tensor of a workgroup's chunk: the last t with chunk_start[t] <= block.
+__device__ __forceinline__ int tensor_of(const int* chunk_start, int count, int block) {
+  int t = 0, above = count;
+  while (above - t > 1) {
+    const int mid = (t + above) >> 1;
+    if (chunk_start[mid] <= block) t = mid;
+    else above = mid;
+  }
+  return t;
+}
+
+// One pass of a thread: four elements of each array.  The gradient is read
+// with ordinary loads (the norm pass has just read it); LOAD_NT streams the
+// loads of p, m and v, STORE_NT their stores.
+template <bool LOAD_NT>
+struct Pass {
+  float4 p, g, m, v;
+  __device__ __forceinline__ void load(const float* pp, const float* gg, const float* mm,
+                                       const float* vv, int64_t i) {
+    p = LOAD_NT ? rv::ld_f4s(pp + i) : rv::ld_f4(pp + i);
+    g = rv::ld_f4(gg + i);
+    m = LOAD_NT ? rv::ld_f4s(mm + i) : rv::ld_f4(mm + i);
+    v = LOAD_NT ? rv::ld_f4s(vv + i) : rv::ld_f4(vv + i);
+  }
+};
+
+template <bool STORE_NT>
+__device__ __forceinline__ void put(float* dst, float4 x) {
+  if constexpr (STORE_NT) rv::st_f4s(dst, x);
+  else rv::st_f4(dst, x);
+}
+
+// Memory-bound: 28 bytes per parameter against about 60 VALU instructions
+// (sqrt and two divisions).  The next pass's loads are issued before the
+// current pass's arithmetic, the first one's before the bias corrections'
+// double-precision pow; see kStreamLoadBytes for the cache hints.
+template <bool LOAD_NT, bool STORE_NT>
 __global__ __launch_bounds__(kThreads)
 void adamw_k(TensorTable tab, Hyper h) {
   if (h.found_inf != nullptr && *h.found_inf != 0.0f) return;  // uniform skip
-  // tensor of this chunk: last t with chunk_start[t] <= blockIdx.x
-  int t = 0;
-  for (int i = 1; i < tab.count; ++i)
-    if (tab.chunk_start[i] <= (int)blockIdx.x) t = i;
+  const int t = tensor_of(tab.chunk_start, tab.count, (int)blockIdx.x);
   const int64_t off = (int64_t)(blockIdx.x - tab.chunk_start[t]) * kChunk;
   const int64_t end = off + kChunk < tab.n[t] ? off + kChunk : tab.n[t];
+  float* p = tab.p[t];
+  const float* g = tab.g[t];
+  float* m = tab.m[t];
+  float* v = tab.v[t];
+  const bool vec = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g) |
+                     reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(v)) & 15) == 0;
+  int64_t i = off + threadIdx.x * 4;
+  bool live = vec && i + 4 <= end;
+  Pass<LOAD_NT> cur;
+  if (live) cur.load(p, g, m, v, i);  // in flight during the bias corrections' double pow
+  __builtin_amdgcn_sched_barrier(0);
   const double step = (double)*h.step;
   Scalars s;
   s.w1 = (float)(1.0 - h.beta1_d);
@@ -91,26 +136,23 @@ void adamw_k(TensorTable tab, Hyper h) {
   s.bc2_sqrt = (float)sqrt(1.0 - pow(h.beta2_d, step));
   s.inv = h.inv_scale != nullptr ? *h.inv_scale : 1.0f;
   s.clip = h.clip != nullptr ? *h.clip : 1.0f;
-  float* p = tab.p[t];
-  const float* g = tab.g[t];
-  float* m = tab.m[t];
-  float* v = tab.v[t];
-  const bool vec = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g) |
-                     reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(v)) & 15) == 0;
-  int64_t i = off + threadIdx.x * 4;
   if (vec) {
-    for (; i + 4 <= end; i += kThreads * 4) {
-      float4 pp = *reinterpret_cast<const float4*>(p + i);
-      const float4 gg = *reinterpret_cast<const float4*>(g + i);
-      float4 mm = *reinterpret_cast<const float4*>(m + i);
-      float4 vv = *reinterpret_cast<const float4*>(v + i);
-      update1(pp.x, gg.x, mm.x, vv.x, h, s);
-      update1(pp.y, gg.y, mm.y, vv.y, h, s);
-      update1(pp.z, gg.z, mm.z, vv.z, h, s);
-      update1(pp.w, gg.w, mm.w, vv.w, h, s);
-      *reinterpret_cast<float4*>(p + i) = pp;
-      *reinterpret_cast<float4*>(m + i) = mm;
-      *reinterpret_cast<float4*>(v + i) = vv;
+    while (live) {
+      const int64_t next = i + kThreads * 4;
+      const bool more = next + 4 <= end;
+      Pass<LOAD_NT> ahead;
+      if (more) ahead.load(p, g, m, v, next);  // the next pass's loads before this one's math
+      __builtin_amdgcn_sched_barrier(0);
+      update1(cur.p.x, cur.g.x, cur.m.x, cur.v.x, h, s);
+      update1(cur.p.y, cur.g.y, cur.m.y, cur.v.y, h, s);
+      update1(cur.p.z, cur.g.z, cur.m.z, cur.v.z, h, s);
+      update1(cur.p.w, cur.g.w, cur.m.w, cur.v.w, h, s);
+      put<STORE_NT>(p + i, cur.p);
+      put<STORE_NT>(m + i, cur.m);
+      put<STORE_NT>(v + i, cur.v);
+      cur = ahead;
+      i = next;
+      live = more;
     }
     // tail (< 4 elements at the very end of the tensor)
     for (int64_t j = (i < end ? i : end); j < end; ++j) update1(p[j], g[j], m[j], v[j], h, s);
@@ -135,9 +177,7 @@ struct GradTable {
 __global__ __launch_bounds__(kThreads)
 void grad_sq_k(GradTable tab, const float* __restrict__ inv_scale, float* __restrict__ part,
                float* __restrict__ flag, int first) {
-  int t = 0;
-  for (int i = 1; i < tab.count; ++i)
-    if (tab.chunk_start[i] <= (int)blockIdx.x) t = i;
+  const int t = tensor_of(tab.chunk_start, tab.count, (int)blockIdx.x);
   const int64_t off = (int64_t)(blockIdx.x - tab.chunk_start[t]) * kChunk;
   const int64_t end = off + kChunk < tab.n[t] ? off + kChunk : tab.n[t];
   const float inv = inv_scale != nullptr ? *inv_scale : 1.0f;
@@ -151,6 +191,21 @@ void grad_sq_k(GradTable tab, const float* __restrict__ inv_scale, float* __rest
   };
   int64_t i = off + threadIdx.x * 4;
   if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
+    // eight loads in flight, added in order (103.9 M gradients 76 -> 72 us hot)
+    constexpr int kAhead = 8;
+    for (; i + (kAhead - 1) * kThreads * 4 + 4 <= end; i += kAhead * kThreads * 4) {
+      float4 q[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) q[u] = rv::ld_f4(g + i + u * kThreads * 4);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        add(q[u].x);
+        add(q[u].y);
+        add(q[u].z);
+        add(q[u].w);
+      }
+    }
     for (; i + 4 <= end; i += kThreads * 4) {
       const float4 q = *reinterpret_cast<const float4*>(g + i);
       add(q.x);
@@ -238,6 +293,15 @@ void grad_clip_k(const float* __restrict__ part, const float* __restrict__ flag,
   }
 }
 
+// Cache hints by the bytes of the four arrays (16 per parameter), against the
+// 256 MB Infinity Cache.  Norm pass and update, us, with everything else
+// evicted before each call (plain / streamed loads / loads and stores; 32 MB
+// also with nothing evicted): 32 MB 36 / 32 / 32 (24 / 26 / 28), 325 MB 122 / 109 /
+// 120, 430 MB 118 / 106 / 113, 1.66 GB 652 / 624 / 605 (656 / 646 / 568: the
+// gradients then stay cached between the two passes).
+constexpr int64_t kStreamLoadBytes = int64_t(64) << 20;
+constexpr int64_t kStreamStoreBytes = int64_t(512) << 20;
+
 __global__ void adamw_advance_k(float* step, const float* found_inf) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     if (found_inf == nullptr || *found_inf == 0.0f) *step = *step + 1.0f;
@@ -322,6 +386,7 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
   TensorTable tab{};
   Hyper h{};
   int chunks = 0;
+  int64_t bytes = 0;
   for (int i = 0; i < count; ++i) {
     if (!params[i] || !grads[i] || !exp_avg[i] || !exp_avg_sq[i]) return RV_ERR_NULL_POINTER;
     if (numel[i] <= 0) return RV_ERR_BAD_SIZE;
@@ -330,6 +395,7 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
     tab.m[i] = exp_avg[i];
     tab.v[i] = exp_avg_sq[i];
     tab.n[i] = numel[i];
+    bytes += 16 * numel[i];
     tab.chunk_start[i] = chunks;
     const int64_t c = (numel[i] + kChunk - 1) / kChunk;
     if ((int64_t)chunks + c > 0x7fffffff) return RV_ERR_UNSUPPORTED;
@@ -349,8 +415,14 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
   h.found_inf = found_inf;
   h.inv_scale = inv_scale;
   h.clip = clip_coef;
-  hipLaunchKernelGGL(adamw_k, dim3((unsigned)chunks), dim3(kThreads), 0, (hipStream_t)stream, tab,
-                     h);
+  const dim3 grid((unsigned)chunks), block(kThreads);
+  const hipStream_t s = (hipStream_t)stream;
+  if (bytes > kStreamStoreBytes)
+    hipLaunchKernelGGL((adamw_k<true, true>), grid, block, 0, s, tab, h);
+  else if (bytes > kStreamLoadBytes)
+    hipLaunchKernelGGL((adamw_k<true, false>), grid, block, 0, s, tab, h);
+  else
+    hipLaunchKernelGGL((adamw_k<false, false>), grid, block, 0, s, tab, h);
   return rv_host::check_launch();
 }
 

@@ -212,3 +212,29 @@ def test_clip_without_scaler(cuda_device):
             p.grad = torch.zeros_like(p)
         opt_b.unscale_clip_(sc, 1.0)
         opt_b.unscale_clip_(sc, 1.0)
+
+
+@pytest.mark.parametrize("numel", [1023, 16384 * 3 + 5, 5_000_003, 36_000_001])
+def test_update_by_size_of_the_arrays(cuda_device, numel):
+    """Tensors on both sides of the update's streaming thresholds (64 MB and 512
+    MB of the four arrays) and off the vector and chunk lengths: two steps of
+    unscale_clip_ + step equal torch's clip and AdamW to the bar above, and
+    the norm to 1e-6."""
+    g = torch.Generator(device=cuda_device).manual_seed(17)
+    def rand(std):
+        return std * torch.randn(numel, generator=g, device=cuda_device)
+    base = rand(0.02)
+    a, b = base.clone().requires_grad_(True), base.clone().requires_grad_(True)
+    ta = torch.optim.AdamW([a], lr=6e-4, betas=(0.9, 0.95), weight_decay=0.1, foreach=True)
+    fb = FusedAdamW([b], lr=6e-4, betas=(0.9, 0.95), weight_decay=0.1)
+    for _ in range(2):
+        grad = rand(1e-2)
+        a.grad, b.grad = grad.clone(), grad
+        na = torch.nn.utils.clip_grad_norm_([a], 1.0)
+        nb = fb.unscale_clip_(None, 1.0)
+        assert abs(float(na) - float(nb)) <= 1e-6 * float(na)
+        ta.step()
+        fb.step()
+        assert _close(b.detach(), a.detach())
+    sa, sb = ta.state[a], fb.state[b]
+    assert _close(sb["exp_avg"], sa["exp_avg"]) and _close(sb["exp_avg_sq"], sa["exp_avg_sq"])
