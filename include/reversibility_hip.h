@@ -324,6 +324,20 @@ int rv_linear_fwd(const void* x, int64_t ldx, const void* w, int64_t rows,
 int rv_linear_dx(const void* dy, const void* w, int64_t rows, int64_t in,
                  int64_t out, void* dx, int dx_dtype, void* stream);
 
+/*
+ * rv_linear_fwd / rv_linear_dx with a workspace: products with few output tiles
+ * and a long reduction are split over it (fp32 partial sums added in a fixed
+ * order; the plan depends on the sizes only).  rv_linear_splitk_workspace_bytes
+ * (rows, n, k) is the size needed for an n-column output reduced over k (fwd: n
+ * = out, k = in; dx: n = in, k = out); where it is 0 these are the calls above.
+ */
+int64_t rv_linear_splitk_workspace_bytes(int64_t rows, int64_t n, int64_t k);
+int rv_linear_fwd_ws(const void* x, int64_t ldx, const void* w, int64_t rows, int64_t in,
+                     int64_t out, void* y, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int64_t out, void* dx,
+                    int dx_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Scratch bytes rv_linear_dw needs (split-K partial sums; may be 0). */
 int64_t rv_linear_dw_workspace_bytes(int64_t rows, int64_t in, int64_t out);
 

@@ -61,6 +61,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 
 #include "rv_device.h"
@@ -769,7 +770,9 @@ void wgrad_pair_kernel(GemmPair pair) {
   template __global__ void gemm_kernel<SHAPE, false, false, Epi::StoreF16>(GemmArgs); \
   template __global__ void gemm_kernel<SHAPE, false, true, Epi::SwiGLUBwd>(GemmArgs); \
   template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF16>(GemmArgs);  \
-  template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF32OfF16>(GemmArgs);
+  template __global__ void gemm_kernel<SHAPE, false, true, Epi::StoreF32OfF16>(GemmArgs); \
+  template __global__ void gemm_kernel<SHAPE, false, false, Epi::PartialF32>(GemmArgs);  \
+  template __global__ void gemm_kernel<SHAPE, false, true, Epi::PartialF32>(GemmArgs);
 #define RV_WGRAD_KERNELS(SHAPE)                                                       \
   template __global__ void gemm_kernel<SHAPE, true, true, Epi::AccF32OfF16>(GemmArgs); \
   template __global__ void gemm_kernel<SHAPE, true, true, Epi::PartialF32>(GemmArgs);    \
@@ -828,6 +831,41 @@ void wgrad_reduce(ReduceSeg a, ReduceSeg b, int accumulate) {
     r = make_float4(p.x + r.x, p.y + r.y, p.z + r.z, p.w + r.w);
   }
   *o = r;
+}
+
+// An activation GEMM's split-K finish: out[i] = fp16(sum_s part[s][i]), splits
+// summed in order, stored as fp16 or as that value widened to fp32.  n % 4 == 0.
+template <typename T>
+__global__ __launch_bounds__(256)
+void act_reduce(const float* __restrict__ part, T* __restrict__ out, int64_t n, int splits) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  float4 s = *reinterpret_cast<const float4*>(part + i);
+  int k = 1;
+  for (; k + 4 <= splits; k += 4) {  // four splits' loads in flight, added in order
+    float4 t[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      t[j] = *reinterpret_cast<const float4*>(part + (int64_t)(k + j) * n + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      s.x = s.x + t[j].x; s.y = s.y + t[j].y; s.z = s.z + t[j].z; s.w = s.w + t[j].w;
+    }
+  }
+  for (; k < splits; ++k) {
+    const float4 t = *reinterpret_cast<const float4*>(part + (int64_t)k * n + i);
+    s.x = s.x + t.x; s.y = s.y + t.y; s.z = s.z + t.z; s.w = s.w + t.w;
+  }
+  const __half2 lo = __floats2half2_rn(s.x, s.y), hi = __floats2half2_rn(s.z, s.w);
+  if constexpr (std::is_same<T, float>::value) {
+    *reinterpret_cast<float4*>(out + i) =
+        make_float4(__low2float(lo), __high2float(lo), __low2float(hi), __high2float(hi));
+  } else {
+    uint2 v;
+    v.x = *reinterpret_cast<const uint32_t*>(&lo);
+    v.y = *reinterpret_cast<const uint32_t*>(&hi);
+    *reinterpret_cast<uint2*>(out + i) = v;
+  }
 }
 
 // dst = fp16(src), round to nearest even; 8 elements per thread.
@@ -930,13 +968,13 @@ int launch(int shape, const GemmArgs& a, int64_t splits, hipStream_t s) {
 // Activation GEMMs: C is m x n_out where n_out = n (or n/2 output columns for
 // SwiGLU, whose tile covers bn/2 of them).  The largest tile that gives at
 // least one workgroup per CU; otherwise the one with the most workgroups.
-int pick_act(int64_t m, int64_t n_cols, bool swiglu) {
+int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits) {
   int best = -1;
   int64_t best_blocks = -1;
   for (int i = 0; i < kRuleShapes; ++i) {
     const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
     if (n_cols % cols) continue;
-    const int64_t blocks = ((m + kShapes[i].bm - 1) / kShapes[i].bm) * (n_cols / cols);
+    const int64_t blocks = ((m + kShapes[i].bm - 1) / kShapes[i].bm) * (n_cols / cols) * splits;
     if (blocks >= kCUs) return i;
     if (blocks > best_blocks) best = i, best_blocks = blocks;
   }
@@ -975,14 +1013,14 @@ bool capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
+// a.k_chunk < a.k: split-K, one partial (Epi::PartialF32) per k_chunk of k.
 template <bool A_RC, bool B_RC, Epi EPI>
 int launch_shape(int shape, GemmArgs a, int64_t n_cols, hipStream_t s) {
   const bool swiglu = EPI == Epi::SwiGLU;
   const TileShape t = kShapes[shape];
   a.tiles_m = (a.m + t.bm - 1) / t.bm;
   a.tiles_n = n_cols / (swiglu ? t.bn / 2 : t.bn);
-  a.k_chunk = a.k;
-  return launch<A_RC, B_RC, EPI>(shape, a, 1, s);
+  return launch<A_RC, B_RC, EPI>(shape, a, (a.k + a.k_chunk - 1) / a.k_chunk, s);
 }
 
 template <bool A_RC, bool B_RC, Epi EPI>
@@ -1022,7 +1060,9 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
 template <bool A_RC, bool B_RC, Epi EPI>
 int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
   const bool swiglu = EPI == Epi::SwiGLU;
-  int shape = pick_act(a.m, n_cols, swiglu);
+  if (EPI != Epi::PartialF32) a.k_chunk = a.k;
+  const int64_t splits = (a.k + a.k_chunk - 1) / a.k_chunk;
+  int shape = pick_act(a.m, n_cols, swiglu, splits);
   if (shape < 0) return RV_ERR_UNSUPPORTED;
   const int forced = g_forced_shape.load();
   if (forced >= 0) {
@@ -1036,7 +1076,7 @@ int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
     // amounts and are tuned apart
     const int variant = (EPI == Epi::SwiGLU && a.u != nullptr) ? 1 : 0;
     const TuneKey key{(int)EPI * 4 + (A_RC ? 2 : 0) + (B_RC ? 1 : 0), device, variant, a.m,
-                      n_cols, a.k};
+                      n_cols, EPI == Epi::PartialF32 ? a.k * 64 + splits : a.k};
     std::lock_guard<std::mutex> lock(g_tune_mu);
     const auto it = g_tuned.find(key);
     if (it != g_tuned.end()) {
@@ -1047,6 +1087,53 @@ int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
     }
   }
   return launch_shape<A_RC, B_RC, EPI>(shape, a, n_cols, s);
+}
+
+// Split count of an activation GEMM without a fused epilogue: the reduction is
+// cut into `splits` partials (fp32, summed in order by act_reduce) when few
+// output tiles would leave most CUs idle behind a long serial k loop.  Modelled
+// on the 64 x 128 tile: 0.33 us per 64 of k for up to one workgroup per CU,
+// against 4.5 us for the second launch and the partials' traffic (8 bytes each
+// at 5 TB/s); a split has to save a fifth.  Measured (us, unsplit -> best count):
+// 51 x 256 x 2048 (m, n, k) 12.9 -> 7.4, 51 x 1024 x 4096 23.0 -> 9.0, 512 x 1024 x
+// 4096 23.5 -> 13.9, 1024 x 1024 x 8192 44.9 -> 30.1; not worth it: 51 x 256 x 1024
+// 7.9 (6.8), 4096 x 256 x 2048 13.8 (15.8), 2331 x 512 x 1536 11.3 (16.0), 3062 x 1024 x
+// 8192 70 (66), 8192 x 1024 x 4096 67 (76).  Depends on the sizes only, so a
+// recomputed product has the same bits.
+int64_t act_splits(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + 63) / 64) * (n / 128);
+  if (tiles <= 0 || tiles > kCUs / 2) return 1;
+  const double stages = (double)k / kSplitStep * 0.33;
+  int64_t best = 1;
+  double best_us = 0.8 * stages;
+  for (int64_t s = 2; s <= 32 && k / s >= 2 * kSplitStep; ++s) {
+    const int64_t wgs = tiles * s;
+    const double us = stages / s * (wgs > kCUs ? (double)wgs / kCUs : 1.0) + 4.5 +
+                      8.0 * m * n * s / 5e6;
+    if (us < best_us) best = s, best_us = us;
+  }
+  return best;
+}
+int64_t act_chunk(int64_t m, int64_t n, int64_t k) {
+  const int64_t splits = act_splits(m, n, k);
+  return ((k + splits - 1) / splits + kSplitStep - 1) / kSplitStep * kSplitStep;
+}
+int64_t act_part_bytes(int64_t m, int64_t n, int64_t k) {
+  const int64_t chunk = act_chunk(m, n, k), splits = (k + chunk - 1) / chunk;
+  return splits > 1 ? splits * m * n * (int64_t)sizeof(float) : 0;
+}
+
+template <bool B_RC, typename T>
+int run_split(GemmArgs a, T* out, float* part, hipStream_t s) {
+  a.k_chunk = act_chunk(a.m, a.n, a.k);
+  a.c = part;
+  a.ldc = a.n;
+  const int st = run_act<false, B_RC, Epi::PartialF32>(a, a.n, s);
+  if (st != RV_OK) return st;
+  const int64_t n = a.m * a.n, splits = (a.k + a.k_chunk - 1) / a.k_chunk;
+  hipLaunchKernelGGL(act_reduce<T>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, part,
+                     out, n, (int)splits);
+  return rv_host::check_launch();
 }
 
 // Weight-gradient plan for an ni x nj output reduced over `rows` tokens: tile
@@ -1353,6 +1440,51 @@ int rv_linear_dx(const void* dy, const void* w, int64_t rows, int64_t in, int64_
   const hipStream_t s = (hipStream_t)stream;
   return dx_dtype == RV_F16 ? run_act<false, true, Epi::StoreF16>(a, in, s)
                             : run_act<false, true, Epi::StoreF32OfF16>(a, in, s);
+}
+
+int64_t rv_linear_splitk_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
+  if (rows <= 0 || n <= 0 || k <= 0) return -(int64_t)RV_ERR_BAD_SIZE;
+  return act_part_bytes(rows, n, k);
+}
+
+int rv_linear_fwd_ws(const void* x, int64_t ldx, const void* w, int64_t rows, int64_t in,
+                     int64_t out, void* y, void* workspace, int64_t workspace_bytes,
+                     void* stream) {
+  const int64_t need = in > 0 && out > 0 && rows > 0 ? act_part_bytes(rows, out, in) : 0;
+  if (need == 0) return rv_linear_fwd(x, ldx, w, rows, in, out, y, stream);
+  if (!x || !w || !y) return RV_ERR_NULL_POINTER;
+  if (ldx < in) return RV_ERR_BAD_SIZE;
+  if (in % 128 || out % 128 || ldx % 8) return RV_ERR_UNSUPPORTED;
+  if (!ok16(x) || !ok16(w) || !ok16(y)) return RV_ERR_UNSUPPORTED;
+  if (!fits32(rows * ldx) || !fits32(out * in)) return RV_ERR_UNSUPPORTED;
+  if (!workspace || workspace_bytes < need || !ok16(workspace)) return RV_ERR_WORKSPACE;
+  GemmArgs a{};
+  a.a = static_cast<const __half*>(x); a.lda = ldx; a.a_bytes = rows * ldx * 2;
+  a.b = static_cast<const __half*>(w); a.ldb = in; a.b_bytes = out * in * 2;
+  a.m = rows; a.n = out; a.k = in;
+  return run_split<false>(a, static_cast<__half*>(y), static_cast<float*>(workspace),
+                          (hipStream_t)stream);
+}
+
+int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int64_t out, void* dx,
+                    int dx_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t need = in > 0 && out > 0 && rows > 0 ? act_part_bytes(rows, in, out) : 0;
+  if (need == 0) return rv_linear_dx(dy, w, rows, in, out, dx, dx_dtype, stream);
+  if (!dy || !w || !dx) return RV_ERR_NULL_POINTER;
+  if (in % 128 || out % 128) return RV_ERR_UNSUPPORTED;
+  if (dx_dtype != RV_F16 && dx_dtype != RV_F32) return RV_ERR_UNSUPPORTED;
+  if (!ok16(dy) || !ok16(w) || !ok16(dx)) return RV_ERR_UNSUPPORTED;
+  if (!fits32(rows * out) || !fits32(out * in)) return RV_ERR_UNSUPPORTED;
+  if (!workspace || workspace_bytes < need || !ok16(workspace)) return RV_ERR_WORKSPACE;
+  GemmArgs a{};
+  a.a = static_cast<const __half*>(dy); a.lda = out; a.a_bytes = rows * out * 2;
+  a.b = static_cast<const __half*>(w); a.ldb = in;  // B(i, o) = W[o][i]: RC
+  a.b_bytes = out * in * 2;
+  a.m = rows; a.n = in; a.k = out;
+  const hipStream_t s = (hipStream_t)stream;
+  float* part = static_cast<float*>(workspace);
+  return dx_dtype == RV_F16 ? run_split<true>(a, static_cast<__half*>(dx), part, s)
+                            : run_split<true>(a, static_cast<float*>(dx), part, s);
 }
 
 int64_t rv_linear_dw_workspace_bytes(int64_t rows, int64_t in, int64_t out) {

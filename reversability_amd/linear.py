@@ -27,7 +27,7 @@ from torch.autograd.function import once_differentiable
 
 from . import paths
 from ._hip import RV_F16, RV_F32, _check, _stream, library
-from .mlp import cast_operands
+from .mlp import cast_operands, splitk_workspace
 
 
 def supported(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
@@ -50,8 +50,10 @@ class FusedLinear(torch.autograd.Function):
         x16, w16 = cast_operands(flat.contiguous(), weight)
         y = torch.empty(rows, out_f, device=x.device, dtype=torch.float16)
         if rows:
-            _check(library().rv_linear_fwd(x16.data_ptr(), in_f, w16.data_ptr(), rows, in_f,
-                                           out_f, y.data_ptr(), _stream(x)), "rv_linear_fwd")
+            ws, nbytes = splitk_workspace(x16, rows, out_f, in_f)
+            _check(library().rv_linear_fwd_ws(
+                x16.data_ptr(), in_f, w16.data_ptr(), rows, in_f, out_f, y.data_ptr(),
+                ws.data_ptr() if ws is not None else None, nbytes, _stream(x)), "rv_linear_fwd")
         # the weight's cast serves the backward too (2 bytes per weight)
         ctx.save_for_backward(x16, weight, w16)
         ctx.x_dtype, ctx.x_shape = x.dtype, x.shape
@@ -72,8 +74,10 @@ class FusedLinear(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = torch.empty(rows, in_f, device=dy.device, dtype=ctx.x_dtype)
             code = RV_F32 if ctx.x_dtype == torch.float32 else RV_F16
-            _check(lib.rv_linear_dx(dy.data_ptr(), w16.data_ptr(), rows, in_f, out_f,
-                                    dx.data_ptr(), code, _stream(dy)), "rv_linear_dx")
+            ws, nbytes = splitk_workspace(dy, rows, in_f, out_f)
+            _check(lib.rv_linear_dx_ws(
+                dy.data_ptr(), w16.data_ptr(), rows, in_f, out_f, dx.data_ptr(), code,
+                ws.data_ptr() if ws is not None else None, nbytes, _stream(dy)), "rv_linear_dx")
             dx = dx.reshape(ctx.x_shape)
         if ctx.needs_input_grad[1]:
             dw = torch.empty_like(weight)

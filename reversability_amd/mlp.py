@@ -25,7 +25,7 @@ import threading
 
 import torch
 
-from ._hip import RV_F16, _check, _stream, library
+from ._hip import RV_F16, RV_F32, _check, _stream, library
 
 
 def supported(x: torch.Tensor, up: torch.Tensor, down: torch.Tensor) -> bool:
@@ -195,12 +195,27 @@ def up_swiglu(x: torch.Tensor, up: torch.Tensor, keep_u: bool = False):
     return o, u
 
 
+def splitk_workspace(like: torch.Tensor, rows: int, n: int, k: int):
+    """(workspace or None, its bytes) of a rows x n product reduced over k:
+    few output tiles and a long reduction are split (csrc/mlp_gemm.hip)."""
+    nbytes = library().rv_linear_splitk_workspace_bytes(rows, n, k)
+    if nbytes <= 0:
+        return None, 0
+    return torch.empty(nbytes // 4, device=like.device, dtype=torch.float32), nbytes
+
+
 def down(o: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     _f16(o, "o"), _f16(w, "W_down")
     rows, f = o.shape
     d = w.shape[0]
-    _check(library().rv_mlp_down(o.data_ptr(), w.data_ptr(), rows, d, f, out.data_ptr(),
-                                 _stream(o)), "rv_mlp_down")
+    ws, nbytes = splitk_workspace(o, rows, d, f)
+    if ws is not None:  # the same contraction as a linear layer's forward
+        _check(library().rv_linear_fwd_ws(o.data_ptr(), f, w.data_ptr(), rows, f, d,
+                                          out.data_ptr(), ws.data_ptr(), nbytes, _stream(o)),
+               "rv_linear_fwd_ws")
+    else:
+        _check(library().rv_mlp_down(o.data_ptr(), w.data_ptr(), rows, d, f, out.data_ptr(),
+                                     _stream(o)), "rv_mlp_down")
     return out
 
 
@@ -222,14 +237,20 @@ def dx(du: torch.Tensor, w_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     d = w_up.shape[1]
     if tuple(out.shape) != (rows, d) or not out.is_contiguous():
         raise ValueError("dx output must be a contiguous [rows, d] tensor")
-    if out.dtype == torch.float32:
+    if out.dtype not in (torch.float32, torch.float16):
+        raise ValueError("dx output must be fp32 or fp16")
+    ws, nbytes = splitk_workspace(du, rows, d, two_f)
+    if ws is not None:
+        code = RV_F32 if out.dtype == torch.float32 else RV_F16
+        _check(library().rv_linear_dx_ws(du.data_ptr(), w_up.data_ptr(), rows, d, two_f,
+                                         out.data_ptr(), code, ws.data_ptr(), nbytes,
+                                         _stream(du)), "rv_linear_dx_ws")
+    elif out.dtype == torch.float32:
         _check(library().rv_mlp_dx(du.data_ptr(), w_up.data_ptr(), rows, d, two_f // 2,
                                    out.data_ptr(), _stream(du)), "rv_mlp_dx")
-    elif out.dtype == torch.float16:  # the same contraction as a linear layer's dx
+    else:  # the same contraction as a linear layer's dx
         _check(library().rv_linear_dx(du.data_ptr(), w_up.data_ptr(), rows, d, two_f,
                                       out.data_ptr(), RV_F16, _stream(du)), "rv_linear_dx")
-    else:
-        raise ValueError("dx output must be fp32 or fp16")
     return out
 
 

@@ -99,3 +99,50 @@ def test_enable_linear_falls_back_outside_fp16_autocast(cuda_device):
     with torch.autocast("cuda", dtype=torch.float16):
         assert supported(x, layer.weight, None)
         assert linear(x, layer.weight).dtype == torch.float16
+
+
+@pytest.mark.parametrize("rows,in_f,out_f", [(1, 2048, 128), (51, 4096, 256), (65, 8192, 128),
+                                             (512, 4096, 1024), (500, 4224, 1152)])
+def test_split_reduction(cuda_device, rows, in_f, out_f):
+    """Products with few output tiles and a long reduction are split over it:
+    the fp64 bound for the forward and the fp16 and fp32 input gradients,
+    identical bits on every tile shape, and a workspace that is too small is
+    refused."""
+    from reversability_amd._hip import RV_F16, RV_F32, _stream, library
+    lib = library()
+    g = torch.Generator().manual_seed(23)
+    x = torch.randn(rows, in_f, generator=g).half().to(cuda_device)
+    w = (0.02 * torch.randn(out_f, in_f, generator=g)).half().to(cuda_device)
+    wt = w.t().contiguous()  # [in_f, out_f]: dx of a layer with out = in_f, in = out_f
+    need = lib.rv_linear_splitk_workspace_bytes(rows, out_f, in_f)
+    assert need > 0 and need % (4 * rows * out_f) == 0
+    ws = torch.empty(need // 4, device=cuda_device)
+    st = _stream(x)
+    first = None
+    try:
+        for shape in range(-1, lib.rv_gemm_num_shapes()):
+            assert lib.rv_gemm_force_shape(shape) == 0
+            y, d16 = (torch.empty(rows, out_f, device=cuda_device, dtype=torch.float16)
+                      for _ in range(2))
+            d32 = torch.empty(rows, out_f, device=cuda_device)
+            args = (ws.data_ptr(), need, st)
+            codes = [lib.rv_linear_fwd_ws(x.data_ptr(), in_f, w.data_ptr(), rows, in_f, out_f,
+                                          y.data_ptr(), *args)]
+            for dx, code in ((d16, RV_F16), (d32, RV_F32)):
+                codes.append(lib.rv_linear_dx_ws(x.data_ptr(), wt.data_ptr(), rows, out_f, in_f,
+                                                 dx.data_ptr(), code, *args))
+            if shape >= 0 and codes[0] == 3:  # the width does not divide this tile
+                assert codes == [3, 3, 3]
+                continue
+            assert codes == [0, 0, 0], shape
+            if first is None:
+                first = (y, d16, d32)
+                assert within_gemm_bound(y, x, w, in_f)
+                assert within_gemm_bound(d16, x, w, in_f)
+                assert torch.equal(d32, d16.float())
+            else:
+                assert all(torch.equal(a, b) for a, b in zip(first, (y, d16, d32))), shape
+    finally:
+        lib.rv_gemm_force_shape(-1)
+    assert lib.rv_linear_fwd_ws(x.data_ptr(), in_f, w.data_ptr(), rows, in_f, out_f,
+                                first[0].data_ptr(), ws.data_ptr(), need - 1, st) != 0
