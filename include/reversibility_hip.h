@@ -338,6 +338,15 @@ int rv_linear_fwd_ws(const void* x, int64_t ldx, const void* w, int64_t rows, in
 int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int64_t out, void* dx,
                     int dx_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Two layers' weight gradients over the same rows in one launch: dw_a[out_a,
+ * in_a] (+)= fp32(fp16(dy_a^T x_a)) and dw_b likewise (x_a, x_b contiguous). */
+int64_t rv_linear_dw_pair_workspace_bytes(int64_t rows, int64_t in_a, int64_t out_a,
+                                          int64_t in_b, int64_t out_b);
+int rv_linear_dw_pair(const void* dy_a, const void* x_a, int64_t in_a, int64_t out_a,
+                      float* dw_a, const void* dy_b, const void* x_b, int64_t in_b,
+                      int64_t out_b, float* dw_b, int64_t rows, int accumulate,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Scratch bytes rv_linear_dw needs (split-K partial sums; may be 0). */
 int64_t rv_linear_dw_workspace_bytes(int64_t rows, int64_t in, int64_t out);
 

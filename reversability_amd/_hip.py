@@ -60,6 +60,9 @@ SIGNATURES = {
     "rv_linear_splitk_workspace_bytes": (_I64, [_I64, _I64, _I64]),
     "rv_linear_fwd_ws": (_I, [_P, _I64, _P, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "rv_linear_dx_ws": (_I, [_P, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _P]),
+    "rv_linear_dw_pair_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
+    "rv_linear_dw_pair": (_I, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _I64, _P, _I64, _I, _P, _I64,
+                               _P]),
     "rv_linear_dw_workspace_bytes": (_I64, [_I64, _I64, _I64]),
     "rv_linear_dw": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _I, _P, _I64, _P]),
     "rv_adamw_max_tensors": (_I, []),

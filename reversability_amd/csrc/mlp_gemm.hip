@@ -1192,19 +1192,20 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
   return best;
 }
 
-// The plans of an MLP's two weight gradients (a: 2f x d, b: d x f).  With one
-// tile shape for both they share a launch (launch_pair): the shape with the
-// least total cost among those whose two plans are both split or both not.
+// The plans of two weight gradients over the same rows (a: ai x aj, b: bi x
+// bj).  With one tile shape for both they share a launch (launch_pair): the
+// shape with the least total cost among those whose two plans are both split
+// or both not.
 struct PairPlan {
   WgradPlan a, b;
   bool paired;
 };
-PairPlan plan_mlp(int64_t rows, int64_t d, int64_t f) {
-  PairPlan best{plan_wgrad(rows, 2 * f, d), plan_wgrad(rows, d, f), false};
+PairPlan plan_pair(int64_t rows, int64_t ai, int64_t aj, int64_t bi, int64_t bj) {
+  PairPlan best{plan_wgrad(rows, ai, aj), plan_wgrad(rows, bi, bj), false};
   double best_cost = 0, ca, cb;
   WgradPlan a, b;
   for (int i = 0; i < kRuleShapes; ++i) {
-    if (!plan_shape(i, rows, 2 * f, d, a, ca) || !plan_shape(i, rows, d, f, b, cb)) continue;
+    if (!plan_shape(i, rows, ai, aj, a, ca) || !plan_shape(i, rows, bi, bj, b, cb)) continue;
     if ((a.splits > 1) != (b.splits > 1)) continue;
     if (!best.paired || ca + cb < best_cost) {
       best = PairPlan{a, b, true};
@@ -1282,9 +1283,43 @@ int64_t part_bytes(const WgradPlan& p, int64_t ni, int64_t nj) {
   return p.splits > 1 ? p.splits * ni * nj * (int64_t)sizeof(float) : 0;
 }
 
-bool ok16(const void* p) { return rv_host::aligned16(p); }
-
 int64_t align256(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
+
+// Both partial sums of a pair side by side (b's first), reduced by one launch.
+int64_t pair_bytes(const PairPlan& p, int64_t ai, int64_t aj, int64_t bi, int64_t bj) {
+  if (p.a.shape < 0 || p.b.shape < 0) return -(int64_t)RV_ERR_UNSUPPORTED;
+  const int64_t a = part_bytes(p.a, ai, aj), b = part_bytes(p.b, bi, bj);
+  return (a > 0 ? align256(b) : b) + a;
+}
+
+// A weight gradient of a pair: out[ni][nj] (+)= sum_m a[m][ni] b[m][nj].
+struct WgradOperands {
+  const __half* a;
+  int64_t lda;
+  const __half* b;
+  int64_t ldb;
+  int64_t ni, nj;
+  float* out;
+};
+int run_pair(const WgradOperands& x, const WgradOperands& y, int64_t rows, int accumulate,
+             float* part, hipStream_t s) {
+  const PairPlan p = plan_pair(rows, x.ni, x.nj, y.ni, y.nj);
+  float* part_x = part + align256(part_bytes(p.b, y.ni, y.nj)) / (int64_t)sizeof(float);
+  const WgradJob jy = plan_job(p.b, y.a, y.lda, y.b, y.ldb, rows, y.ni, y.nj, y.out, accumulate, part);
+  const WgradJob jx = plan_job(p.a, x.a, x.lda, x.b, x.ldb, rows, x.ni, x.nj, x.out, accumulate, part_x);
+  int st;
+  if (p.paired) {
+    st = p.a.splits > 1 ? launch_pair<Epi::PartialF32>(jx, jy, s)
+                        : launch_pair<Epi::AccF32OfF16>(jx, jy, s);
+  } else {
+    st = launch_job(jy, s);
+    if (st == RV_OK) st = launch_job(jx, s);
+  }
+  if (st != RV_OK) return st;
+  return launch_reduce(jy.seg, jx.seg, accumulate, s);
+}
+
+bool ok16(const void* p) { return rv_host::aligned16(p); }
 
 // Buffer loads address an operand with 32-bit byte offsets.
 bool fits32(int64_t elems) { return elems > 0 && elems * 2 <= (int64_t)INT32_MAX - (int64_t)(1 << 24); }
@@ -1510,12 +1545,39 @@ int rv_linear_dw(const void* dy, const void* x, int64_t ldx, int64_t rows, int64
                    out, in, dw, accumulate, static_cast<float*>(workspace), (hipStream_t)stream);
 }
 
+int64_t rv_linear_dw_pair_workspace_bytes(int64_t rows, int64_t in_a, int64_t out_a, int64_t in_b,
+                                          int64_t out_b) {
+  if (rows <= 0 || in_a <= 0 || out_a <= 0 || in_b <= 0 || out_b <= 0)
+    return -(int64_t)RV_ERR_BAD_SIZE;
+  return pair_bytes(plan_pair(rows, out_a, in_a, out_b, in_b), out_a, in_a, out_b, in_b);
+}
+
+int rv_linear_dw_pair(const void* dy_a, const void* x_a, int64_t in_a, int64_t out_a, float* dw_a,
+                      const void* dy_b, const void* x_b, int64_t in_b, int64_t out_b, float* dw_b,
+                      int64_t rows, int accumulate, void* workspace, int64_t workspace_bytes,
+                      void* stream) {
+  if (!dy_a || !x_a || !dw_a || !dy_b || !x_b || !dw_b) return RV_ERR_NULL_POINTER;
+  if (rows <= 0 || in_a <= 0 || out_a <= 0 || in_b <= 0 || out_b <= 0) return RV_ERR_BAD_SIZE;
+  if (in_a % 128 || out_a % 128 || in_b % 128 || out_b % 128) return RV_ERR_UNSUPPORTED;
+  if (!ok16(dy_a) || !ok16(x_a) || !ok16(dw_a) || !ok16(dy_b) || !ok16(x_b) || !ok16(dw_b))
+    return RV_ERR_UNSUPPORTED;
+  if (!fits32(rows * out_a) || !fits32(rows * in_a) || !fits32(rows * out_b) ||
+      !fits32(rows * in_b))
+    return RV_ERR_UNSUPPORTED;
+  const int64_t need = rv_linear_dw_pair_workspace_bytes(rows, in_a, out_a, in_b, out_b);
+  if (need < 0) return (int)-need;
+  if (need > 0 && (workspace == nullptr || workspace_bytes < need || !ok16(workspace)))
+    return RV_ERR_WORKSPACE;
+  return run_pair({static_cast<const __half*>(dy_a), out_a, static_cast<const __half*>(x_a), in_a,
+                   out_a, in_a, dw_a},
+                  {static_cast<const __half*>(dy_b), out_b, static_cast<const __half*>(x_b), in_b,
+                   out_b, in_b, dw_b},
+                  rows, accumulate, static_cast<float*>(workspace), (hipStream_t)stream);
+}
+
 int64_t rv_mlp_wgrad_workspace_bytes(int64_t rows, int64_t d, int64_t f) {
   if (rows <= 0 || d <= 0 || f <= 0) return -(int64_t)RV_ERR_BAD_SIZE;
-  const PairPlan p = plan_mlp(rows, d, f);
-  if (p.a.shape < 0 || p.b.shape < 0) return -(int64_t)RV_ERR_UNSUPPORTED;
-  const int64_t down = part_bytes(p.b, d, f), up = part_bytes(p.a, 2 * f, d);
-  return (up > 0 ? align256(down) : down) + up;  // both at once (one reduction launch)
+  return pair_bytes(plan_pair(rows, 2 * f, d, d, f), 2 * f, d, d, f);
 }
 
 int rv_mlp_wgrad(const void* dy, const void* o, const void* du, const void* x, int64_t ldx,
@@ -1532,27 +1594,11 @@ int rv_mlp_wgrad(const void* dy, const void* o, const void* du, const void* x, i
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !ok16(workspace)))
     return RV_ERR_WORKSPACE;
   const hipStream_t s = (hipStream_t)stream;
-  // dW_down[d][f] = sum_m dy[m][d] o[m][f]; dW_up[2f][d] = sum_m du[m][j] x16[m][d],
-  // their partial sums side by side, reduced by one launch
-  const PairPlan p = plan_mlp(rows, d, f);
-  float* part_down = static_cast<float*>(workspace);
-  float* part_up = part_down + align256(part_bytes(p.b, d, f)) / (int64_t)sizeof(float);
-  const WgradJob down =
-      plan_job(p.b, static_cast<const __half*>(dy), d, static_cast<const __half*>(o), f, rows, d,
-               f, ddown, accumulate, part_down);
-  const WgradJob up =
-      plan_job(p.a, static_cast<const __half*>(du), 2 * f, static_cast<const __half*>(x), ldx,
-               rows, 2 * f, d, dup, accumulate, part_up);
-  int st;
-  if (p.paired) {
-    st = p.a.splits > 1 ? launch_pair<Epi::PartialF32>(up, down, s)
-                        : launch_pair<Epi::AccF32OfF16>(up, down, s);
-  } else {
-    st = launch_job(down, s);
-    if (st == RV_OK) st = launch_job(up, s);
-  }
-  if (st != RV_OK) return st;
-  return launch_reduce(down.seg, up.seg, accumulate, s);
+  // dW_up[2f][d] = sum_m du[m][j] x16[m][d], dW_down[d][f] = sum_m dy[m][d] o[m][f]
+  return run_pair({static_cast<const __half*>(du), 2 * f, static_cast<const __half*>(x), ldx, 2 * f,
+                   d, dup},
+                  {static_cast<const __half*>(dy), d, static_cast<const __half*>(o), f, d, f, ddown},
+                  rows, accumulate, static_cast<float*>(workspace), s);
 }
 
 }  // extern "C"

@@ -24,6 +24,7 @@ import types
 import torch
 import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import paths
 from ._hip import RV_F16, RV_F32, _check, _stream, library
@@ -111,5 +112,16 @@ def enable_linear(model: torch.nn.Module) -> None:
         return linear(x, layer.weight, layer.bias)
     for block in model.blocks:
         for layer in (block.attn.qkv, block.attn.proj):
-            layer.forward = types.MethodType(forward, layer)
+            layer.forward = layer._rv_forward = types.MethodType(forward, layer)
             layer._rv_linear = True  # its weight is cast by mlp.cast_weight
+
+
+def plain_layer(layer: torch.nn.Module) -> bool:
+    """Whether calling ``layer`` is exactly ``linear(x, layer.weight, None)``:
+    an ``nn.Linear`` as ``enable_linear`` left it -- no bias, no later patch
+    of its forward, no hooks of its own or global ones."""
+    return (type(layer) is torch.nn.Linear and layer.bias is None
+            and getattr(layer, "_rv_forward", None) is not None
+            and layer.forward is layer._rv_forward
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                     or layer._backward_pre_hooks or _has_any_global_hook()))

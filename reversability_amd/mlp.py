@@ -263,7 +263,8 @@ def wgrad(dy, o, du, x, ddown, dup, accumulate: bool) -> None:
     nbytes = lib.rv_mlp_wgrad_workspace_bytes(rows, d, f)
     if nbytes < 0:
         _check(-nbytes, "rv_mlp_wgrad_workspace_bytes")
-    ws = torch.empty(max(nbytes, 4) // 4, device=dy.device, dtype=torch.float32)
+    ws = torch.empty(nbytes // 4, device=dy.device, dtype=torch.float32) if nbytes else None
     _check(lib.rv_mlp_wgrad(dy.data_ptr(), o.data_ptr(), du.data_ptr(), x.data_ptr(),
                             x.stride(0), rows, d, f, ddown.data_ptr(), dup.data_ptr(),
-                            int(accumulate), ws.data_ptr(), nbytes, _stream(dy)), "rv_mlp_wgrad")
+                            int(accumulate), ws.data_ptr() if nbytes else None, nbytes,
+                            _stream(dy)), "rv_mlp_wgrad")

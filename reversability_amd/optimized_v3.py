@@ -124,6 +124,7 @@ class TiledMLP(torch.autograd.Function):
         flat = x.reshape(-1, x.shape[-1])
         output = torch.empty((flat.shape[0], down.shape[0]), device=x.device, dtype=cdt)
         mfma = _use_mfma(flat, up, down, fused, cdt)
+        ctx.mfma = mfma
         _record_mlp_path(flat, up, down, fused, cdt, mfma)
         if not need_output and not (keep_tiles and mfma):
             # the output is only differentiated and there are no tiles to keep:
@@ -136,10 +137,12 @@ class TiledMLP(torch.autograd.Function):
             # would produce on every tile
             x16, up16, down16 = mlp.cast_operands(flat.contiguous(), up, down)
             tiles = [] if keep_tiles else None
+            whole = flat.shape[0] <= tokens  # one tile: no slices
             for start in range(0, flat.shape[0], tokens):
-                o, u = mlp.up_swiglu(x16[start:start + tokens], up16, keep_u=keep_tiles)
+                o, u = mlp.up_swiglu(x16 if whole else x16[start:start + tokens], up16,
+                                     keep_u=keep_tiles)
                 if need_output:
-                    mlp.down(o, down16, output[start:start + tokens])
+                    mlp.down(o, down16, output if whole else output[start:start + tokens])
                 if keep_tiles:
                     tiles.append((o, u))
             ctx.tiles = tiles
@@ -167,7 +170,7 @@ class TiledMLP(torch.autograd.Function):
         flat = x.reshape(-1, x.shape[-1])
         dy = gradient.reshape(-1, gradient.shape[-1]).to(cdt)
         dx = torch.empty_like(flat)
-        if _use_mfma(flat, up, down, ctx.fused, cdt):
+        if ctx.mfma:
             from . import mlp
             dy = dy.contiguous()
             if cast:
@@ -176,16 +179,17 @@ class TiledMLP(torch.autograd.Function):
                 x16, up16, down16 = mlp.cast_operands(flat.contiguous(), up, down)
             dup, ddown = torch.empty_like(up), torch.empty_like(down)
             tiles, ctx.tiles = ctx.tiles, None
+            whole = flat.shape[0] <= ctx.tokens  # one tile: no slices
             for i, start in enumerate(range(0, flat.shape[0], ctx.tokens)):
                 stop = start + ctx.tokens
-                x_t, g = x16[start:stop], dy[start:stop]
+                x_t, g = (x16, dy) if whole else (x16[start:stop], dy[start:stop])
                 if tiles is not None:  # kept by the forward: the same values
                     o, u = tiles[i]
                     tiles[i] = None
                 else:
                     o, u = mlp.up_swiglu(x_t, up16, keep_u=True)
                 du = mlp.dgate(g, down16, u)
-                mlp.dx(du, up16, dx[start:stop])
+                mlp.dx(du, up16, dx if whole else dx[start:stop])
                 mlp.wgrad(g, o, du, x_t, ddown, dup, accumulate=i > 0)
                 del o, u, du
             return dx.reshape_as(x), dup, ddown, None, None, None, None

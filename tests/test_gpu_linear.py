@@ -146,3 +146,49 @@ def test_split_reduction(cuda_device, rows, in_f, out_f):
         lib.rv_gemm_force_shape(-1)
     assert lib.rv_linear_fwd_ws(x.data_ptr(), in_f, w.data_ptr(), rows, in_f, out_f,
                                 first[0].data_ptr(), ws.data_ptr(), need - 1, st) != 0
+
+
+@pytest.mark.parametrize("xdtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("batch,seq,heads,hd", [(1, 1, 4, 32), (3, 17, 8, 32), (2, 130, 4, 64),
+                                                (1, 257, 3, 128), (5, 96, 16, 64)])
+def test_attention_layer_matches_its_parts(cuda_device, batch, seq, heads, hd, xdtype):
+    """The one-node attention layer against the three Functions it stands for
+    (a forward hook on a projection keeps the parts): the same output and
+    input-gradient bits, weight gradients within 2e-3 (their rows are summed
+    in another order), frozen weights, and the same recorded paths."""
+    from reversability_amd import paths
+    from reversability_amd.attention import AttentionLayer, enable_attention
+    from reversability_amd.model import BaselineLM, ModelConfig
+    d = heads * hd
+    torch.manual_seed(3)
+    model = BaselineLM(ModelConfig(vocab_size=64, max_sequence_length=seq, n_layers=1,
+                                   n_heads=heads, d_model=d, d_ff=d)).to(cuda_device)
+    enable_linear(model)
+    enable_attention(model)
+    attn = model.blocks[0].attn
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(batch, seq, d, generator=g).to(cuda_device, xdtype).requires_grad_(True)
+    dy = torch.randn(batch, seq, d, generator=g).half().to(cuda_device)
+    leaves = (x, attn.qkv.weight, attn.proj.weight)
+
+    def once(wanted=leaves):
+        paths.reset()
+        with torch.autocast("cuda", dtype=torch.float16):
+            y = attn(x)
+        node = type(y.grad_fn).__name__
+        return y, torch.autograd.grad(y, wanted, dy), node, paths.report()
+
+    y, grads, node, report = once()
+    assert node == AttentionLayer.__name__ + "Backward"
+    frozen = once((x,))[1]
+    handle = attn.proj.register_forward_hook(lambda *a: None)
+    y_parts, grads_parts, node_parts, report_parts = once()
+    handle.remove()
+    assert node_parts != node and report == report_parts
+    assert torch.equal(y, y_parts) and torch.equal(grads[0], grads_parts[0])
+    assert torch.equal(frozen[0], grads[0])
+    for a, b in zip(grads[1:], grads_parts[1:]):
+        assert rel_l2(a, b) < 2e-3
+    attn.qkv.weight.requires_grad_(False)
+    partial = once((x, attn.proj.weight))[1]
+    assert torch.equal(partial[0], grads[0]) and torch.equal(partial[1], grads[2])
