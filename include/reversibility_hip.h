@@ -338,6 +338,26 @@ int rv_linear_fwd_ws(const void* x, int64_t ldx, const void* w, int64_t rows, in
 int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int64_t out, void* dx,
                     int dx_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The tied head's three products, fp16 with a vocabulary padded to a multiple
+ * of 64 (head rows vocab .. padded - 1 zero; logits row stride padded), d a
+ * multiple of 128 (src/reversibility/optimized_v3.py:151-192):
+ *   logits  logits[rows, padded] = fp16(x head^T), columns vocab .. zero
+ *   dx      dx[rows, d] = fp16(dlogits head), over all padded columns (the pad
+ *           columns of dlogits have to be finite)
+ *   dw      dw[vocab, d] = fp16(dlogits^T x), stored as fp16, or (+)= that
+ *           value widened to fp32
+ * rv_head_workspace_bytes covers dx and dw (one workspace may serve both in
+ * stream order). */
+int rv_head_logits(const void* x, const void* head, int64_t rows, int64_t d, int64_t vocab,
+                   int64_t padded, void* logits, void* stream);
+int64_t rv_head_workspace_bytes(int64_t rows, int64_t d, int64_t vocab, int64_t padded);
+int rv_head_dx(const void* dlogits, const void* head, int64_t rows, int64_t d, int64_t vocab,
+               int64_t padded, void* dx, void* workspace, int64_t workspace_bytes,
+               void* stream);
+int rv_head_dw(const void* dlogits, const void* x, int64_t rows, int64_t d, int64_t vocab,
+               int64_t padded, void* dw, int dw_dtype, int accumulate, void* workspace,
+               int64_t workspace_bytes, void* stream);
+
 /* Two layers' weight gradients over the same rows in one launch: dw_a[out_a,
  * in_a] (+)= fp32(fp16(dy_a^T x_a)) and dw_b likewise (x_a, x_b contiguous). */
 int64_t rv_linear_dw_pair_workspace_bytes(int64_t rows, int64_t in_a, int64_t out_a,

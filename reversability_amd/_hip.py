@@ -60,6 +60,10 @@ SIGNATURES = {
     "rv_linear_splitk_workspace_bytes": (_I64, [_I64, _I64, _I64]),
     "rv_linear_fwd_ws": (_I, [_P, _I64, _P, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "rv_linear_dx_ws": (_I, [_P, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _P]),
+    "rv_head_logits": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _P]),
+    "rv_head_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64]),
+    "rv_head_dx": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
+    "rv_head_dw": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _I, _I, _P, _I64, _P]),
     "rv_linear_dw_pair_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
     "rv_linear_dw_pair": (_I, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _I64, _P, _I64, _I, _P, _I64,
                                _P]),

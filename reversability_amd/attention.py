@@ -128,6 +128,7 @@ class AttentionLayer(torch.autograd.Function):
         _check(lib.rv_attn_bwd(qkv.data_ptr(), mixed.data_ptr(), dmixed.data_ptr(), lse.data_ptr(),
                                batch, seq, heads, d // heads, dqkv.data_ptr(), ws.data_ptr(),
                                nbytes, st), "rv_attn_bwd")
+        del dmixed, ws  # free for the buffers below
         dx = dw_qkv = dw_proj = None
         if ctx.needs_input_grad[0]:
             dx = torch.empty(batch, seq, d, device=dev, dtype=ctx.x_dtype)

@@ -129,11 +129,13 @@ __device__ __forceinline__ void lds_barrier() {
 // ---------------------------------------------------------------------------
 // Row maps for KC sources: LDS row r of the tile -> source row.
 // ---------------------------------------------------------------------------
+// Relative to origin, the row the copies' base address is moved to (so that
+// offsets stay 32-bit whatever the operand's size).
 struct MapDirect {  // row0 + r, clamped to the last valid row (results never stored)
   int64_t row0, rows;
+  __device__ __forceinline__ int64_t origin() const { return row0; }
   __device__ __forceinline__ int64_t operator()(int r) const {
-    const int64_t g = row0 + r;
-    return g < rows ? g : rows - 1;
+    return row0 + r < rows ? r : rows - 1 - row0;
   }
 };
 // SwiGLU up projection: a BN-row B tile holds BN/2 output columns, as gate
@@ -143,6 +145,7 @@ struct MapDirect {  // row0 + r, clamped to the last valid row (results never st
 template <int BN, int WCOLS>
 struct MapGateValue {
   int64_t col0, f;
+  __device__ __forceinline__ int64_t origin() const { return 0; }
   __device__ __forceinline__ int64_t operator()(int r) const {
     constexpr int kCol = BN / WCOLS, kHalf = kCol / 2;
     const int wn = r / kCol, w = r % kCol;
@@ -184,8 +187,9 @@ struct Dma {
   template <class Map>
   __device__ __forceinline__ void init_kc(const __half* p, int64_t bytes, int64_t ld,
                                           const Map& map, int64_t kbeg, int wave, int lane) {
-    base = uniform(reinterpret_cast<int64_t>(p + kbeg));
-    left = uniform(bytes - kbeg * 2);
+    const int64_t first = map.origin() * ld + kbeg;
+    base = uniform(reinterpret_cast<int64_t>(p + first));
+    left = uniform(bytes - first * 2);
     kstep = BK * 2;
 #pragma unroll
     for (int it = 0; it < kPerWave; ++it) {
@@ -219,7 +223,8 @@ struct Dma {
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t stage(int st, bool live) const {
     const int64_t at = (int64_t)st * kstep, n = left - at;
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(base + at), 0,
-                                             live && n > 0 ? (int)n : 0, kRsrcWord3);
+                                             !live || n <= 0 ? 0 : n < INT32_MAX ? (int)n : INT32_MAX,
+                                             kRsrcWord3);
   }
   // Wave instruction `it` of a stage into the tile at `lds`.
   __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rsrc, _Float16* lds, int it,
@@ -324,6 +329,7 @@ struct GemmArgs {
   void* u; int64_t ldu;    // SwiGLU: optional u output; SwiGLUBwd: u input
   int64_t f;               // SwiGLU / SwiGLUBwd: value column offset
   int accumulate;          // AccF32OfF16
+  int64_t valid;           // StoreF16: columns valid .. n - 1 are written as zero (0: none)
 };
 
 // Workgroups are dispatched to the 8 XCDs round robin.  Tiles are numbered in
@@ -676,8 +682,14 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) 
 #pragma unroll 4
       for (int r = lane / CPR; r < WM; r += RPP) {
         const int64_t row = row0 + r;
-        if (row >= args.m) break;
-        const u32x4 dw = *reinterpret_cast<const u32x4*>(stage + r * S + c * 8);
+        if (row >= args.m || col >= args.n) break;
+        u32x4 dw = *reinterpret_cast<const u32x4*>(stage + r * S + c * 8);
+        if (args.valid != 0 && col + 8 > args.valid) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (col + e >= args.valid)
+              dw[e >> 1] = (e & 1) ? dw[e >> 1] & 0xffffu : dw[e >> 1] & 0xffff0000u;
+        }
         __builtin_nontemporal_store(dw, reinterpret_cast<u32x4*>(static_cast<__half*>(args.c) + row * args.ldc + col));
       }
     } else {
@@ -775,6 +787,7 @@ void wgrad_pair_kernel(GemmPair pair) {
   template __global__ void gemm_kernel<SHAPE, false, true, Epi::PartialF32>(GemmArgs);
 #define RV_WGRAD_KERNELS(SHAPE)                                                       \
   template __global__ void gemm_kernel<SHAPE, true, true, Epi::AccF32OfF16>(GemmArgs); \
+  template __global__ void gemm_kernel<SHAPE, true, true, Epi::StoreF16>(GemmArgs);      \
   template __global__ void gemm_kernel<SHAPE, true, true, Epi::PartialF32>(GemmArgs);    \
   template __global__ void wgrad_pair_kernel<SHAPE, Epi::AccF32OfF16>(GemmPair);         \
   template __global__ void wgrad_pair_kernel<SHAPE, Epi::PartialF32>(GemmPair);
@@ -968,13 +981,14 @@ int launch(int shape, const GemmArgs& a, int64_t splits, hipStream_t s) {
 // Activation GEMMs: C is m x n_out where n_out = n (or n/2 output columns for
 // SwiGLU, whose tile covers bn/2 of them).  The largest tile that gives at
 // least one workgroup per CU; otherwise the one with the most workgroups.
-int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits) {
+int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits, bool ragged) {
   int best = -1;
   int64_t best_blocks = -1;
   for (int i = 0; i < kRuleShapes; ++i) {
     const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
-    if (n_cols % cols) continue;
-    const int64_t blocks = ((m + kShapes[i].bm - 1) / kShapes[i].bm) * (n_cols / cols) * splits;
+    if (n_cols % cols && !ragged) continue;
+    const int64_t blocks =
+        ((m + kShapes[i].bm - 1) / kShapes[i].bm) * ((n_cols + cols - 1) / cols) * splits;
     if (blocks >= kCUs) return i;
     if (blocks > best_blocks) best = i, best_blocks = blocks;
   }
@@ -1019,12 +1033,13 @@ int launch_shape(int shape, GemmArgs a, int64_t n_cols, hipStream_t s) {
   const bool swiglu = EPI == Epi::SwiGLU;
   const TileShape t = kShapes[shape];
   a.tiles_m = (a.m + t.bm - 1) / t.bm;
-  a.tiles_n = n_cols / (swiglu ? t.bn / 2 : t.bn);
+  const int64_t cols = swiglu ? t.bn / 2 : t.bn;
+  a.tiles_n = (n_cols + cols - 1) / cols;
   return launch<A_RC, B_RC, EPI>(shape, a, (a.k + a.k_chunk - 1) / a.k_chunk, s);
 }
 
 template <bool A_RC, bool B_RC, Epi EPI>
-int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
+int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback, bool ragged) {
   const bool swiglu = EPI == Epi::SwiGLU;
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return fallback;
@@ -1038,7 +1053,7 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
   for (int sweep = 0; sweep < 2; ++sweep)
     for (int i = 0; i < kNumShapes; ++i) {
       const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
-      if (n_cols % cols) continue;
+      if (n_cols % cols && !ragged) continue;
       if (launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) != RV_OK) continue;
       bool ok = hipEventRecord(e0, s) == hipSuccess;
       ok = ok && launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) == RV_OK;
@@ -1058,15 +1073,16 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
 }
 
 template <bool A_RC, bool B_RC, Epi EPI>
-int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
+int run_act(GemmArgs a, int64_t n_cols, hipStream_t s, bool ragged = false) {
   const bool swiglu = EPI == Epi::SwiGLU;
   if (EPI != Epi::PartialF32) a.k_chunk = a.k;
   const int64_t splits = (a.k + a.k_chunk - 1) / a.k_chunk;
-  int shape = pick_act(a.m, n_cols, swiglu, splits);
+  int shape = pick_act(a.m, n_cols, swiglu, splits, ragged);
   if (shape < 0) return RV_ERR_UNSUPPORTED;
   const int forced = g_forced_shape.load();
   if (forced >= 0) {
-    if (n_cols % (swiglu ? kShapes[forced].bn / 2 : kShapes[forced].bn)) return RV_ERR_UNSUPPORTED;
+    if (n_cols % (swiglu ? kShapes[forced].bn / 2 : kShapes[forced].bn) && !ragged)
+      return RV_ERR_UNSUPPORTED;
     return launch_shape<A_RC, B_RC, EPI>(forced, a, n_cols, s);
   }
   if (tuning_enabled()) {
@@ -1074,7 +1090,7 @@ int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
     (void)hipGetDevice(&device);
     // the SwiGLU epilogue with and without its u output store different
     // amounts and are tuned apart
-    const int variant = (EPI == Epi::SwiGLU && a.u != nullptr) ? 1 : 0;
+    const int variant = (EPI == Epi::SwiGLU && a.u != nullptr) ? 1 : ragged ? 2 : 0;
     const TuneKey key{(int)EPI * 4 + (A_RC ? 2 : 0) + (B_RC ? 1 : 0), device, variant, a.m,
                       n_cols, EPI == Epi::PartialF32 ? a.k * 64 + splits : a.k};
     std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -1082,7 +1098,7 @@ int run_act(GemmArgs a, int64_t n_cols, hipStream_t s) {
     if (it != g_tuned.end()) {
       shape = it->second;
     } else if (!capturing(s)) {
-      shape = tune_act<A_RC, B_RC, EPI>(a, n_cols, s, shape);
+      shape = tune_act<A_RC, B_RC, EPI>(a, n_cols, s, shape, ragged);
       g_tuned[key] = shape;
     }
   }
@@ -1123,9 +1139,9 @@ int64_t act_part_bytes(int64_t m, int64_t n, int64_t k) {
   return splits > 1 ? splits * m * n * (int64_t)sizeof(float) : 0;
 }
 
+// a.k_chunk set; fp32 partials of each chunk in `part`, summed into out.
 template <bool B_RC, typename T>
 int run_split(GemmArgs a, T* out, float* part, hipStream_t s) {
-  a.k_chunk = act_chunk(a.m, a.n, a.k);
   a.c = part;
   a.ldc = a.n;
   const int st = run_act<false, B_RC, Epi::PartialF32>(a, a.n, s);
@@ -1152,7 +1168,8 @@ struct WgradPlan {
   int shape;
   int64_t tiles_m, tiles_n, splits, chunk;
 };
-bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, double& cost) {
+bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, double& cost,
+                bool ragged = false) {
   // per-shape efficiencies measured on the split-K weight gradients (the
   // 128 x 256 tile's 0.55: at C5's attention-projection shape, 1024 x 1024
   // over 32768 tokens, it took 113 us with 8 splits where 256 x 256 with 16
@@ -1163,8 +1180,8 @@ bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, do
   // over 16896)
   static const double eff[kRuleShapes] = {0.8, 0.55, 0.5, 0.42};
   const TileShape t = kShapes[i];
-  if (ni % t.bm || nj % t.bn) return false;
-  const int64_t tiles = (ni / t.bm) * (nj / t.bn);
+  if ((ni % t.bm && !ragged) || nj % t.bn) return false;
+  const int64_t tiles_i = (ni + t.bm - 1) / t.bm, tiles = tiles_i * (nj / t.bn);
   int64_t splits = tiles >= kCUs ? 1 : kCUs / tiles;
   const int64_t max_splits = (rows + 2 * kSplitStep - 1) / (2 * kSplitStep);
   if (splits > max_splits) splits = max_splits;
@@ -1178,14 +1195,15 @@ bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, do
   const double flops = 2.0 * rows * ni * nj / (eff[i] * fill);
   const double bytes = splits > 1 ? 8.0 * splits * ni * nj : 0.0;
   cost = flops + 250.0 * bytes;
-  plan = WgradPlan{i, ni / t.bm, nj / t.bn, splits, chunk};
+  plan = WgradPlan{i, tiles_i, nj / t.bn, splits, chunk};
   return true;
 }
-WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj) {
+// ragged: ni need not be a multiple of the tile (rows past it are not stored).
+WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj, bool ragged = false) {
   WgradPlan best{-1, 0, 0, 0, 0}, plan;
   double best_cost = 0, cost;
   for (int i = 0; i < kRuleShapes; ++i)
-    if (plan_shape(i, rows, ni, nj, plan, cost) && (best.shape < 0 || cost < best_cost)) {
+    if (plan_shape(i, rows, ni, nj, plan, cost, ragged) && (best.shape < 0 || cost < best_cost)) {
       best = plan;
       best_cost = cost;
     }
@@ -1320,6 +1338,34 @@ int run_pair(const WgradOperands& x, const WgradOperands& y, int64_t rows, int a
 }
 
 bool ok16(const void* p) { return rv_host::aligned16(p); }
+
+// Splits of the tied head's input gradient (rows x d over the vocabulary): as
+// act_splits where even 64 x 128 tiles leave the chip half empty; otherwise the
+// largest count that keeps the 256 x 256 tiles within one round of the CUs
+// (16896 x 256 over 50304, us by splits: 1 682, 2 531, 3 441, 5 522, 7 444, 8 517).
+int64_t head_chunk(int64_t rows, int64_t d, int64_t k) {
+  int64_t splits = act_splits(rows, d, k);
+  if (splits == 1) {
+    const int64_t tiles = ((rows + 255) / 256) * ((d + 255) / 256);
+    splits = tiles < kCUs ? kCUs / tiles : 1;
+    const int64_t most = k / 2048 > 1 ? k / 2048 : 1;  // partials' traffic below the operand's
+    if (splits > most) splits = most;
+  }
+  return ((k + splits - 1) / splits + kSplitStep - 1) / kSplitStep * kSplitStep;
+}
+int64_t head_dx_bytes(int64_t rows, int64_t d, int64_t k) {
+  const int64_t chunk = head_chunk(rows, d, k), splits = (k + chunk - 1) / chunk;
+  return splits > 1 ? splits * rows * d * (int64_t)sizeof(float) : 0;
+}
+
+// A tile's rows of an operand with this row stride stay within 32-bit offsets.
+bool span32(int64_t ld) { return ld > 0 && 256 * ld * 2 <= (int64_t)INT32_MAX - (int64_t)(1 << 24); }
+
+int head_check(int64_t rows, int64_t d, int64_t vocab, int64_t padded) {
+  if (rows <= 0 || d <= 0 || vocab <= 0 || padded < vocab) return RV_ERR_BAD_SIZE;
+  if (d % 128 || padded % 64 || !span32(padded) || !span32(d)) return RV_ERR_UNSUPPORTED;
+  return RV_OK;
+}
 
 // Buffer loads address an operand with 32-bit byte offsets.
 bool fits32(int64_t elems) { return elems > 0 && elems * 2 <= (int64_t)INT32_MAX - (int64_t)(1 << 24); }
@@ -1496,7 +1542,7 @@ int rv_linear_fwd_ws(const void* x, int64_t ldx, const void* w, int64_t rows, in
   GemmArgs a{};
   a.a = static_cast<const __half*>(x); a.lda = ldx; a.a_bytes = rows * ldx * 2;
   a.b = static_cast<const __half*>(w); a.ldb = in; a.b_bytes = out * in * 2;
-  a.m = rows; a.n = out; a.k = in;
+  a.m = rows; a.n = out; a.k = in; a.k_chunk = act_chunk(rows, out, in);
   return run_split<false>(a, static_cast<__half*>(y), static_cast<float*>(workspace),
                           (hipStream_t)stream);
 }
@@ -1515,7 +1561,7 @@ int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int
   a.a = static_cast<const __half*>(dy); a.lda = out; a.a_bytes = rows * out * 2;
   a.b = static_cast<const __half*>(w); a.ldb = in;  // B(i, o) = W[o][i]: RC
   a.b_bytes = out * in * 2;
-  a.m = rows; a.n = in; a.k = out;
+  a.m = rows; a.n = in; a.k = out; a.k_chunk = act_chunk(rows, in, out);
   const hipStream_t s = (hipStream_t)stream;
   float* part = static_cast<float*>(workspace);
   return dx_dtype == RV_F16 ? run_split<true>(a, static_cast<__half*>(dx), part, s)
@@ -1543,6 +1589,80 @@ int rv_linear_dw(const void* dy, const void* x, int64_t ldx, int64_t rows, int64
   // dW[out][in] = sum_m dy[m][o] x[m][i]
   return run_wgrad(static_cast<const __half*>(dy), out, static_cast<const __half*>(x), ldx, rows,
                    out, in, dw, accumulate, static_cast<float*>(workspace), (hipStream_t)stream);
+}
+
+int rv_head_logits(const void* x, const void* head, int64_t rows, int64_t d, int64_t vocab,
+                   int64_t padded, void* logits, void* stream) {
+  if (!x || !head || !logits) return RV_ERR_NULL_POINTER;
+  const int bad = head_check(rows, d, vocab, padded);
+  if (bad) return bad;
+  if (!ok16(x) || !ok16(head) || !ok16(logits)) return RV_ERR_UNSUPPORTED;
+  GemmArgs a{};
+  a.a = static_cast<const __half*>(x); a.lda = d; a.a_bytes = rows * d * 2;
+  a.b = static_cast<const __half*>(head); a.ldb = d; a.b_bytes = padded * d * 2;
+  a.m = rows; a.n = padded; a.k = d;
+  a.c = logits; a.ldc = padded; a.valid = vocab;
+  return run_act<false, false, Epi::StoreF16>(a, padded, (hipStream_t)stream, true);
+}
+
+int64_t rv_head_workspace_bytes(int64_t rows, int64_t d, int64_t vocab, int64_t padded) {
+  const int bad = head_check(rows, d, vocab, padded);
+  if (bad) return -(int64_t)bad;
+  const WgradPlan p = plan_wgrad(rows, vocab, d, true);
+  if (p.shape < 0) return -(int64_t)RV_ERR_UNSUPPORTED;
+  const int64_t dx = head_dx_bytes(rows, d, padded), dw = part_bytes(p, vocab, d);
+  return dx > dw ? dx : dw;
+}
+
+int rv_head_dx(const void* dlogits, const void* head, int64_t rows, int64_t d, int64_t vocab,
+               int64_t padded, void* dx, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!dlogits || !head || !dx) return RV_ERR_NULL_POINTER;
+  const int bad = head_check(rows, d, vocab, padded);
+  if (bad) return bad;
+  if (!ok16(dlogits) || !ok16(head) || !ok16(dx)) return RV_ERR_UNSUPPORTED;
+  GemmArgs a{};
+  a.a = static_cast<const __half*>(dlogits); a.lda = padded; a.a_bytes = rows * padded * 2;
+  a.b = static_cast<const __half*>(head); a.ldb = d;  // B(d, v) = head[v][d]: RC
+  a.b_bytes = padded * d * 2;
+  a.m = rows; a.n = d; a.k = padded; a.k_chunk = head_chunk(rows, d, padded);
+  const hipStream_t s = (hipStream_t)stream;
+  const int64_t need = head_dx_bytes(rows, d, padded);
+  if (need == 0) {
+    a.c = dx; a.ldc = d;
+    return run_act<false, true, Epi::StoreF16>(a, d, s);
+  }
+  if (!workspace || workspace_bytes < need || !ok16(workspace)) return RV_ERR_WORKSPACE;
+  return run_split<true>(a, static_cast<__half*>(dx), static_cast<float*>(workspace), s);
+}
+
+int rv_head_dw(const void* dlogits, const void* x, int64_t rows, int64_t d, int64_t vocab,
+               int64_t padded, void* dw, int dw_dtype, int accumulate, void* workspace,
+               int64_t workspace_bytes, void* stream) {
+  if (!dlogits || !x || !dw) return RV_ERR_NULL_POINTER;
+  const int bad = head_check(rows, d, vocab, padded);
+  if (bad) return bad;
+  if (dw_dtype != RV_F32 && (dw_dtype != RV_F16 || accumulate)) return RV_ERR_UNSUPPORTED;
+  if (!ok16(dlogits) || !ok16(x) || !ok16(dw)) return RV_ERR_UNSUPPORTED;
+  const WgradPlan p = plan_wgrad(rows, vocab, d, true);
+  if (p.shape < 0) return RV_ERR_UNSUPPORTED;
+  const int64_t need = part_bytes(p, vocab, d);
+  if (need > 0 && (!workspace || workspace_bytes < need || !ok16(workspace)))
+    return RV_ERR_WORKSPACE;
+  const hipStream_t s = (hipStream_t)stream;
+  float* part = static_cast<float*>(workspace);
+  // dW[v][d] = sum_m dlogits[m][v] x[m][d]
+  WgradJob j = plan_job(p, static_cast<const __half*>(dlogits), padded,
+                        static_cast<const __half*>(x), d, rows, vocab, d,
+                        static_cast<float*>(dw), accumulate, part);
+  if (dw_dtype == RV_F16 && p.splits == 1)
+    return launch<true, true, Epi::StoreF16>(p.shape, j.g, 1, s);
+  const int st = launch_job(j, s);
+  if (st != RV_OK) return st;
+  if (dw_dtype == RV_F32) return launch_reduce(j.seg, ReduceSeg{}, accumulate, s);
+  const int64_t n = vocab * d;
+  hipLaunchKernelGGL(act_reduce<__half>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
+                     part, static_cast<__half*>(dw), n, (int)p.splits);
+  return rv_host::check_launch();
 }
 
 int64_t rv_linear_dw_pair_workspace_bytes(int64_t rows, int64_t in_a, int64_t out_a, int64_t in_b,

@@ -66,7 +66,8 @@ FUSED_CE_MAX_COLS = 65536
 
 
 def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: torch.Tensor,
-                 grad: torch.Tensor, dx_out: torch.Tensor | None = None):
+                 grad: torch.Tensor, dx_out: torch.Tensor | None = None,
+                 dw_out: torch.Tensor | None = None, accumulate: bool = False):
     """One chunk of the tied head and its summed cross-entropy, forward and
     backward, with the logits stored at a padded row stride.
 
@@ -75,12 +76,15 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     gradient ``grad`` (a device fp32 scalar): logits = fp16(x16 W^T); loss and
     dlogits from one pass of rv_ce_fused over each logits row (the two-pass
     rv_ce_fwd / rv_ce_bwd above FUSED_CE_MAX_COLS, same bits); dx = dlogits W and
-    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  ``head16`` is
-    the fp16 head with its rows padded to a multiple of VOCAB_ALIGN (the pad
-    rows zero), so every logits row starts 16-byte aligned: with the odd
-    vocabulary (50257) as the row stride, hipBLASLt's GEMMs over the logits
-    run 15-25% slower on MI355X.  Returns (loss sum, dx16, dW16 [vocab, d]);
-    dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when given.
+    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The three
+    products run on the MFMA kernels (``head_supported``; 16896 x 256 over 50257:
+    logits 685 -> 637 us against torch's GEMM, dx 566 -> 448, dW 554 -> 442), otherwise
+    on torch's GEMMs.  ``head16`` is the fp16 head with its rows padded to a
+    multiple of VOCAB_ALIGN (the pad rows zero), so every logits row starts
+    16-byte aligned.  Returns (loss sum, dx16, dW16 [vocab, d]);
+    dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when given, and
+    dW -- the same fp16 values widened -- into ``dw_out`` (contiguous fp32 [vocab,
+    d]; added to it with ``accumulate``), which is then returned for dW16.
     """
     rows, d = x16.shape
     padded = head16.shape[0]
@@ -90,10 +94,19 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
             or labels.numel() != rows or not x16.is_cuda):
         raise ValueError("tied_head_ce needs contiguous CUDA fp16 x [rows, d], a padded fp16 "
                          "head [padded, d] and int64 labels [rows]")
-    from ._hip import RV_F16, _check, _stream, library
+    from ._hip import RV_F16, RV_F32, _check, _stream, library
     lib = library()
     labels = labels.contiguous()
-    logits = torch.mm(x16, head16.t())                       # [rows, padded] fp16
+    own = (head_supported(rows, d, padded)
+           and x16.data_ptr() % 16 == 0 and head16.data_ptr() % 16 == 0
+           and (dx_out is None or (dx_out.dtype == torch.float16 and dx_out.is_contiguous()
+                                   and dx_out.shape == x16.shape and dx_out.data_ptr() % 16 == 0)))
+    if own:
+        logits = torch.empty(rows, padded, device=x16.device, dtype=torch.float16)
+        _check(lib.rv_head_logits(x16.data_ptr(), head16.data_ptr(), rows, d, vocab, padded,
+                                  logits.data_ptr(), _stream(x16)), "rv_head_logits")
+    else:
+        logits = torch.mm(x16, head16.t())                   # [rows, padded] fp16
     rmax, rlse, losses = (torch.empty(rows, device=x16.device, dtype=torch.float32)
                           for _ in range(3))
     st = _stream(x16)
@@ -105,6 +118,8 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
                                losses.data_ptr(), dlogits.data_ptr(), st), "rv_ce_fused")
     else:
         dlogits = torch.empty_like(logits)
+        if own:
+            dlogits[:, vocab:].zero_()  # rv_head_dx reads the pad columns
         if rows:
             _check(lib.rv_ce_fwd(logits.data_ptr(), RV_F16, padded, labels.data_ptr(), rows,
                                  vocab, IGNORE_INDEX, rmax.data_ptr(), rlse.data_ptr(),
@@ -113,13 +128,41 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
                                  rmax.data_ptr(), rlse.data_ptr(), grad.data_ptr(), rows, vocab,
                                  IGNORE_INDEX, dlogits.data_ptr(), st), "rv_ce_bwd")
     del logits
+    if own:
+        nbytes = lib.rv_head_workspace_bytes(rows, d, vocab, padded)
+        if nbytes < 0:
+            _check(-nbytes, "rv_head_workspace_bytes")
+        ws = torch.empty(nbytes // 4, device=x16.device, dtype=torch.float32) if nbytes else None
+        ws_ptr = ws.data_ptr() if nbytes else None
+        dx16 = dx_out if dx_out is not None else torch.empty_like(x16)
+        _check(lib.rv_head_dx(dlogits.data_ptr(), head16.data_ptr(), rows, d, vocab, padded,
+                              dx16.data_ptr(), ws_ptr, nbytes, st), "rv_head_dx")
+        dw = dw_out if dw_out is not None else torch.empty(vocab, d, device=x16.device,
+                                                           dtype=torch.float16)
+        _check(lib.rv_head_dw(dlogits.data_ptr(), x16.data_ptr(), rows, d, vocab, padded,
+                              dw.data_ptr(), RV_F16 if dw_out is None else RV_F32,
+                              int(accumulate and dw_out is not None), ws_ptr, nbytes, st),
+               "rv_head_dw")
+        return losses.sum(), dx16, dw
     d_view = dlogits[:, :vocab]
     if dx_out is not None:
         dx16 = torch.mm(d_view, head16[:vocab], out=dx_out)
     else:
         dx16 = torch.mm(d_view, head16[:vocab])
     dw16 = torch.mm(d_view.t(), x16)
-    return losses.sum(), dx16, dw16
+    if dw_out is None:
+        return losses.sum(), dx16, dw16
+    if accumulate:
+        dw_out.add_(dw16)
+    else:
+        dw_out.copy_(dw16)
+    return losses.sum(), dx16, dw_out
+
+
+def head_supported(rows: int, d: int, padded: int) -> bool:
+    """Whether the MFMA kernels take a head of this size (widths that are
+    multiples of 128; a 256-row tile of the logits within 2 GiB)."""
+    return rows > 0 and d % 128 == 0 and 512 * padded < (1 << 31) - (1 << 24)
 
 
 def padded_head(weight: torch.Tensor) -> torch.Tensor:

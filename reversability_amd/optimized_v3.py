@@ -359,17 +359,22 @@ def _fused_head(hidden, weight, labels, denominator, chunk_tokens, scaler, preci
         stop = start + chunk_tokens
         rows = dflat[start:stop]
         direct = rows.dtype == torch.float16 and rows.is_contiguous()
-        loss, dx16, dw16 = tied_head_ce(x16[start:stop], head16, vocab, targets[start:stop],
-                                        grad.reshape(1), dx_out=rows if direct else None)
+        # the head's gradient goes straight into the tied weight's (fp32)
+        first = weight.grad is None
+        sink = torch.empty_like(weight) if first else weight.grad
+        direct_dw = (sink.is_contiguous() and sink.dtype == torch.float32
+                     and sink.data_ptr() % 16 == 0)
+        loss, dx16, dw = tied_head_ce(x16[start:stop], head16, vocab, targets[start:stop],
+                                      grad.reshape(1), dx_out=rows if direct else None,
+                                      dw_out=sink if direct_dw else None, accumulate=not first)
         if not direct:
             rows.copy_(dx16)
-        chunk_grad = dw16.to(weight.dtype)
-        if weight.grad is None:
-            weight.grad = chunk_grad
-        else:
-            weight.grad.add_(chunk_grad)
+        if first:
+            weight.grad = sink if direct_dw else dw.to(weight.dtype)
+        elif not direct_dw:
+            weight.grad.add_(dw.to(weight.dtype))
         total += loss.detach().float()
-        del dx16, dw16, chunk_grad
+        del dx16, dw, sink
     del head16, x16
     with amp_context(device, precision):
         hidden.backward(dflat.reshape_as(hidden))
@@ -470,7 +475,10 @@ def _cached_head_backward(model, ids, labels, denominator, chunk_tokens, scaler,
     weight = model.lm_head.weight
     if (loss_backend in ("triton", "hip") and precision == "fp16" and ids.device.type == "cuda"
             and weight.dtype == torch.float32):
-        _paths.took("tied_head", "fused-ce+hipblaslt")
+        from .kernels import VOCAB_ALIGN, head_supported
+        padded = -(-weight.shape[0] // VOCAB_ALIGN) * VOCAB_ALIGN
+        own = head_supported(labels.numel(), weight.shape[1], padded)
+        _paths.took("tied_head", "fused-ce+mfma" if own else "fused-ce+hipblaslt")
         return _fused_head(hidden, weight, labels, denominator, chunk_tokens, scaler, precision,
                            ids.device)
     if loss_backend in ("triton", "hip") and ids.device.type == "cuda":

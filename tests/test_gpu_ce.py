@@ -241,3 +241,94 @@ def test_fused_matches_oracle_and_rejects_wide_rows(cuda_device):
             loss.data_ptr(), wide.data_ptr(), _stream(wide))
     assert lib.rv_ce_fused(wide.data_ptr(), RV_F16, 65544, *args) == RV_ERR_UNSUPPORTED
     assert lib.rv_ce_fused(wide.data_ptr(), RV_F32, 65544, *args) == RV_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows,d,vocab", [(1, 128, 161), (65, 256, 1001), (300, 384, 192),
+                                           (513, 128, 7000), (700, 256, 9999)])
+def test_head_products(cuda_device, rows, d, vocab):
+    """The head's three GEMMs at vocabularies whose padded width is not a
+    multiple of the tiles: the fp64 bound, identical bits on every tile shape,
+    pad columns zero also for a row of infinities, dW as fp16, widened, and
+    accumulated, from one workspace."""
+    from gemm_bounds import within_gemm_bound
+    from reversability_amd._hip import RV_F16, RV_F32, _stream, library
+    lib = library()
+    padded = -(-vocab // 64) * 64
+    g = torch.Generator().manual_seed(19)
+    x = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    head = torch.zeros(padded, d)
+    head[:vocab] = 0.05 * torch.randn(vocab, d, generator=g)
+    head = head.half().to(cuda_device)
+    grad = torch.zeros(rows, padded)
+    grad[:, :vocab] = 1e-2 * torch.randn(rows, vocab, generator=g)
+    grad = grad.half().to(cuda_device)
+    size = (rows, d, vocab, padded)
+    st = _stream(x)
+    nbytes = lib.rv_head_workspace_bytes(*size)
+    assert nbytes >= 0
+    ws = torch.empty(max(nbytes, 16) // 4, device=cuda_device)
+    first = None
+    try:
+        for shape in range(-1, lib.rv_gemm_num_shapes()):
+            assert lib.rv_gemm_force_shape(shape) == 0
+            logits = torch.full((rows, padded), 3.0, device=cuda_device, dtype=torch.float16)
+            dx = torch.empty_like(x)
+            assert lib.rv_head_logits(x.data_ptr(), head.data_ptr(), *size, logits.data_ptr(),
+                                      st) == 0
+            rc = lib.rv_head_dx(grad.data_ptr(), head.data_ptr(), *size, dx.data_ptr(),
+                                ws.data_ptr(), nbytes, st)
+            if rc == 3 and shape >= 0:  # d does not divide this tile
+                dx = first[1]
+            else:
+                assert rc == 0
+            if first is None:
+                first = (logits, dx)
+                assert within_gemm_bound(logits, x, head, d)
+                assert within_gemm_bound(dx, grad, head, padded, transpose_b=False)
+            assert torch.equal(logits, first[0]) and torch.equal(dx, first[1]), shape
+    finally:
+        lib.rv_gemm_force_shape(-1)
+    dw16 = torch.empty(vocab, d, device=cuda_device, dtype=torch.float16)
+    dw32 = torch.empty(vocab, d, device=cuda_device)
+    call = lambda out, code, acc: lib.rv_head_dw(
+        grad.data_ptr(), x.data_ptr(), *size, out.data_ptr(), code, acc, ws.data_ptr(), nbytes, st)
+    assert call(dw16, RV_F16, 0) == 0 and call(dw32, RV_F32, 0) == 0
+    assert within_gemm_bound(dw16, grad[:, :vocab].t(), x.t(), rows)
+    assert torch.equal(dw32, dw16.float())
+    assert call(dw32, RV_F32, 1) == 0
+    assert torch.equal(dw32, 2 * dw16.float())
+    x[0] = float("inf")
+    assert lib.rv_head_logits(x.data_ptr(), head.data_ptr(), *size, logits.data_ptr(), st) == 0
+    assert not logits[:, vocab:].any()
+
+
+def test_head_products_past_32_bit_offsets(cuda_device):
+    """A logits matrix above 2 GiB: its last rows' logits and input gradient and
+    the whole weight gradient (whose sum runs past the 2 GiB mark) against
+    fp32 products of the same operands."""
+    from reversability_amd._hip import RV_F32, _stream, library
+    lib = library()
+    rows, d, vocab, padded = 22000, 128, 50257, 50304
+    assert rows * padded * 2 > 1 << 31
+    g = torch.Generator(device=cuda_device).manual_seed(3)
+    x = torch.randn(rows, d, generator=g, device=cuda_device).half()
+    head = torch.zeros(padded, d, device=cuda_device, dtype=torch.float16)
+    head[:vocab] = 0.05 * torch.randn(vocab, d, generator=g, device=cuda_device)
+    size, st = (rows, d, vocab, padded), _stream(x)
+    logits = torch.empty(rows, padded, device=cuda_device, dtype=torch.float16)
+    assert lib.rv_head_logits(x.data_ptr(), head.data_ptr(), *size, logits.data_ptr(), st) == 0
+    nbytes = lib.rv_head_workspace_bytes(*size)
+    ws = torch.empty(max(nbytes, 16) // 4, device=cuda_device)
+    dx, dw = torch.empty_like(x), torch.empty(vocab, d, device=cuda_device)
+    assert lib.rv_head_dx(logits.data_ptr(), head.data_ptr(), *size, dx.data_ptr(), ws.data_ptr(),
+                          nbytes, st) == 0
+    assert lib.rv_head_dw(logits.data_ptr(), x.data_ptr(), *size, dw.data_ptr(), RV_F32, 0,
+                          ws.data_ptr(), nbytes, st) == 0
+    rel = lambda a, b: float((a.float() - b).norm() / b.norm())
+    for rows_ in (slice(0, 64), slice(-64, None)):
+        assert rel(logits[rows_], x[rows_].float() @ head.float().t()) < 1e-3
+        assert rel(dx[rows_], logits[rows_].float() @ head.float()) < 1e-3
+    ref = torch.zeros(vocab, d, device=cuda_device)
+    for at in range(0, rows, 2000):
+        ref += logits[at:at + 2000, :vocab].float().t() @ x[at:at + 2000].float()
+    assert rel(dw, ref) < 1e-3
