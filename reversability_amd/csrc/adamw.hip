@@ -5,7 +5,7 @@
 // One launch updates up to kMaxTensors fp32 parameter tensors: the pointer
 // table and the per-tensor chunk prefix sums travel in the kernel arguments
 // (gradients are fresh tensors every step), each workgroup updates one chunk of
-// kChunk elements of one tensor with 16-byte accesses:
+// kUpdateChunk elements of one tensor with 16-byte accesses:
 //
 //     p  = p * (1 - lr wd)
 //     m  = lerp(m, g, 1 - b1)                       (torch's lerp formula)
@@ -18,7 +18,7 @@
 // parameter group): rv_adamw_advance adds 1 unless *found_inf != 0, and the
 // update kernel skips every element when *found_inf != 0, so a skipped step
 // (GradScaler overflow) changes nothing and needs no host synchronisation.
-// The bias corrections are computed per workgroup in double from t.
+// The bias corrections are computed in double from t.
 
 #include <cmath>
 
@@ -28,9 +28,14 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxTensors = 48;
-// elements per workgroup: 16384 (C4's 20.3M parameters in ~1250 workgroups
-// rather than ~330; C4 step 6.93 -> 6.87 ms against 65536 in same-box runs)
+// Elements per workgroup of the gradient-norm pass (one partial sum each).
 constexpr int64_t kChunk = 16384;
+// Elements per workgroup of the update: one pass, so that consecutive
+// workgroups, and the HBM pages they touch in the seven streams, stay close
+// together (update alone, us, 103.9 M / 2.0 M parameters: 65536 elements 589 / -,
+// 16384 551 / 20, 4096 519 / 12, 1024 545 / 15 with two double pow per thread, 470 /
+// 16.5 with one exp2 each).
+constexpr int64_t kUpdateChunk = kThreads * 4;
 
 struct TensorTable {
   float* p[kMaxTensors];
@@ -45,6 +50,7 @@ struct TensorTable {
 struct Hyper {
   float lr, beta1, beta2, eps, decay;  // decay = fp32(1 - lr * wd)
   double lr_d, beta1_d, beta2_d;       // the bias corrections are formed in double
+  double log2_beta1, log2_beta2;       // beta^t = 2^(t log2 beta)
   const float* step;                   // t after this update (already advanced)
   const float* found_inf;              // nullable
   const float* inv_scale;              // nullable
@@ -85,77 +91,62 @@ __device__ __forceinline__ int tensor_of(const int* chunk_start, int count, int 
   return t;
 }
 
-// One pass of a thread: four elements of each array.  The gradient is read
-// with ordinary loads (the norm pass has just read it); LOAD_NT streams the
-// loads of p, m and v, STORE_NT their stores.
-template <bool LOAD_NT>
-struct Pass {
-  float4 p, g, m, v;
-  __device__ __forceinline__ void load(const float* pp, const float* gg, const float* mm,
-                                       const float* vv, int64_t i) {
-    p = LOAD_NT ? rv::ld_f4s(pp + i) : rv::ld_f4(pp + i);
-    g = rv::ld_f4(gg + i);
-    m = LOAD_NT ? rv::ld_f4s(mm + i) : rv::ld_f4(mm + i);
-    v = LOAD_NT ? rv::ld_f4s(vv + i) : rv::ld_f4(vv + i);
-  }
-};
-
-template <bool STORE_NT>
+template <bool NT>
+__device__ __forceinline__ float4 get(const float* src) {
+  return NT ? rv::ld_f4s(src) : rv::ld_f4(src);
+}
+template <bool NT>
 __device__ __forceinline__ void put(float* dst, float4 x) {
-  if constexpr (STORE_NT) rv::st_f4s(dst, x);
+  if constexpr (NT) rv::st_f4s(dst, x);
   else rv::st_f4(dst, x);
 }
 
 // Memory-bound: 28 bytes per parameter against about 60 VALU instructions
-// (sqrt and two divisions).  The next pass's loads are issued before the
-// current pass's arithmetic, the first one's before the bias corrections'
-// double-precision pow; see kStreamLoadBytes for the cache hints.
+// (sqrt and two divisions).  The loads are issued before the bias corrections'
+// double-precision arithmetic.  The gradient is read with ordinary loads (the
+// norm pass has just read it); LOAD_NT streams the loads of p, m and v,
+// STORE_NT their stores (see kStreamLoadBytes).
 template <bool LOAD_NT, bool STORE_NT>
 __global__ __launch_bounds__(kThreads)
 void adamw_k(TensorTable tab, Hyper h) {
   if (h.found_inf != nullptr && *h.found_inf != 0.0f) return;  // uniform skip
   const int t = tensor_of(tab.chunk_start, tab.count, (int)blockIdx.x);
-  const int64_t off = (int64_t)(blockIdx.x - tab.chunk_start[t]) * kChunk;
-  const int64_t end = off + kChunk < tab.n[t] ? off + kChunk : tab.n[t];
+  const int64_t off = (int64_t)(blockIdx.x - tab.chunk_start[t]) * kUpdateChunk;
+  const int64_t end = off + kUpdateChunk < tab.n[t] ? off + kUpdateChunk : tab.n[t];
   float* p = tab.p[t];
   const float* g = tab.g[t];
   float* m = tab.m[t];
   float* v = tab.v[t];
   const bool vec = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g) |
                      reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(v)) & 15) == 0;
-  int64_t i = off + threadIdx.x * 4;
-  bool live = vec && i + 4 <= end;
-  Pass<LOAD_NT> cur;
-  if (live) cur.load(p, g, m, v, i);  // in flight during the bias corrections' double pow
+  const int64_t i = off + threadIdx.x * 4;
+  const bool full = vec && i + 4 <= end;
+  float4 pp, gg, mm, vv;
+  if (full) {
+    pp = get<LOAD_NT>(p + i);
+    gg = rv::ld_f4(g + i);
+    mm = get<LOAD_NT>(m + i);
+    vv = get<LOAD_NT>(v + i);
+  }
   __builtin_amdgcn_sched_barrier(0);
   const double step = (double)*h.step;
   Scalars s;
   s.w1 = (float)(1.0 - h.beta1_d);
   s.one_minus_b2 = (float)(1.0 - h.beta2_d);
-  s.step_size = (float)(h.lr_d / (1.0 - pow(h.beta1_d, step)));
-  s.bc2_sqrt = (float)sqrt(1.0 - pow(h.beta2_d, step));
+  s.step_size = (float)(h.lr_d / (1.0 - exp2(step * h.log2_beta1)));
+  s.bc2_sqrt = (float)sqrt(1.0 - exp2(step * h.log2_beta2));
   s.inv = h.inv_scale != nullptr ? *h.inv_scale : 1.0f;
   s.clip = h.clip != nullptr ? *h.clip : 1.0f;
-  if (vec) {
-    while (live) {
-      const int64_t next = i + kThreads * 4;
-      const bool more = next + 4 <= end;
-      Pass<LOAD_NT> ahead;
-      if (more) ahead.load(p, g, m, v, next);  // the next pass's loads before this one's math
-      __builtin_amdgcn_sched_barrier(0);
-      update1(cur.p.x, cur.g.x, cur.m.x, cur.v.x, h, s);
-      update1(cur.p.y, cur.g.y, cur.m.y, cur.v.y, h, s);
-      update1(cur.p.z, cur.g.z, cur.m.z, cur.v.z, h, s);
-      update1(cur.p.w, cur.g.w, cur.m.w, cur.v.w, h, s);
-      put<STORE_NT>(p + i, cur.p);
-      put<STORE_NT>(m + i, cur.m);
-      put<STORE_NT>(v + i, cur.v);
-      cur = ahead;
-      i = next;
-      live = more;
-    }
-    // tail (< 4 elements at the very end of the tensor)
-    for (int64_t j = (i < end ? i : end); j < end; ++j) update1(p[j], g[j], m[j], v[j], h, s);
+  if (full) {
+    update1(pp.x, gg.x, mm.x, vv.x, h, s);
+    update1(pp.y, gg.y, mm.y, vv.y, h, s);
+    update1(pp.z, gg.z, mm.z, vv.z, h, s);
+    update1(pp.w, gg.w, mm.w, vv.w, h, s);
+    put<STORE_NT>(p + i, pp);
+    put<STORE_NT>(m + i, mm);
+    put<STORE_NT>(v + i, vv);
+  } else if (vec) {  // < 4 elements at the very end of the tensor
+    for (int64_t j = i; j < end; ++j) update1(p[j], g[j], m[j], v[j], h, s);
   } else {
     for (int64_t j = off + threadIdx.x; j < end; j += kThreads) update1(p[j], g[j], m[j], v[j], h, s);
   }
@@ -294,11 +285,11 @@ void grad_clip_k(const float* __restrict__ part, const float* __restrict__ flag,
 }
 
 // Cache hints by the bytes of the four arrays (16 per parameter), against the
-// 256 MB Infinity Cache.  Norm pass and update, us, with everything else
-// evicted before each call (plain / streamed loads / loads and stores; 32 MB
-// also with nothing evicted): 32 MB 36 / 32 / 32 (24 / 26 / 28), 325 MB 122 / 109 /
-// 120, 430 MB 118 / 106 / 113, 1.66 GB 652 / 624 / 605 (656 / 646 / 568: the
-// gradients then stay cached between the two passes).
+// 256 MB Infinity Cache.  Norm pass and update, us, with everything else evicted
+// before each call, at 16384 elements per workgroup (plain / streamed loads /
+// loads and stores; 32 MB also with nothing evicted): 32 MB 36 / 32 / 32 (24 / 26 /
+// 28), 325 MB 122 / 109 / 120, 430 MB 118 / 106 / 113, 1.66 GB 652 / 624 / 605 (656 /
+// 646 / 568: the gradients then stay cached between the two passes).
 constexpr int64_t kStreamLoadBytes = int64_t(64) << 20;
 constexpr int64_t kStreamStoreBytes = int64_t(512) << 20;
 
@@ -397,7 +388,7 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
     tab.n[i] = numel[i];
     bytes += 16 * numel[i];
     tab.chunk_start[i] = chunks;
-    const int64_t c = (numel[i] + kChunk - 1) / kChunk;
+    const int64_t c = (numel[i] + kUpdateChunk - 1) / kUpdateChunk;
     if ((int64_t)chunks + c > 0x7fffffff) return RV_ERR_UNSUPPORTED;
     chunks += (int)c;
   }
@@ -411,6 +402,8 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
   h.lr_d = lr;
   h.beta1_d = beta1;
   h.beta2_d = beta2;
+  h.log2_beta1 = std::log2(beta1);  // beta 0: -inf, and 2^-inf = 0 = beta^t for t >= 1
+  h.log2_beta2 = std::log2(beta2);
   h.step = step;
   h.found_inf = found_inf;
   h.inv_scale = inv_scale;
