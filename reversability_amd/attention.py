@@ -115,29 +115,31 @@ class AttentionLayer(torch.autograd.Function):
         rows = batch * seq
         lib, st, dev = library(), _stream(x16), x16.device
         dy = gradient.reshape(rows, out_f).to(torch.float16).contiguous()
-        dmixed = torch.empty_like(mixed)
-        ws, nbytes = splitk_workspace(dy, rows, d, out_f)
-        _check(lib.rv_linear_dx_ws(dy.data_ptr(), proj16.data_ptr(), rows, d, out_f,
-                                   dmixed.data_ptr(), RV_F16, ws.data_ptr() if nbytes else None,
-                                   nbytes, st), "rv_linear_dx")
-        dqkv = torch.empty_like(qkv)
-        nbytes = lib.rv_attn_bwd_workspace_bytes(batch, seq, heads)
-        if nbytes < 0:
-            _check(-nbytes, "rv_attn_bwd_workspace_bytes")
-        ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
-        _check(lib.rv_attn_bwd(qkv.data_ptr(), mixed.data_ptr(), dmixed.data_ptr(), lse.data_ptr(),
-                               batch, seq, heads, d // heads, dqkv.data_ptr(), ws.data_ptr(),
-                               nbytes, st), "rv_attn_bwd")
-        del dmixed, ws  # free for the buffers below
         dx = dw_qkv = dw_proj = None
-        if ctx.needs_input_grad[0]:
+        need_x, need_qkv, need_proj = ctx.needs_input_grad[:3]
+        if need_x or need_qkv:
+            dmixed = torch.empty_like(mixed)
+            ws, nbytes = splitk_workspace(dy, rows, d, out_f)
+            _check(lib.rv_linear_dx_ws(dy.data_ptr(), proj16.data_ptr(), rows, d, out_f,
+                                       dmixed.data_ptr(), RV_F16, ws.data_ptr() if nbytes else None,
+                                       nbytes, st), "rv_linear_dx")
+            dqkv = torch.empty_like(qkv)
+            nbytes = lib.rv_attn_bwd_workspace_bytes(batch, seq, heads)
+            if nbytes < 0:
+                _check(-nbytes, "rv_attn_bwd_workspace_bytes")
+            ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
+            _check(lib.rv_attn_bwd(qkv.data_ptr(), mixed.data_ptr(), dmixed.data_ptr(), lse.data_ptr(),
+                                   batch, seq, heads, d // heads, dqkv.data_ptr(), ws.data_ptr(),
+                                   nbytes, st), "rv_attn_bwd")
+            del dmixed, ws  # free for the buffers below
+        if need_x:
             dx = torch.empty(batch, seq, d, device=dev, dtype=ctx.x_dtype)
             ws, nbytes = splitk_workspace(dqkv, rows, d, 3 * d)
             code = RV_F32 if ctx.x_dtype == torch.float32 else RV_F16
             _check(lib.rv_linear_dx_ws(dqkv.data_ptr(), qkv16.data_ptr(), rows, d, 3 * d,
                                        dx.data_ptr(), code, ws.data_ptr() if nbytes else None,
                                        nbytes, st), "rv_linear_dx")
-        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
+        if need_qkv and need_proj:
             dw_qkv, dw_proj = torch.empty_like(w_qkv), torch.empty_like(w_proj)
             nbytes = lib.rv_linear_dw_pair_workspace_bytes(rows, d, 3 * d, d, out_f)
             if nbytes < 0:
@@ -147,8 +149,11 @@ class AttentionLayer(torch.autograd.Function):
                 dqkv.data_ptr(), x16.data_ptr(), d, 3 * d, dw_qkv.data_ptr(), dy.data_ptr(),
                 mixed.data_ptr(), d, out_f, dw_proj.data_ptr(), rows, 0,
                 ws.data_ptr() if nbytes else None, nbytes, st), "rv_linear_dw_pair")
-        return (dx, dw_qkv if ctx.needs_input_grad[1] else None,
-                dw_proj if ctx.needs_input_grad[2] else None, None)
+        elif need_qkv:  # the other projection is frozen
+            dw_qkv = _linear.weight_grad(dqkv.view(rows, 3 * d), x16, w_qkv)
+        elif need_proj:
+            dw_proj = _linear.weight_grad(dy, mixed, w_proj)
+        return dx, dw_qkv, dw_proj, None
 
 
 def _layer_supported(attn: torch.nn.Module, x: torch.Tensor, dropout: float) -> bool:

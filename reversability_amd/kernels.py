@@ -94,11 +94,17 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
             or labels.numel() != rows or not x16.is_cuda):
         raise ValueError("tied_head_ce needs contiguous CUDA fp16 x [rows, d], a padded fp16 "
                          "head [padded, d] and int64 labels [rows]")
+    if dw_out is not None and (dw_out.dtype != torch.float32 or not dw_out.is_contiguous()
+                               or tuple(dw_out.shape) != (vocab, d)
+                               or dw_out.device != x16.device):
+        raise ValueError("tied_head_ce's dw_out must be a contiguous fp32 [vocab, d] tensor on "
+                         "x's device")
     from ._hip import RV_F16, RV_F32, _check, _stream, library
     lib = library()
     labels = labels.contiguous()
     own = (head_supported(rows, d, padded)
            and x16.data_ptr() % 16 == 0 and head16.data_ptr() % 16 == 0
+           and (dw_out is None or dw_out.data_ptr() % 16 == 0)
            and (dx_out is None or (dx_out.dtype == torch.float16 and dx_out.is_contiguous()
                                    and dx_out.shape == x16.shape and dx_out.data_ptr() % 16 == 0)))
     if own:

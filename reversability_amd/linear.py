@@ -81,15 +81,22 @@ class FusedLinear(torch.autograd.Function):
                 ws.data_ptr() if ws is not None else None, nbytes, _stream(dy)), "rv_linear_dx")
             dx = dx.reshape(ctx.x_shape)
         if ctx.needs_input_grad[1]:
-            dw = torch.empty_like(weight)
-            nbytes = lib.rv_linear_dw_workspace_bytes(rows, in_f, out_f)
-            if nbytes < 0:
-                _check(-nbytes, "rv_linear_dw_workspace_bytes")
-            ws = torch.empty(max(nbytes, 4) // 4, device=dy.device, dtype=torch.float32)
-            _check(lib.rv_linear_dw(dy.data_ptr(), x16.data_ptr(), in_f, rows, in_f, out_f,
-                                    dw.data_ptr(), 0, ws.data_ptr(), nbytes, _stream(dy)),
-                   "rv_linear_dw")
+            dw = weight_grad(dy, x16, weight)
         return dx, dw
+
+
+def weight_grad(dy: torch.Tensor, x16: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """fp32(fp16(dy^T x16)) in a new tensor like ``weight`` (dy [rows, out], x16 [rows, in])."""
+    rows, (out_f, in_f) = dy.shape[0], weight.shape
+    lib = library()
+    dw = torch.empty_like(weight)
+    nbytes = lib.rv_linear_dw_workspace_bytes(rows, in_f, out_f)
+    if nbytes < 0:
+        _check(-nbytes, "rv_linear_dw_workspace_bytes")
+    ws = torch.empty(max(nbytes, 4) // 4, device=dy.device, dtype=torch.float32)
+    _check(lib.rv_linear_dw(dy.data_ptr(), x16.data_ptr(), in_f, rows, in_f, out_f,
+                            dw.data_ptr(), 0, ws.data_ptr(), nbytes, _stream(dy)), "rv_linear_dw")
+    return dw
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Tensor:

@@ -155,7 +155,7 @@ def test_attention_layer_matches_its_parts(cuda_device, batch, seq, heads, hd, x
     """The one-node attention layer against the three Functions it stands for
     (a forward hook on a projection keeps the parts): the same output and
     input-gradient bits, weight gradients within 2e-3 (their rows are summed
-    in another order), frozen weights, and the same recorded paths."""
+    in another order, as a lone layer's are), frozen weights, and the same recorded paths."""
     from reversability_amd import paths
     from reversability_amd.attention import AttentionLayer, enable_attention
     from reversability_amd.model import BaselineLM, ModelConfig
@@ -191,4 +191,9 @@ def test_attention_layer_matches_its_parts(cuda_device, batch, seq, heads, hd, x
         assert rel_l2(a, b) < 2e-3
     attn.qkv.weight.requires_grad_(False)
     partial = once((x, attn.proj.weight))[1]
-    assert torch.equal(partial[0], grads[0]) and torch.equal(partial[1], grads[2])
+    assert torch.equal(partial[0], grads[0]) and rel_l2(partial[1], grads[2]) < 2e-3
+    x.requires_grad_(False)  # the output projection alone: no attention backward
+    assert torch.equal(once((attn.proj.weight,))[1][0], partial[1])
+    attn.qkv.weight.requires_grad_(True)
+    attn.proj.weight.requires_grad_(False)
+    assert rel_l2(once((attn.qkv.weight,))[1][0], grads[1]) < 2e-3
