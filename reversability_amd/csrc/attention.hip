@@ -240,6 +240,19 @@ struct FragOffsets {
   }
 };
 
+// LDS fragments are read ahead of the work that hides their latency: the row
+// fragments of a 32-row half before its score MFMAs, the transposed ones before
+// the exponentials (in the dK/dV kernel half of them: the rest would not fit
+// beside two workgroups per CU).  The scheduling barriers keep them there; left
+// to itself the compiler reads each pair next to its two MFMAs and waits for
+// the LDS every time.  Same bits.  us, before -> after: forward 16 x 1024 tokens, 8
+// heads of 128 86 -> 77, 16 x 2048, 16 heads of 64 208 -> 200, 16 x 700 35.6 -> 34.1;
+// backward 224 -> 211, 630 -> 623, 114 -> 107, 2 x 2048, 8 heads of 64 91 -> 83.  At HD = 32
+// the dQ kernel passes 128 registers and loses a workgroup per CU (16 x 2048, 16
+// heads 403 -> 414), and the forward gains nothing (41.9 -> 43.3, 159 -> 153).
+template <int HD>
+constexpr bool kReadAhead = HD >= 64;
+
 // One 64-key tile for one wave.  MASK: the causal diagonal crosses the tile;
 // key offset (within the tile) k is visible to the lane's query iff
 // k <= rel, rel = q - k0.  live1: the second 32-key half has a visible key
@@ -255,9 +268,13 @@ __device__ __forceinline__ void fwd_tile(FwdState<HD>& st, const _Float16* Ks, c
 #pragma unroll
   for (int sub = 0; sub < 2; ++sub) {
     if (sub == 1 && MASK && !live1) break;
-    s[sub] = mfma(fo.rowf(Ks, sub, 0), qf[0], zero16());
+    f16x8 kf[KK];
 #pragma unroll
-    for (int kk = 1; kk < KK; ++kk) s[sub] = mfma(fo.rowf(Ks, sub, kk), qf[kk], s[sub]);
+    for (int kk = 0; kk < KK; ++kk) kf[kk] = fo.rowf(Ks, sub, kk);
+    if constexpr (kReadAhead<HD>) __builtin_amdgcn_sched_barrier(0);
+    s[sub] = mfma(kf[0], qf[0], zero16());
+#pragma unroll
+    for (int kk = 1; kk < KK; ++kk) s[sub] = mfma(kf[kk], qf[kk], s[sub]);
   }
   const bool two = !MASK || live1;
   prio_valu();
@@ -288,6 +305,14 @@ __device__ __forceinline__ void fwd_tile(FwdState<HD>& st, const _Float16* Ks, c
 #pragma unroll
   for (int sub = 0; sub < 2; ++sub) {
     if (sub == 1 && !two) break;
+    f16x8 vf[2][DT];
+    if constexpr (kReadAhead<HD>) {
+#pragma unroll
+      for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vf[cc][dt] = fo.trf(Vs, sub, cc, dt);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     float rowsum = 0.f;
     prio_valu();
 #pragma unroll
@@ -302,7 +327,10 @@ __device__ __forceinline__ void fwd_tile(FwdState<HD>& st, const _Float16* Ks, c
     for (int cc = 0; cc < 2; ++cc) {
       const f16x8 pf = pack8(s[sub], cc);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) st.o[dt] = mfma(fo.trf(Vs, sub, cc, dt), pf, st.o[dt]);
+      for (int dt = 0; dt < DT; ++dt) {
+        if constexpr (!kReadAhead<HD>) vf[cc][dt] = fo.trf(Vs, sub, cc, dt);
+        st.o[dt] = mfma(vf[cc][dt], pf, st.o[dt]);
+      }
     }
   }
 }
@@ -406,12 +434,28 @@ __device__ __forceinline__ void kv_rows(f32x16 (&dk)[HD / 32], f32x16 (&dv)[HD /
   const int hl = lane >> 5;
   const int sub = r0 / 32;
   prio_mfma();
-  f32x16 s = mfma(fo.rowf(Qs, sub, 0), kf[0], zero16());
-  f32x16 dp = mfma(fo.rowf(Gs, sub, 0), vf[0], zero16());
+  f16x8 qf[KK], gf[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) {
+    qf[kk] = fo.rowf(Qs, sub, kk);
+    gf[kk] = fo.rowf(Gs, sub, kk);
+  }
+  if constexpr (kReadAhead<HD>) __builtin_amdgcn_sched_barrier(0);
+  f32x16 s = mfma(qf[0], kf[0], zero16());
+  f32x16 dp = mfma(gf[0], vf[0], zero16());
 #pragma unroll
   for (int kk = 1; kk < KK; ++kk) {
-    s = mfma(fo.rowf(Qs, sub, kk), kf[kk], s);
-    dp = mfma(fo.rowf(Gs, sub, kk), vf[kk], dp);
+    s = mfma(qf[kk], kf[kk], s);
+    dp = mfma(gf[kk], vf[kk], dp);
+  }
+  f16x8 qt[2][DT], gt[2][DT];
+  if constexpr (kReadAhead<HD>) {  // the second half's do not fit in the registers
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      gt[0][dt] = fo.trf(Gs, sub, 0, dt);
+      qt[0][dt] = fo.trf(Qs, sub, 0, dt);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   prio_valu();
 #pragma unroll
@@ -437,8 +481,12 @@ __device__ __forceinline__ void kv_rows(f32x16 (&dk)[HD / 32], f32x16 (&dv)[HD /
     const f16x8 pf = pack8(s, cc), dsf = pack8(dp, cc);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      dv[dt] = mfma(fo.trf(Gs, sub, cc, dt), pf, dv[dt]);
-      dk[dt] = mfma(fo.trf(Qs, sub, cc, dt), dsf, dk[dt]);
+      if (cc == 1 || !kReadAhead<HD>) {
+        gt[cc][dt] = fo.trf(Gs, sub, cc, dt);
+        qt[cc][dt] = fo.trf(Qs, sub, cc, dt);
+      }
+      dv[dt] = mfma(gt[cc][dt], pf, dv[dt]);
+      dk[dt] = mfma(qt[cc][dt], dsf, dk[dt]);
     }
   }
 }
@@ -456,12 +504,27 @@ __device__ __forceinline__ void q_rows(f32x16 (&dq)[HD / 32], const _Float16* Ks
   const int hl = lane >> 5;
   const int sub = r0 / 32;
   prio_mfma();
-  f32x16 s = mfma(fo.rowf(Ks, sub, 0), qf[0], zero16());
-  f32x16 dp = mfma(fo.rowf(Vs, sub, 0), gf[0], zero16());
+  f16x8 kf[KK], vf[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) {
+    kf[kk] = fo.rowf(Ks, sub, kk);
+    vf[kk] = fo.rowf(Vs, sub, kk);
+  }
+  if constexpr (kReadAhead<HD>) __builtin_amdgcn_sched_barrier(0);
+  f32x16 s = mfma(kf[0], qf[0], zero16());
+  f32x16 dp = mfma(vf[0], gf[0], zero16());
 #pragma unroll
   for (int kk = 1; kk < KK; ++kk) {
-    s = mfma(fo.rowf(Ks, sub, kk), qf[kk], s);
-    dp = mfma(fo.rowf(Vs, sub, kk), gf[kk], dp);
+    s = mfma(kf[kk], qf[kk], s);
+    dp = mfma(vf[kk], gf[kk], dp);
+  }
+  f16x8 kt[2][DT];
+  if constexpr (kReadAhead<HD>) {
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) kt[cc][dt] = fo.trf(Ks, sub, cc, dt);
+    __builtin_amdgcn_sched_barrier(0);
   }
   const float neg_l = -Lq;
   prio_valu();
@@ -477,8 +540,10 @@ __device__ __forceinline__ void q_rows(f32x16 (&dq)[HD / 32], const _Float16* Ks
   for (int cc = 0; cc < 2; ++cc) {
     const f16x8 dsf = pack8(dp, cc);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      dq[dt] = mfma(fo.trf(Ks, sub, cc, dt), dsf, dq[dt]);
+    for (int dt = 0; dt < DT; ++dt) {
+      if constexpr (!kReadAhead<HD>) kt[cc][dt] = fo.trf(Ks, sub, cc, dt);
+      dq[dt] = mfma(kt[cc][dt], dsf, dq[dt]);
+    }
   }
 }
 
