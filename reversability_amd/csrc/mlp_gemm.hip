@@ -329,21 +329,22 @@ struct GemmArgs {
   void* u; int64_t ldu;    // SwiGLU: optional u output; SwiGLUBwd: u input
   int64_t f;               // SwiGLU / SwiGLUBwd: value column offset
   int accumulate;          // AccF32OfF16
+  int64_t group = 8;       // M tiles per group of the tile order (tile_of)
   int64_t valid;           // StoreF16: columns valid .. n - 1 are written as zero (0: none)
 };
 
 // Workgroups are dispatched to the 8 XCDs round robin.  Tiles are numbered in
-// groups of 8 M-tiles (M fastest inside a group), and each XCD receives a
+// groups of `rows` M-tiles (M fastest inside a group), and each XCD receives a
 // contiguous range of tile numbers, so the workgroups sharing one XCD's L2 at
 // a time cover a compact block of M x N tiles.
 __device__ __forceinline__ void tile_of(int64_t t, int64_t tiles_m, int64_t tiles_n,
-                                        int64_t& tm, int64_t& tn) {
+                                        int64_t rows, int64_t& tm, int64_t& tn) {
   const int64_t tiles = tiles_m * tiles_n;
   if ((tiles & 7) == 0) t = (t & 7) * (tiles >> 3) + (t >> 3);
-  const int64_t group = 8 * tiles_n;
+  const int64_t group = rows * tiles_n;
   const int64_t g = t / group, r = t % group;
-  const int64_t first = g * 8;
-  const int64_t gm = tiles_m - first < 8 ? tiles_m - first : 8;
+  const int64_t first = g * rows;
+  const int64_t gm = tiles_m - first < rows ? tiles_m - first : rows;
   tm = first + r % gm;
   tn = r / gm;
 }
@@ -380,7 +381,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) 
   const int64_t tiles = args.tiles_m * args.tiles_n;
   const int64_t split = block / tiles;
   int64_t tm, tn;
-  tile_of(block % tiles, args.tiles_m, args.tiles_n, tm, tn);
+  tile_of(block % tiles, args.tiles_m, args.tiles_n, args.group, tm, tn);
   const int64_t m0 = tm * BM;
   const int64_t n0 = (EPI == Epi::SwiGLU) ? tn * (BN / 2) : tn * BN;
   const int64_t kbeg = split * args.k_chunk;
@@ -507,7 +508,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) 
       });
 #pragma unroll
       for (int d = 0; d < ND; ++d)
-        if ((2 * d + 1) * kM / (2 * ND) == q) dma(D0 + d);
+        if ((2 * d + 1) * kM / (ND ? 2 * ND : 1) == q) dma(D0 + d);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -760,7 +761,8 @@ void gemm_kernel(GemmArgs args) {
 // leave, so one's loads and partial sums overlap the other's MFMAs (both
 // gradients and their reduce, us, two launches -> one: 51 x 256 x 1024 8.4 -> 4.7,
 // 2048 x 256 x 1024 21.3 -> 16.8, 16896 x 256 x 1024 60.8 -> 53.8, 1000 x 768 x 3072
-// 34.9 -> 27.7, 3062 x 1024 x 4096 100.7 -> 97.0, 32768 x 1024 x 4096 690 -> 687).
+// 34.9 -> 27.7, 3062 x 1024 x 4096 100.7 -> 97.0, 32768 x 1024 x 4096 690 -> 687; tiles in
+// groups of 8 on both sides, see wgrad_group).
 struct GemmPair {
   GemmArgs g[2];
   int64_t first;
@@ -1241,6 +1243,26 @@ struct WgradJob {
   GemmArgs g;
   ReduceSeg seg;
 };
+// M tiles per group of a weight gradient's tile order.  Each XCD gets an eighth
+// of every split's tiles, a contiguous range of their order: the group makes
+// that range as square as the shapes allow, so that its L2 fetches the fewest
+// distinct rows of the two operands.  us, groups of 8 -> this rule (an MLP's two
+// gradients, rows x d x f): 8192 x 256 x 1024 30.7 -> 27.9, 16896 x 256 x 1024 52.0 -> 48.9,
+// 20000 x 384 x 1536 119 -> 109, 32768 x 1024 x 4096 689 -> 676, 8192 x 1024 x 4096 212.2 ->
+// 213.8, 51 x 256 x 1024 4.7 either way.  The activation products keep 8 (up, down, dgate
+// and dx at 32768 x 1024 x 4096: 8 is the fastest or within 2% of it among 1 .. 32).
+int64_t wgrad_group(const WgradPlan& p) {
+  const int64_t tiles = p.tiles_m * p.tiles_n, share = tiles / 8;
+  if (tiles % 8) return 8;
+  int64_t best = 8, least = 0;
+  for (int64_t g = 8; g >= 1; g /= 2) {
+    int64_t n = (share + g - 1) / g;
+    if (n > p.tiles_n) n = p.tiles_n;
+    const int64_t rows = (share + n - 1) / n * kShapes[p.shape].bm + n * kShapes[p.shape].bn;
+    if (least == 0 || rows < least) best = g, least = rows;
+  }
+  return best;
+}
 WgradJob plan_job(const WgradPlan& p, const __half* a, int64_t lda, const __half* b, int64_t ldb,
                   int64_t rows, int64_t ni, int64_t nj, float* out, int accumulate, float* part) {
   WgradJob j{p, {}, {nullptr, nullptr, 0, 0, 0}};
@@ -1249,7 +1271,7 @@ WgradJob plan_job(const WgradPlan& p, const __half* a, int64_t lda, const __half
   g.a = a; g.lda = lda; g.a_bytes = rows * lda * 2;
   g.b = b; g.ldb = ldb; g.b_bytes = rows * ldb * 2;
   g.m = ni; g.n = nj; g.k = rows; g.k_chunk = p.chunk;
-  g.tiles_m = p.tiles_m; g.tiles_n = p.tiles_n;
+  g.tiles_m = p.tiles_m; g.tiles_n = p.tiles_n; g.group = wgrad_group(p);
   g.ldc = nj; g.accumulate = accumulate;
   g.c = p.splits == 1 ? out : part;
   if (p.splits > 1) {

@@ -333,3 +333,21 @@ def test_wgrad_pair_plans(cuda_device, rows, d, f):
     first = (ddown.clone(), dup.clone())
     mlp.wgrad(dy, o, du, x16, ddown, dup, accumulate=True)
     assert torch.equal(ddown, first[0] + first[0]) and torch.equal(dup, first[1] + first[1])
+
+
+@pytest.mark.parametrize("rows,d,f", [(700, 256, 1024), (8192, 256, 1024), (2500, 256, 2048),
+                                      (1500, 640, 2560), (3001, 384, 1536), (900, 1024, 512)])
+def test_wgrad_tile_order(cuda_device, rows, d, f):
+    """Output widths whose weight gradients number their tiles in groups of
+    1, 2, 4 and 8, with tile counts that the group does not divide: every tile is
+    computed once (the fp64 bound over an output filled with NaN)."""
+    g = torch.Generator().manual_seed(43)
+    dy = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    o = torch.randn(rows, f, generator=g).half().to(cuda_device)
+    du = (0.3 * torch.randn(rows, 2 * f, generator=g)).half().to(cuda_device)
+    x16 = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    ddown = torch.full((d, f), float("nan"), device=cuda_device)
+    dup = torch.full((2 * f, d), float("nan"), device=cuda_device)
+    mlp.wgrad(dy, o, du, x16, ddown, dup, accumulate=False)
+    assert within_gemm_bound(ddown, dy.t(), o.t(), rows)
+    assert within_gemm_bound(dup, du.t(), x16.t(), rows)
