@@ -624,7 +624,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) 
     // (row stride WN + 8 halves), then moves whole rows, 16 bytes per lane,
     // so every global access instruction covers full row segments.  The
     // stores are streaming (nt): measured 1-5% faster per GEMM and 0.3-0.5%
-    // per configs[3]/[4] training step, consumers included.
+    // per training step of the two decoders, consumers included.
     constexpr int S = WN + 8;
     _Float16* stage = lds + wave * (WM * S);
 #pragma unroll

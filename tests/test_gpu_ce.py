@@ -332,3 +332,24 @@ def test_head_products_past_32_bit_offsets(cuda_device):
     for at in range(0, rows, 2000):
         ref += logits[at:at + 2000, :vocab].float().t() @ x[at:at + 2000].float()
     assert rel(dw, ref) < 1e-3
+
+
+def test_tied_head_ce_refuses_a_wrong_dw_out(cuda_device):
+    """The weight gradient's output has to be a contiguous fp32 [vocab, d]; one
+    off a 16-byte boundary is taken (torch's products)."""
+    from reversability_amd.kernels import padded_head, tied_head_ce
+    g = torch.Generator().manual_seed(9)
+    x16 = torch.randn(32, 128, generator=g).half().to(cuda_device)
+    head16 = padded_head((0.05 * torch.randn(100, 128, generator=g)).to(cuda_device))
+    labels = torch.randint(0, 100, (32,), generator=g).to(cuda_device)
+    args = (x16, head16, 100, labels, torch.ones(1, device=cuda_device))
+    for wrong in (torch.empty(99, 128, device=cuda_device),
+                  torch.empty(100, 128, device=cuda_device, dtype=torch.float16),
+                  torch.empty(128, 100, device=cuda_device).t(), torch.empty(100, 128)):
+        with pytest.raises(ValueError):
+            tied_head_ce(*args, dw_out=wrong)
+    _, dx, dw = tied_head_ce(*args, dw_out=torch.empty(100, 128, device=cuda_device))
+    odd = torch.empty(100 * 128 + 1, device=cuda_device)[1:].view(100, 128)
+    _, dx_odd, dw_odd = tied_head_ce(*args, dw_out=odd)
+    for a, b in ((dx, dx_odd), (dw, dw_odd)):  # the same products, summed in another order
+        assert float((a.float() - b.float()).norm() / a.float().norm()) < 2e-3
