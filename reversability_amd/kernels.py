@@ -94,6 +94,9 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
             or labels.numel() != rows or not x16.is_cuda):
         raise ValueError("tied_head_ce needs contiguous CUDA fp16 x [rows, d], a padded fp16 "
                          "head [padded, d] and int64 labels [rows]")
+    # the kernels take raw pointers: memory of another device would fault there
+    if any(t is not None and t.device != x16.device for t in (head16, labels, grad, dx_out)):
+        raise ValueError("tied_head_ce needs its head, labels, gradient and dx_out on x's device")
     if dw_out is not None and (dw_out.dtype != torch.float32 or not dw_out.is_contiguous()
                                or tuple(dw_out.shape) != (vocab, d)
                                or dw_out.device != x16.device):

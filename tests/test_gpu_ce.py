@@ -353,3 +353,20 @@ def test_tied_head_ce_refuses_a_wrong_dw_out(cuda_device):
     _, dx_odd, dw_odd = tied_head_ce(*args, dw_out=odd)
     for a, b in ((dx, dx_odd), (dw, dw_odd)):  # the same products, summed in another order
         assert float((a.float() - b.float()).norm() / a.float().norm()) < 2e-3
+
+
+@pytest.mark.parametrize("which", ["head16", "labels", "grad", "dx_out"])
+def test_tied_head_ce_refuses_other_devices(cuda_device, which):
+    """An operand or output in host memory is refused before any kernel gets its pointer."""
+    from reversability_amd.kernels import padded_head, tied_head_ce
+    g = torch.Generator().manual_seed(9)
+    args = {"x16": torch.randn(32, 128, generator=g).half().to(cuda_device),
+            "head16": padded_head((0.05 * torch.randn(100, 128, generator=g)).to(cuda_device)),
+            "vocab": 100, "labels": torch.randint(0, 100, (32,), generator=g).to(cuda_device),
+            "grad": torch.ones(1, device=cuda_device),
+            "dx_out": torch.empty(32, 128, device=cuda_device, dtype=torch.float16)}
+    _, dx, _ = tied_head_ce(**args)
+    assert dx.data_ptr() == args["dx_out"].data_ptr()
+    args[which] = args[which].cpu()
+    with pytest.raises(ValueError, match="device"):
+        tied_head_ce(**args)
