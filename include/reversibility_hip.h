@@ -339,11 +339,11 @@ int rv_linear_dx_ws(const void* dy, const void* w, int64_t rows, int64_t in, int
                     int dx_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The tied head's three products, fp16 with a vocabulary padded to a multiple
- * of 64 (head rows vocab .. padded - 1 zero; logits row stride padded), d a
+ * of 64 (head of padded rows; logits row stride padded), d a
  * multiple of 128 (src/reversibility/optimized_v3.py:151-192):
  *   logits  logits[rows, padded] = fp16(x head^T), columns vocab .. zero
- *   dx      dx[rows, d] = fp16(dlogits head), over all padded columns (the pad
- *           columns of dlogits have to be finite)
+ *   dx      dx[rows, d] = fp16(dlogits head) over the vocab rows of head (its pad
+ *           rows are not read; the pad columns of dlogits have to be finite)
  *   dw      dw[vocab, d] = fp16(dlogits^T x), stored as fp16, or (+)= that
  *           value widened to fp32
  * rv_head_workspace_bytes covers dx and dw (one workspace may serve both in

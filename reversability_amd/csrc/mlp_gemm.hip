@@ -1645,7 +1645,7 @@ int rv_head_dx(const void* dlogits, const void* head, int64_t rows, int64_t d, i
   GemmArgs a{};
   a.a = static_cast<const __half*>(dlogits); a.lda = padded; a.a_bytes = rows * padded * 2;
   a.b = static_cast<const __half*>(head); a.ldb = d;  // B(d, v) = head[v][d]: RC
-  a.b_bytes = padded * d * 2;
+  a.b_bytes = vocab * d * 2;  // the operand ends here: the pad rows read as zero
   a.m = rows; a.n = d; a.k = padded; a.k_chunk = head_chunk(rows, d, padded);
   const hipStream_t s = (hipStream_t)stream;
   const int64_t need = head_dx_bytes(rows, d, padded);

@@ -370,3 +370,20 @@ def test_tied_head_ce_refuses_other_devices(cuda_device, which):
     args[which] = args[which].cpu()
     with pytest.raises(ValueError, match="device"):
         tied_head_ce(**args)
+
+
+@pytest.mark.parametrize("vocab", [1001, 70001])
+def test_head_pad_rows_do_not_matter(cuda_device, vocab):
+    """Whatever a caller left in the head's pad rows (NaN here), loss and
+    gradients are those of zero pad rows, with the one-pass cross-entropy and
+    the two-pass one of a wide vocabulary."""
+    from reversability_amd.kernels import padded_head, tied_head_ce
+    g = torch.Generator().manual_seed(5)
+    x16 = torch.randn(48, 128, generator=g).half().to(cuda_device)
+    head16 = padded_head((0.05 * torch.randn(vocab, 128, generator=g)).to(cuda_device))
+    labels = torch.randint(0, vocab, (48,), generator=g).to(cuda_device)
+    args = (vocab, labels, torch.ones(1, device=cuda_device))
+    clean = tied_head_ce(x16, head16, *args)
+    head16[vocab:] = float("nan")
+    for a, b in zip(clean, tied_head_ce(x16, head16, *args)):
+        assert torch.equal(a, b)
