@@ -1136,7 +1136,10 @@ int64_t act_chunk(int64_t m, int64_t n, int64_t k) {
   const int64_t splits = act_splits(m, n, k);
   return ((k + splits - 1) / splits + kSplitStep - 1) / kSplitStep * kSplitStep;
 }
+// 0 (no split) also for sizes that the split entry points do not take; an unsplit
+// one may take them (rv_mlp_down and rv_mlp_dx: reductions of any multiple of 32).
 int64_t act_part_bytes(int64_t m, int64_t n, int64_t k) {
+  if (n % 128 || k % 128) return 0;
   const int64_t chunk = act_chunk(m, n, k), splits = (k + chunk - 1) / chunk;
   return splits > 1 ? splits * m * n * (int64_t)sizeof(float) : 0;
 }

@@ -351,3 +351,18 @@ def test_wgrad_tile_order(cuda_device, rows, d, f):
     mlp.wgrad(dy, o, du, x16, ddown, dup, accumulate=False)
     assert within_gemm_bound(ddown, dy.t(), o.t(), rows)
     assert within_gemm_bound(dup, du.t(), x16.t(), rows)
+
+
+@pytest.mark.parametrize("rows", [51, 3000])
+def test_long_reductions_off_128(cuda_device, rows):
+    """down and dx over a long reduction that is a multiple of 32 but not of 128:
+    the split products do not take it, the unsplit ones do, at few rows as at
+    many."""
+    d, k = 256, 4128
+    g = torch.Generator().manual_seed(31)
+    a = torch.randn(rows, k, generator=g).half().to(cuda_device)
+    w = (0.02 * torch.randn(d, k, generator=g)).half().to(cuda_device)
+    y = mlp.down(a, w, torch.empty(rows, d, device=cuda_device, dtype=torch.float16))
+    assert within_gemm_bound(y, a, w, k)
+    dx = mlp.dx(a, w.t().contiguous(), torch.empty(rows, d, device=cuda_device))
+    assert torch.equal(dx, y.float())
