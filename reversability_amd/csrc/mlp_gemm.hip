@@ -336,20 +336,11 @@ struct GemmArgs {
 // Workgroups are dispatched to the 8 XCDs round robin.  Tiles are numbered in
 // groups of `rows` M-tiles (M fastest inside a group), and each XCD receives a
 // contiguous range of tile numbers, so the workgroups sharing one XCD's L2 at
-// a time cover a compact block of M x N tiles.  `skew` is the XCD of tile 0 (the
-// workgroups before it, modulo 8): with u = t + skew, XCD x = u % 8 owns the u / 8
-// th tile after those of the XCDs below it, less one where its first turn lies
-// before tile 0.
-// Numbers of tiles that 8 does not divide used to go round the XCDs tile by
-// tile, each L2 fetching nearly all of both operands (us, before -> now:
-// dW of 31899 rows, 896 x 896 119 -> 68, 24714 rows, 640 x 1792 107 -> 69, 30844
-// rows, 384 x 384 38 -> 28; logits of 1500 x 512 over 32000 80 -> 66; 512 weight
-// gradients at such numbers 2.7% less on average, the worst 32768 rows, 2816 x 768
-// 152 -> 171).
-__device__ __forceinline__ void tile_of(int64_t t, int64_t skew, int64_t tiles_m, int64_t tiles_n,
+// a time cover a compact block of M x N tiles.
+__device__ __forceinline__ void tile_of(int64_t t, int64_t tiles_m, int64_t tiles_n,
                                         int64_t rows, int64_t& tm, int64_t& tn) {
-  const int64_t u = t + skew, x = u & 7, end = tiles_m * tiles_n + skew, odd = end & 7;
-  t = x * (end >> 3) + (x < odd ? x : odd) - (x < skew ? x : skew) + (u >> 3) - (x < skew);
+  const int64_t tiles = tiles_m * tiles_n;
+  if ((tiles & 7) == 0) t = (t & 7) * (tiles >> 3) + (t >> 3);
   const int64_t group = rows * tiles_n;
   const int64_t g = t / group, r = t % group;
   const int64_t first = g * rows;
@@ -369,10 +360,8 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// block: workgroup number within this product; before: the launch's workgroups
-// ahead of its first.
 template <int SHAPE, bool A_RC, bool B_RC, Epi EPI>
-__device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block, int64_t before) {
+__device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block) {
   constexpr int BM = kShapes[SHAPE].bm, BN = kShapes[SHAPE].bn, WAVES = kShapes[SHAPE].waves;
   constexpr int BK = kShapes[SHAPE].bk, RA = kShapes[SHAPE].ra, RB = kShapes[SHAPE].rb;
   // waves: 2 rows x WCOLS columns, each owning a WM x WN block of the tile
@@ -392,8 +381,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, int64_t block, 
   const int64_t tiles = args.tiles_m * args.tiles_n;
   const int64_t split = block / tiles;
   int64_t tm, tn;
-  tile_of(block % tiles, (before + split * tiles) & 7, args.tiles_m, args.tiles_n, args.group, tm,
-          tn);
+  tile_of(block % tiles, args.tiles_m, args.tiles_n, args.group, tm, tn);
   const int64_t m0 = tm * BM;
   const int64_t n0 = (EPI == Epi::SwiGLU) ? tn * (BN / 2) : tn * BN;
   const int64_t kbeg = split * args.k_chunk;
@@ -764,7 +752,7 @@ template <int SHAPE, bool A_RC, bool B_RC, Epi EPI>
 __global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
                              kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
 void gemm_kernel(GemmArgs args) {
-  gemm_block<SHAPE, A_RC, B_RC, EPI>(args, blockIdx.x, 0);
+  gemm_block<SHAPE, A_RC, B_RC, EPI>(args, blockIdx.x);
 }
 
 // Two independent GEMMs in one launch: workgroups [0, first) run g[0], the rest
@@ -784,8 +772,7 @@ __global__ __launch_bounds__(kShapes[SHAPE].waves * 64,
                              kShapes[SHAPE].per_cu * kShapes[SHAPE].waves / 4)
 void wgrad_pair_kernel(GemmPair pair) {
   const int second = (int64_t)blockIdx.x >= pair.first;
-  const int64_t before = second ? pair.first : 0;
-  gemm_block<SHAPE, true, true, EPI>(pair.g[second], blockIdx.x - before, before);
+  gemm_block<SHAPE, true, true, EPI>(pair.g[second], blockIdx.x - (second ? pair.first : 0));
 }
 
 // Explicit instantiations of every (tile shape, operand layout, epilogue) the
@@ -1268,7 +1255,8 @@ struct WgradJob {
 // 213.8, 51 x 256 x 1024 4.7 either way.  The activation products keep 8 (up, down, dgate
 // and dx at 32768 x 1024 x 4096: 8 is the fastest or within 2% of it among 1 .. 32).
 int64_t wgrad_group(const WgradPlan& p) {
-  const int64_t tiles = p.tiles_m * p.tiles_n, share = (tiles + 7) / 8;
+  const int64_t tiles = p.tiles_m * p.tiles_n, share = tiles / 8;
+  if (tiles % 8) return 8;
   int64_t best = 8, least = 0;
   for (int64_t g = 8; g >= 1; g /= 2) {
     int64_t n = (share + g - 1) / g;

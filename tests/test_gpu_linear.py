@@ -197,46 +197,3 @@ def test_attention_layer_matches_its_parts(cuda_device, batch, seq, heads, hd, x
     attn.qkv.weight.requires_grad_(True)
     attn.proj.weight.requires_grad_(False)
     assert rel_l2(once((attn.qkv.weight,))[1][0], grads[1]) < 2e-3
-
-
-@pytest.mark.parametrize("rows,in_f,out_f", [(1, 128, 128), (700, 384, 640), (1500, 128, 1408),
-                                             (2300, 640, 1152)])
-def test_tile_numbering(cuda_device, rows, in_f, out_f):
-    """Numbers of tiles that 8 does and does not divide, in every tile shape and
-    at every place of the second of two paired products: no tile is left out
-    (outputs start as NaN) and the values are the product's."""
-    from reversability_amd._hip import _stream, library
-    lib = library()
-    g = torch.Generator().manual_seed(29)
-    x = torch.randn(rows, in_f, generator=g).half().to(cuda_device)
-    w = (0.02 * torch.randn(out_f, in_f, generator=g)).half().to(cuda_device)
-    dy = torch.randn(rows, out_f, generator=g).half().to(cuda_device)
-    st = _stream(x)
-    nan = lambda *s: torch.full(s, float("nan"), device=cuda_device)
-    first = None
-    try:
-        for shape in range(lib.rv_gemm_num_shapes()):
-            assert lib.rv_gemm_force_shape(shape) == 0
-            y = nan(rows, out_f).half()
-            rc = lib.rv_linear_fwd(x.data_ptr(), in_f, w.data_ptr(), rows, in_f, out_f,
-                                   y.data_ptr(), st)
-            if rc == 3:  # the width does not divide this tile
-                continue
-            assert rc == 0
-            if first is None:
-                first = y
-                assert within_gemm_bound(y, x, w, in_f)
-            assert torch.equal(y, first), shape
-    finally:
-        lib.rv_gemm_force_shape(-1)
-    assert first is not None
-    for out_a in range(128, 1280, 128):  # the first product's workgroups, modulo 8
-        dy_a = torch.randn(rows, out_a, generator=g).half().to(cuda_device)
-        dw_a, dw = nan(out_a, in_f), nan(out_f, in_f)
-        need = lib.rv_linear_dw_pair_workspace_bytes(rows, in_f, out_a, in_f, out_f)
-        ws = torch.empty(max(need, 16) // 4, device=cuda_device)
-        assert lib.rv_linear_dw_pair(dy_a.data_ptr(), x.data_ptr(), in_f, out_a, dw_a.data_ptr(),
-                                     dy.data_ptr(), x.data_ptr(), in_f, out_f, dw.data_ptr(), rows,
-                                     0, ws.data_ptr(), need, st) == 0
-        assert within_gemm_bound(dw_a, dy_a.t(), x.t(), rows)
-        assert within_gemm_bound(dw, dy.t(), x.t(), rows)
