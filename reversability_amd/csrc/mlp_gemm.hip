@@ -983,14 +983,13 @@ int launch(int shape, const GemmArgs& a, int64_t splits, hipStream_t s) {
 // Activation GEMMs: C is m x n_out where n_out = n (or n/2 output columns for
 // SwiGLU, whose tile covers bn/2 of them).  The largest tile that gives at
 // least one workgroup per CU; otherwise the one with the most workgroups.
-int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits, bool ragged) {
+int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits) {
   int best = -1;
   int64_t best_blocks = -1;
   for (int i = 0; i < kRuleShapes; ++i) {
     const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
-    if (n_cols % cols && !ragged) continue;
-    const int64_t blocks =
-        ((m + kShapes[i].bm - 1) / kShapes[i].bm) * ((n_cols + cols - 1) / cols) * splits;
+    if (n_cols % cols) continue;
+    const int64_t blocks = ((m + kShapes[i].bm - 1) / kShapes[i].bm) * (n_cols / cols) * splits;
     if (blocks >= kCUs) return i;
     if (blocks > best_blocks) best = i, best_blocks = blocks;
   }
@@ -1041,7 +1040,7 @@ int launch_shape(int shape, GemmArgs a, int64_t n_cols, hipStream_t s) {
 }
 
 template <bool A_RC, bool B_RC, Epi EPI>
-int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback, bool ragged) {
+int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
   const bool swiglu = EPI == Epi::SwiGLU;
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return fallback;
@@ -1055,7 +1054,7 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback, boo
   for (int sweep = 0; sweep < 2; ++sweep)
     for (int i = 0; i < kNumShapes; ++i) {
       const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
-      if (n_cols % cols && !ragged) continue;
+      if (n_cols % cols) continue;
       if (launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) != RV_OK) continue;
       bool ok = hipEventRecord(e0, s) == hipSuccess;
       ok = ok && launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) == RV_OK;
@@ -1074,25 +1073,28 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback, boo
   return best;
 }
 
+// fixed >= 0: the tile shape, chosen by the caller (no timing).  ragged: the tile's
+// width need not divide n_cols (the epilogue checks columns).
 template <bool A_RC, bool B_RC, Epi EPI>
-int run_act(GemmArgs a, int64_t n_cols, hipStream_t s, bool ragged = false) {
+int run_act(GemmArgs a, int64_t n_cols, hipStream_t s, int fixed = -1, bool ragged = false) {
   const bool swiglu = EPI == Epi::SwiGLU;
   if (EPI != Epi::PartialF32) a.k_chunk = a.k;
   const int64_t splits = (a.k + a.k_chunk - 1) / a.k_chunk;
-  int shape = pick_act(a.m, n_cols, swiglu, splits, ragged);
-  if (shape < 0) return RV_ERR_UNSUPPORTED;
   const int forced = g_forced_shape.load();
-  if (forced >= 0) {
-    if (n_cols % (swiglu ? kShapes[forced].bn / 2 : kShapes[forced].bn) && !ragged)
+  if (forced >= 0) fixed = forced;
+  if (fixed >= 0) {
+    if (n_cols % (swiglu ? kShapes[fixed].bn / 2 : kShapes[fixed].bn) && !ragged)
       return RV_ERR_UNSUPPORTED;
-    return launch_shape<A_RC, B_RC, EPI>(forced, a, n_cols, s);
+    return launch_shape<A_RC, B_RC, EPI>(fixed, a, n_cols, s);
   }
+  int shape = pick_act(a.m, n_cols, swiglu, splits);
+  if (shape < 0) return RV_ERR_UNSUPPORTED;
   if (tuning_enabled()) {
     int device = 0;
     (void)hipGetDevice(&device);
     // the SwiGLU epilogue with and without its u output store different
     // amounts and are tuned apart
-    const int variant = (EPI == Epi::SwiGLU && a.u != nullptr) ? 1 : ragged ? 2 : 0;
+    const int variant = (EPI == Epi::SwiGLU && a.u != nullptr) ? 1 : 0;
     const TuneKey key{(int)EPI * 4 + (A_RC ? 2 : 0) + (B_RC ? 1 : 0), device, variant, a.m,
                       n_cols, EPI == Epi::PartialF32 ? a.k * 64 + splits : a.k};
     std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -1100,7 +1102,7 @@ int run_act(GemmArgs a, int64_t n_cols, hipStream_t s, bool ragged = false) {
     if (it != g_tuned.end()) {
       shape = it->second;
     } else if (!capturing(s)) {
-      shape = tune_act<A_RC, B_RC, EPI>(a, n_cols, s, shape, ragged);
+      shape = tune_act<A_RC, B_RC, EPI>(a, n_cols, s, shape);
       g_tuned[key] = shape;
     }
   }
@@ -1146,10 +1148,10 @@ int64_t act_part_bytes(int64_t m, int64_t n, int64_t k) {
 
 // a.k_chunk set; fp32 partials of each chunk in `part`, summed into out.
 template <bool B_RC, typename T>
-int run_split(GemmArgs a, T* out, float* part, hipStream_t s) {
+int run_split(GemmArgs a, T* out, float* part, hipStream_t s, int fixed = -1) {
   a.c = part;
   a.ldc = a.n;
-  const int st = run_act<false, B_RC, Epi::PartialF32>(a, a.n, s);
+  const int st = run_act<false, B_RC, Epi::PartialF32>(a, a.n, s, fixed);
   if (st != RV_OK) return st;
   const int64_t n = a.m * a.n, splits = (a.k + a.k_chunk - 1) / a.k_chunk;
   hipLaunchKernelGGL(act_reduce<T>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, part,
@@ -1381,6 +1383,39 @@ int64_t head_chunk(int64_t rows, int64_t d, int64_t k) {
 int64_t head_dx_bytes(int64_t rows, int64_t d, int64_t k) {
   const int64_t chunk = head_chunk(rows, d, k), splits = (k + chunk - 1) / chunk;
   return splits > 1 ? splits * rows * d * (int64_t)sizeof(float) : 0;
+}
+
+// Tile shapes of the head's logits and input gradient.  They follow from the
+// sizes, without the timing sweep of run_act: the products are large, a caller's
+// row count may change from call to call, and a sweep of both made the first
+// call at a row count 60 ms (16896 x 256 over 50257) where a call takes 2.1.  The
+// lines (kShapes' indices) are from all shapes timed at widths 128 .. 2048, 64 .. 32768
+// rows and vocabularies 1000 .. 50257, the operands evicted before each product:
+//   logits  4 (eight waves) is the fastest or within 5% of it once its tiles fill
+//           the CUs four times (16896 x 256 over 50257: 619 us, the others 670-999);
+//           1 at d = 128, where two workgroups per CU hide the epilogues of a
+//           short k loop, and below that number of tiles if 8 divides its own
+//           (tile_of: 24000 x 256 over 3000 49 against 57, but 1500 x 512 over 32000 87
+//           against 70); 2 and 3 below one and a half rounds, as pick_act
+//   dx      3 where act_splits splits, 0 (2 at odd multiples of 128) over a long
+//           reduction, else as pick_act with 3 below one round: 1.03 of the
+//           fastest on average
+int head_logits_shape(int64_t rows, int64_t d, int64_t padded) {
+  const auto tiles = [&](int i) {
+    return ((rows + kShapes[i].bm - 1) / kShapes[i].bm) *
+           ((padded + kShapes[i].bn - 1) / kShapes[i].bn);
+  };
+  if (tiles(0) >= 3 * kCUs / 2) {
+    if (d <= 128) return 1;
+    return tiles(1) % 8 == 0 && tiles(0) < (d <= 256 ? 8 : 4) * kCUs ? 1 : 4;
+  }
+  if (tiles(2) < kCUs) return 3;
+  return tiles(2) % 8 == 0 ? 2 : 4;
+}
+int head_dx_shape(int64_t rows, int64_t d, int64_t k) {
+  if (act_splits(rows, d, k) > 1) return 3;
+  if (k >= 4096) return d % 256 ? 2 : 0;
+  return (rows + 127) / 128 * (d / 128) >= kCUs ? pick_act(rows, d, false, 1) : 3;
 }
 
 // A tile's rows of an operand with this row stride stay within 32-bit offsets.
@@ -1627,7 +1662,8 @@ int rv_head_logits(const void* x, const void* head, int64_t rows, int64_t d, int
   a.b = static_cast<const __half*>(head); a.ldb = d; a.b_bytes = padded * d * 2;
   a.m = rows; a.n = padded; a.k = d;
   a.c = logits; a.ldc = padded; a.valid = vocab;
-  return run_act<false, false, Epi::StoreF16>(a, padded, (hipStream_t)stream, true);
+  return run_act<false, false, Epi::StoreF16>(a, padded, (hipStream_t)stream,
+                                              head_logits_shape(rows, d, padded), true);
 }
 
 int64_t rv_head_workspace_bytes(int64_t rows, int64_t d, int64_t vocab, int64_t padded) {
@@ -1652,12 +1688,13 @@ int rv_head_dx(const void* dlogits, const void* head, int64_t rows, int64_t d, i
   a.m = rows; a.n = d; a.k = padded; a.k_chunk = head_chunk(rows, d, padded);
   const hipStream_t s = (hipStream_t)stream;
   const int64_t need = head_dx_bytes(rows, d, padded);
+  const int shape = head_dx_shape(rows, d, padded);
   if (need == 0) {
     a.c = dx; a.ldc = d;
-    return run_act<false, true, Epi::StoreF16>(a, d, s);
+    return run_act<false, true, Epi::StoreF16>(a, d, s, shape);
   }
   if (!workspace || workspace_bytes < need || !ok16(workspace)) return RV_ERR_WORKSPACE;
-  return run_split<true>(a, static_cast<__half*>(dx), static_cast<float*>(workspace), s);
+  return run_split<true>(a, static_cast<__half*>(dx), static_cast<float*>(workspace), s, shape);
 }
 
 int rv_head_dw(const void* dlogits, const void* x, int64_t rows, int64_t d, int64_t vocab,

@@ -387,3 +387,25 @@ def test_head_pad_rows_do_not_matter(cuda_device, vocab):
     head16[vocab:] = float("nan")
     for a, b in zip(clean, tied_head_ce(x16, head16, *args)):
         assert torch.equal(a, b)
+
+
+def test_head_first_call_does_not_wait(cuda_device):
+    """The head's products take their tile shapes from the sizes: a call at a row
+    count that no call had before times nothing, so it returns while earlier
+    work of the stream still runs."""
+    from reversability_amd.kernels import padded_head, tied_head_ce
+    g = torch.Generator().manual_seed(9)
+    head16 = padded_head((0.05 * torch.randn(1001, 256, generator=g)).to(cuda_device))
+    grad = torch.ones(1, device=cuda_device)
+    data = [(torch.randn(rows, 256, generator=g).half().to(cuda_device),
+             torch.randint(0, 1001, (rows,), generator=g).to(cuda_device))
+            for rows in (1237, 1239)]
+    for i, (x16, labels) in enumerate(data):  # the first one loads the kernels
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)
+        slept = torch.cuda.Event()
+        slept.record()
+        tied_head_ce(x16, head16, 1001, labels, grad)
+        busy = not slept.query()
+        torch.cuda.synchronize()
+        assert busy or i == 0
