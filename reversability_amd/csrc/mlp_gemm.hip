@@ -1397,9 +1397,10 @@ int64_t head_dx_bytes(int64_t rows, int64_t d, int64_t k) {
 //           short k loop, and below that number of tiles if 8 divides its own
 //           (tile_of: 24000 x 256 over 3000 49 against 57, but 1500 x 512 over 32000 87
 //           against 70); 2 and 3 below one and a half rounds, as pick_act
-//   dx      3 where act_splits splits, 0 (2 at odd multiples of 128) over a long
-//           reduction, else as pick_act with 3 below one round: 1.03 of the
-//           fastest on average
+//   dx      where act_splits splits, 3 as long as its workgroups fill one round of
+//           the CUs (1000 x 512 over 50257: 81 us, 5 takes 116) and 5 past it (300 x
+//           768: 67, 3 takes 99); 0 (2 at odd multiples of 128) over a long
+//           reduction, else as pick_act with 3 below one round
 int head_logits_shape(int64_t rows, int64_t d, int64_t padded) {
   const auto tiles = [&](int i) {
     return ((rows + kShapes[i].bm - 1) / kShapes[i].bm) *
@@ -1413,7 +1414,8 @@ int head_logits_shape(int64_t rows, int64_t d, int64_t padded) {
   return tiles(2) % 8 == 0 ? 2 : 4;
 }
 int head_dx_shape(int64_t rows, int64_t d, int64_t k) {
-  if (act_splits(rows, d, k) > 1) return 3;
+  const int64_t splits = act_splits(rows, d, k);
+  if (splits > 1) return (rows + 63) / 64 * (d / 128) * splits > kCUs ? 5 : 3;
   if (k >= 4096) return d % 256 ? 2 : 0;
   return (rows + 127) / 128 * (d / 128) >= kCUs ? pick_act(rows, d, false, 1) : 3;
 }

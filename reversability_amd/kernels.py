@@ -76,10 +76,9 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     gradient ``grad`` (a device fp32 scalar): logits = fp16(x16 W^T); loss and
     dlogits from one pass of rv_ce_fused over each logits row (the two-pass
     rv_ce_fwd / rv_ce_bwd above FUSED_CE_MAX_COLS, same bits); dx = dlogits W and
-    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The three
-    products run on the MFMA kernels (``head_supported``; 16896 x 256 over 50257:
-    logits 685 -> 637 us against torch's GEMM, dx 566 -> 448, dW 554 -> 442), otherwise
-    on torch's GEMMs.  ``head16`` is the fp16 head with its rows padded to a
+    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The
+    logits and the two gradients run on the MFMA kernels or on torch's GEMMs
+    (``head_routes``).  ``head16`` is the fp16 head with its rows padded to a
     multiple of VOCAB_ALIGN (the pad rows zero), so every logits row starts
     16-byte aligned.  Returns (loss sum, dx16, dW16 [vocab, d]);
     dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when given, and
@@ -105,17 +104,21 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     from ._hip import RV_F16, RV_F32, _check, _stream, library
     lib = library()
     labels = labels.contiguous()
-    own = (head_supported(rows, d, padded)
-           and x16.data_ptr() % 16 == 0 and head16.data_ptr() % 16 == 0
-           and (dw_out is None or dw_out.data_ptr() % 16 == 0)
-           and (dx_out is None or (dx_out.dtype == torch.float16 and dx_out.is_contiguous()
-                                   and dx_out.shape == x16.shape and dx_out.data_ptr() % 16 == 0)))
-    if own:
+    own_logits, own_grads = head_routes(rows, d, padded)
+    aligned = x16.data_ptr() % 16 == 0 and head16.data_ptr() % 16 == 0
+    own_logits = own_logits and aligned
+    own_grads = (own_grads and aligned and (dw_out is None or dw_out.data_ptr() % 16 == 0)
+                 and (dx_out is None or (dx_out.dtype == torch.float16 and dx_out.is_contiguous()
+                                         and dx_out.shape == x16.shape
+                                         and dx_out.data_ptr() % 16 == 0)))
+    if own_logits:
         logits = torch.empty(rows, padded, device=x16.device, dtype=torch.float16)
         _check(lib.rv_head_logits(x16.data_ptr(), head16.data_ptr(), rows, d, vocab, padded,
                                   logits.data_ptr(), _stream(x16)), "rv_head_logits")
     else:
         logits = torch.mm(x16, head16.t())                   # [rows, padded] fp16
+        if own_grads and vocab < padded:
+            logits[:, vocab:].zero_()  # rv_head_dx reads the pad columns
     rmax, rlse, losses = (torch.empty(rows, device=x16.device, dtype=torch.float32)
                           for _ in range(3))
     st = _stream(x16)
@@ -127,7 +130,7 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
                                losses.data_ptr(), dlogits.data_ptr(), st), "rv_ce_fused")
     else:
         dlogits = torch.empty_like(logits)
-        if own:
+        if own_grads:
             dlogits[:, vocab:].zero_()  # rv_head_dx reads the pad columns
         if rows:
             _check(lib.rv_ce_fwd(logits.data_ptr(), RV_F16, padded, labels.data_ptr(), rows,
@@ -137,7 +140,7 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
                                  rmax.data_ptr(), rlse.data_ptr(), grad.data_ptr(), rows, vocab,
                                  IGNORE_INDEX, dlogits.data_ptr(), st), "rv_ce_bwd")
     del logits
-    if own:
+    if own_grads:
         nbytes = lib.rv_head_workspace_bytes(rows, d, vocab, padded)
         if nbytes < 0:
             _check(-nbytes, "rv_head_workspace_bytes")
@@ -168,10 +171,27 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     return losses.sum(), dx16, dw_out
 
 
-def head_supported(rows: int, d: int, padded: int) -> bool:
-    """Whether the MFMA kernels take a head of this size (widths that are
-    multiples of 128; a 256-row tile of the logits within 2 GiB)."""
-    return rows > 0 and d % 128 == 0 and 512 * padded < (1 << 31) - (1 << 24)
+def head_routes(rows: int, d: int, padded: int) -> tuple[bool, bool]:
+    """Which of the head's products take the MFMA kernels: (logits, gradients).
+    They need a width that is a multiple of 128 and a 256-row tile of the logits
+    within 2 GiB; within that, the side that is faster (us, own / torch's GEMM,
+    operands evicted before each product; widths 128 .. 1024, 64 .. 32768 rows,
+    vocabularies 1000 .. 50257):
+
+    logits     up to width 512, and at any below one round of 256 x 256 tiles:
+               16896 x 256 over 50257 619 / 607, over 10007 149 / 291, 8192 x 512 over
+               50257 498 / 542.  Over a longer reduction the library's tile is the
+               better one: 32768 x 1024 over 50257 3227 / 2878, 8192 x 768 over
+               32000 448 / 372
+    gradients  all but width 384 above 8192 rows, where the 128-column tiles read
+               the logits three times: 24000 x 384 over 32000 1665 / 1228 (dx and dW
+               together); 16896 x 256 over 50257 852 / 1069, 32768 x 1024 5592 / 5976,
+               24000 x 640 over 32000 2123 / 2963, 12288 x 896 1676 / 1727
+    """
+    if rows <= 0 or d % 128 or 512 * padded >= (1 << 31) - (1 << 24):
+        return False, False
+    tiles = -(-rows // 256) * -(-padded // 256)
+    return d <= 512 or tiles <= 256, d != 384 or rows <= 8192
 
 
 def padded_head(weight: torch.Tensor) -> torch.Tensor:

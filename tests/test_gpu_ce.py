@@ -103,13 +103,16 @@ def test_rejects_cpu_and_bad_inputs(cuda_device):
 
 
 @pytest.mark.parametrize("rows,d,vocab", [(1000, 256, 50257), (333, 128, 1001), (64, 256, 64),
-                                           (64, 64, 70001)])
+                                           (64, 64, 70001),
+                                           # the routes of head_routes (own logits, own gradients)
+                                           (5100, 1024, 4001),   # no, yes
+                                           (8200, 384, 1001)])   # yes, no
 def test_tied_head_ce_matches_autograd(cuda_device, rows, d, vocab):
     """The padded-stride head + fused CE (forward and backward in one call;
     two passes above 65536 columns) against autograd of autocast F.linear +
     cross_entropy_sum on the same fp16 operands: the same loss and gradients
-    up to the GEMMs' fp32 accumulation order (the padded logits run other
-    hipBLASLt kernels)."""
+    up to the GEMMs' fp32 accumulation order (the MFMA kernels', or the library's
+    at a padded row stride)."""
     from reversability_amd.kernels import padded_head, tied_head_ce
     g = torch.Generator().manual_seed(5)
     x16 = torch.randn(rows, d, generator=g).half().to(cuda_device)
@@ -372,16 +375,16 @@ def test_tied_head_ce_refuses_other_devices(cuda_device, which):
         tied_head_ce(**args)
 
 
-@pytest.mark.parametrize("vocab", [1001, 70001])
-def test_head_pad_rows_do_not_matter(cuda_device, vocab):
+@pytest.mark.parametrize("rows,d,vocab", [(48, 128, 1001), (48, 128, 70001), (5100, 1024, 4001)])
+def test_head_pad_rows_do_not_matter(cuda_device, rows, d, vocab):
     """Whatever a caller left in the head's pad rows (NaN here), loss and
-    gradients are those of zero pad rows, with the one-pass cross-entropy and
-    the two-pass one of a wide vocabulary."""
+    gradients are those of zero pad rows, with the one-pass cross-entropy, the
+    two-pass one of a wide vocabulary, and torch's product for the logits."""
     from reversability_amd.kernels import padded_head, tied_head_ce
     g = torch.Generator().manual_seed(5)
-    x16 = torch.randn(48, 128, generator=g).half().to(cuda_device)
-    head16 = padded_head((0.05 * torch.randn(vocab, 128, generator=g)).to(cuda_device))
-    labels = torch.randint(0, vocab, (48,), generator=g).to(cuda_device)
+    x16 = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    head16 = padded_head((0.05 * torch.randn(vocab, d, generator=g)).to(cuda_device))
+    labels = torch.randint(0, vocab, (rows,), generator=g).to(cuda_device)
     args = (vocab, labels, torch.ones(1, device=cuda_device))
     clean = tied_head_ce(x16, head16, *args)
     head16[vocab:] = float("nan")

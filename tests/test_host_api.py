@@ -459,3 +459,17 @@ def test_tiled_mlp_records_its_path_on_cpu():
         TiledMLP.apply(x, up, down, 3, False).sum().backward()
     assert paths.report() == {"tiled_mlp": {"torch-gemm": 1}}
     paths.reset()
+
+
+def test_head_routes():
+    """Each of the head's products goes to the side that is faster at its size;
+    sizes the kernels do not take go to torch's GEMMs."""
+    from reversability_amd.kernels import head_routes
+    assert head_routes(16896, 256, 50304) == head_routes(300, 512, 1024) == (True, True)
+    assert head_routes(32768, 1024, 50304) == head_routes(8192, 768, 32000) == (False, True)
+    assert head_routes(64, 1024, 10048) == head_routes(64, 640, 1024) == (True, True)
+    assert head_routes(24000, 384, 32000) == (True, False)
+    assert head_routes(8192, 384, 32000) == (True, True)
+    assert head_routes(12288, 896, 10048) == (False, True)
+    for refused in ((0, 256, 64), (64, 64, 70016), (64, 128, 1 << 22)):
+        assert head_routes(*refused) == (False, False)
