@@ -24,6 +24,7 @@ import types
 import torch
 from torch.autograd.function import once_differentiable
 
+from . import paths
 from ._hip import ops
 
 
@@ -78,7 +79,8 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     rv_ce_fwd / rv_ce_bwd above FUSED_CE_MAX_COLS, same bits); dx = dlogits W and
     dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The
     logits and the two gradients run on the MFMA kernels or on torch's GEMMs
-    (``head_routes``).  ``head16`` is the fp16 head with its rows padded to a
+    (``head_routes``, and operands off a 16-byte boundary; ``paths.report()`` has
+    the sides taken, "mfma", "hipblaslt" or "logits'/gradients'").  ``head16`` is the fp16 head with its rows padded to a
     multiple of VOCAB_ALIGN (the pad rows zero), so every logits row starts
     16-byte aligned.  Returns (loss sum, dx16, dW16 [vocab, d]);
     dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when given, and
@@ -111,6 +113,8 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
                  and (dx_out is None or (dx_out.dtype == torch.float16 and dx_out.is_contiguous()
                                          and dx_out.shape == x16.shape
                                          and dx_out.data_ptr() % 16 == 0)))
+    sides = ["mfma" if own else "hipblaslt" for own in (own_logits, own_grads)]
+    paths.took("tied_head", "fused-ce+" + "/".join(dict.fromkeys(sides)))
     if own_logits:
         logits = torch.empty(rows, padded, device=x16.device, dtype=torch.float16)
         _check(lib.rv_head_logits(x16.data_ptr(), head16.data_ptr(), rows, d, vocab, padded,

@@ -475,10 +475,6 @@ def _cached_head_backward(model, ids, labels, denominator, chunk_tokens, scaler,
     weight = model.lm_head.weight
     if (loss_backend in ("triton", "hip") and precision == "fp16" and ids.device.type == "cuda"
             and weight.dtype == torch.float32):
-        from .kernels import VOCAB_ALIGN, head_routes
-        padded = -(-weight.shape[0] // VOCAB_ALIGN) * VOCAB_ALIGN
-        own = any(head_routes(labels.numel(), weight.shape[1], padded))
-        _paths.took("tied_head", "fused-ce+mfma" if own else "fused-ce+hipblaslt")
         return _fused_head(hidden, weight, labels, denominator, chunk_tokens, scaler, precision,
                            ids.device)
     if loss_backend in ("triton", "hip") and ids.device.type == "cuda":

@@ -412,3 +412,23 @@ def test_head_first_call_does_not_wait(cuda_device):
         busy = not slept.query()
         torch.cuda.synchronize()
         assert busy or i == 0
+
+
+def test_tied_head_records_the_sides_taken(cuda_device):
+    """The record follows the branch, operands' alignment included."""
+    from reversability_amd import paths
+    from reversability_amd.kernels import padded_head, tied_head_ce
+
+    def record(rows, d, vocab, **out):
+        x16 = torch.zeros(rows, d, device=cuda_device, dtype=torch.float16)
+        head16 = padded_head(torch.zeros(vocab, d, device=cuda_device))
+        labels = torch.zeros(rows, device=cuda_device, dtype=torch.int64)
+        paths.reset()
+        tied_head_ce(x16, head16, vocab, labels, torch.ones(1, device=cuda_device), **out)
+        return list(paths.report()["tied_head"])
+
+    assert record(32, 128, 100) == ["fused-ce+mfma"]
+    assert record(32, 64, 100) == ["fused-ce+hipblaslt"]
+    assert record(5100, 1024, 4001) == ["fused-ce+hipblaslt/mfma"]
+    off = torch.empty(100 * 128 + 1, device=cuda_device)[1:].view(100, 128)
+    assert record(32, 128, 100, dw_out=off) == ["fused-ce+mfma/hipblaslt"]
