@@ -56,6 +56,7 @@
 // With lanes 4e..4e+3 addressing 16 consecutive halves of LDS row e, lane i
 // receives column i of rows 0..3: a 4 (k) x 16 (row) block, transposed.
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <map>
@@ -1003,12 +1004,17 @@ int pick_act(int64_t m, int64_t n_cols, bool swiglu, int64_t splits) {
 // output element sums its k blocks in the same order in every shape.  So the
 // first call for each (epilogue and its outputs, operand layouts, m, n, k)
 // times every shape that fits (one warm-up launch, then two timed ones on the
-// caller's stream, which is synchronised after each shape; two sweeps, each
-// shape's faster one counting) and keeps the fastest.  The epilogues tuned
-// here overwrite their outputs, so the extra launches write the same values.
-// A call made while its stream is being captured into a graph never tunes
-// (that would synchronise): it takes the shape already chosen for its key,
-// else pick_act's rule.  RV_GEMM_TUNE=0 in the environment turns tuning off.
+// caller's stream, which is synchronised after each shape), the three fastest
+// of them once more (each shape's faster time counting), and keeps the fastest:
+// at most 30 launches.  64-row tiles are left out of products of four rounds of
+// 256 x 256 tiles and more, where they take 1.4 times the best shape or longer.
+// First forward and backward of an MLP at a new row count, ms (all seven shapes
+// twice -> this): 32768 x 1024 x 4096 85.9 -> 51.9, 3062 x 1024 x 4096 13.0 -> 8.9.  The
+// epilogues tuned here overwrite their outputs, so the extra launches write the
+// same values.  A call made while its stream is being captured into a graph
+// never tunes (that would synchronise): it takes the shape already chosen for
+// its key, else pick_act's rule.  RV_GEMM_TUNE=0 in the environment turns tuning
+// off.
 using TuneKey = std::tuple<int, int, int, int64_t, int64_t, int64_t>;
 std::atomic<int> g_forced_shape{-1};  // rv_gemm_force_shape; -1: measured / rule choice
 std::mutex g_tune_mu;
@@ -1050,11 +1056,19 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
   }
   // two sweeps over the shapes, each shape keeping its faster one: a clock or
   // cache transient during one sweep does not decide the choice alone
+  const int64_t wide = swiglu ? 128 : 256;
+  const bool large = (a.m + 255) / 256 * ((n_cols + wide - 1) / wide) >= 4 * kCUs;
   float ms_of[kNumShapes] = {};
-  for (int sweep = 0; sweep < 2; ++sweep)
+  for (int sweep = 0; sweep < 2; ++sweep) {
+    float first[kNumShapes];
+    std::copy(ms_of, ms_of + kNumShapes, first);
     for (int i = 0; i < kNumShapes; ++i) {
       const int64_t cols = swiglu ? kShapes[i].bn / 2 : kShapes[i].bn;
-      if (n_cols % cols) continue;
+      if (n_cols % cols || (large && kShapes[i].bm == 64)) continue;
+      int faster = 0;  // shapes ahead of this one in the first sweep
+      for (int j = 0; j < kNumShapes; ++j)
+        faster += first[j] > 0.f && (first[i] == 0.f || first[j] < first[i]);
+      if (sweep == 1 && faster >= 3) continue;
       if (launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) != RV_OK) continue;
       bool ok = hipEventRecord(e0, s) == hipSuccess;
       ok = ok && launch_shape<A_RC, B_RC, EPI>(i, a, n_cols, s) == RV_OK;
@@ -1064,6 +1078,7 @@ int tune_act(const GemmArgs& a, int64_t n_cols, hipStream_t s, int fallback) {
       ok = ok && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
       if (ok && ms > 0.f && (ms_of[i] == 0.f || ms < ms_of[i])) ms_of[i] = ms;
     }
+  }
   int best = fallback;
   float best_ms = 0.f;
   for (int i = 0; i < kNumShapes; ++i)

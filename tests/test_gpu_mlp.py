@@ -366,3 +366,23 @@ def test_long_reductions_off_128(cuda_device, rows):
     assert within_gemm_bound(y, a, w, k)
     dx = mlp.dx(a, w.t().contiguous(), torch.empty(rows, d, device=cuda_device))
     assert torch.equal(dx, y.float())
+
+
+def test_first_call_times_at_most_30_launches(cuda_device):
+    """The sweep of tile shapes at a new size: each shape's three launches once,
+    again for the three fastest only."""
+    from torch.profiler import ProfilerActivity, profile
+    g = torch.Generator().manual_seed(37)
+    o = torch.randn(1777, 512, generator=g).half().to(cuda_device)
+    w = (0.02 * torch.randn(256, 512, generator=g)).half().to(cuda_device)
+    out = torch.empty(1777, 256, device=cuda_device, dtype=torch.float16)
+
+    def launches():
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            mlp.down(o, w, out)
+            torch.cuda.synchronize()
+        return sum(e.count for e in prof.key_averages() if "gemm_kernel" in e.key)
+
+    first = launches()
+    assert launches() == 1  # the profiler sees the library's kernels
+    assert 2 <= first <= 31
