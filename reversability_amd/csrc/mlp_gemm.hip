@@ -1181,6 +1181,9 @@ int run_split(GemmArgs a, T* out, float* part, hipStream_t s, int fixed = -1) {
 // 500 the 8192-token tiles' weight gradients kept fewer splits on smaller
 // tiles and took 45.3 us (d 256, f 1024) and 267 us (d 1024, f 4096) against
 // 42.6 and 261 us).
+// A grid past the CU count runs in rounds of all places (CUs times workgroups
+// per CU): 540 workgroups of 64 x 128 tiles, priced as three rounds of the CUs, took
+// 533 us (30791 rows, 6912 x 640) where 270 of 128 x 128 take 364.
 // The split count is the largest that keeps tiles x splits within one round
 // of the CUs: a grid a few workgroups past the CU count (C5's qkv weight
 // gradient: 96 tiles x 3 splits = 288) leaves those CUs a second turn and
@@ -1212,8 +1215,9 @@ bool plan_shape(int i, int64_t rows, int64_t ni, int64_t nj, WgradPlan& plan, do
   int64_t chunk = (rows + splits - 1) / splits;
   chunk = (chunk + kSplitStep - 1) / kSplitStep * kSplitStep;
   splits = (rows + chunk - 1) / chunk;
-  const int64_t wgs = tiles * splits, rounds = (wgs + kCUs - 1) / kCUs;
-  const double fill = (double)wgs / (double)(rounds * kCUs);
+  const int64_t wgs = tiles * splits, places = wgs > kCUs ? kCUs * t.per_cu : kCUs;
+  const int64_t rounds = (wgs + places - 1) / places;
+  const double fill = (double)wgs / (double)(rounds * places);
   const double flops = 2.0 * rows * ni * nj / (eff[i] * fill);
   const double bytes = splits > 1 ? 8.0 * splits * ni * nj : 0.0;
   cost = flops + 250.0 * bytes;
@@ -1225,7 +1229,15 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj, bool ragged = false) 
   WgradPlan best{-1, 0, 0, 0, 0}, plan;
   double best_cost = 0, cost;
   for (int i = 0; i < kRuleShapes; ++i)
-    if (plan_shape(i, rows, ni, nj, plan, cost, ragged) && (best.shape < 0 || cost < best_cost)) {
+    if (plan_shape(i, rows, ni, nj, plan, cost, ragged)) {
+      // alone, 64 x 128 tiles whose number 8 does not divide (tile_of deals them to
+      // the XCDs one by one) rate 0.35 once the operands are past the L2s (4 MB an
+      // XCD): 384 x 384 over 30844 rows 38 us, 128 x 128 tiles 30; 384 x 768 over 16595
+      // 35 and 32, but 896 x 896 over 2093 with qkv's 36 and 41
+      if (i == 3 && !ragged && plan.tiles_m * plan.tiles_n % 8 &&
+          rows * (ni + nj) * 2 > (int64_t)16 << 20)
+        cost *= 0.42 / 0.35;
+      if (best.shape >= 0 && cost >= best_cost) continue;
       best = plan;
       best_cost = cost;
     }
@@ -1235,21 +1247,37 @@ WgradPlan plan_wgrad(int64_t rows, int64_t ni, int64_t nj, bool ragged = false) 
 // The plans of two weight gradients over the same rows (a: ai x aj, b: bi x
 // bj).  With one tile shape for both they share a launch (launch_pair): the
 // shape with the least total cost among those whose two plans are both split
-// or both not.
+// or both not, as long as that is no more than kPairCost of what the two cost
+// with a shape each.  (Each cost is of the product alone: two workgroups per CU
+// fill places that each product leaves idle.  256 x 256 tiles run one per CU, and
+// share a launch only where they are both products' own shape.)  Measured, us,
+// joint / apart, by the ratio of the costs: 1.00 23.9 / 27.8 (3483 rows, d 128, f
+// 3584), 1.21 34.3 / 47.2 (2845, 384, 2944), 1.35 32.8 / 45.7 (3000, 768, 1408); 1.44
+// 350 / 268 (19018, 768, 2432), 1.93 20.2 / 16.3 (307, 896, 768), 2.36 372 / 287 (32768,
+// 768, 1408); 256 x 256 tiles 1.18 78.6 / 64.5 (4325 rows, qkv and proj of 1024).  Over
+// 164 pairs, against two launches with a plan each of the fixed 0.35 weighting
+// this one replaced: 0.71 on average and none above 1.0 (without a line 0.73, worst
+// 1.40).
+constexpr double kPairCost = 1.4;
 struct PairPlan {
   WgradPlan a, b;
   bool paired;
 };
 PairPlan plan_pair(int64_t rows, int64_t ai, int64_t aj, int64_t bi, int64_t bj) {
   PairPlan best{plan_wgrad(rows, ai, aj), plan_wgrad(rows, bi, bj), false};
-  double best_cost = 0, ca, cb;
+  if (best.a.shape < 0 || best.b.shape < 0) return best;
+  double least = 0, ca, cb;
   WgradPlan a, b;
+  plan_shape(best.a.shape, rows, ai, aj, a, ca);
+  plan_shape(best.b.shape, rows, bi, bj, b, cb);
+  const double apart = ca + cb;
   for (int i = 0; i < kRuleShapes; ++i) {
     if (!plan_shape(i, rows, ai, aj, a, ca) || !plan_shape(i, rows, bi, bj, b, cb)) continue;
     if ((a.splits > 1) != (b.splits > 1)) continue;
-    if (!best.paired || ca + cb < best_cost) {
+    if (ca + cb > (kShapes[i].per_cu > 1 ? kPairCost : 1.0) * apart) continue;
+    if (!best.paired || ca + cb < least) {
       best = PairPlan{a, b, true};
-      best_cost = ca + cb;
+      least = ca + cb;
     }
   }
   return best;

@@ -167,6 +167,18 @@ def test_gemm_entry_points_validate_without_device():
     assert lib.rv_linear_dw(fake, fake, 256, rows, 256, 768, odd, 0, fake, 1 << 30, None) == 3
 
 
+@pytest.mark.parametrize("rows,d,f,joint", [(3000, 768, 1408, True), (1121, 384, 1408, True),
+                                            (32768, 768, 1408, False), (307, 896, 768, False)])
+def test_paired_weight_gradients_share_a_launch_only_where_it_is_cheaper(rows, d, f, joint):
+    """Two weight gradients whose own plans cost far less than any common tile
+    shape keep them: the workspace is that of the two plans side by side."""
+    lib = _hip.library()
+    up = lib.rv_linear_dw_workspace_bytes(rows, d, 2 * f)
+    down = lib.rv_linear_dw_workspace_bytes(rows, f, d)
+    apart = up + (-(-down // 256) * 256 if up else down)
+    assert (lib.rv_mlp_wgrad_workspace_bytes(rows, d, f) == apart) != joint
+
+
 def test_fused_cross_entropy_validates_without_device():
     lib = _hip.library()
     fake = ctypes.c_void_p(4096)

@@ -315,10 +315,10 @@ def test_depths_off_the_stage_length(cuda_device, rows, d):
 
 
 @pytest.mark.parametrize("rows", [1, 64, 129, 300, 1025])
-@pytest.mark.parametrize("d,f", [(128, 128), (384, 1664), (1024, 4096)])
+@pytest.mark.parametrize("d,f", [(128, 128), (384, 1664), (1024, 4096), (896, 768)])
 def test_wgrad_pair_plans(cuda_device, rows, d, f):
-    """Both weight gradients in one launch: split and unsplit plans, uneven
-    tile counts of the two, and token counts around a split's granularity
+    """Both weight gradients in one launch, or in two (896 x 768 at 300 rows):
+    split and unsplit plans, uneven tile counts of the two, and token counts around a split's granularity
     (64); the fp64 bound, and the accumulating call adds the same values."""
     g = torch.Generator().manual_seed(41)
     dy = torch.randn(rows, d, generator=g).half().to(cuda_device)
