@@ -36,6 +36,9 @@ constexpr int64_t kChunk = 16384;
 // 16384 551 / 20, 4096 519 / 12, 1024 545 / 15 with two double pow per thread, 470 /
 // 16.5 with one exp2 each).
 constexpr int64_t kUpdateChunk = kThreads * 4;
+// Update workgroups per grid row: a launch dimension holds fewer than 2^32
+// threads, which one row of 2^24 workgroups (17.2 G parameters) would pass.
+constexpr int kGridRow = 1 << 22;
 
 struct TensorTable {
   float* p[kMaxTensors];
@@ -110,8 +113,10 @@ template <bool LOAD_NT, bool STORE_NT>
 __global__ __launch_bounds__(kThreads)
 void adamw_k(TensorTable tab, Hyper h) {
   if (h.found_inf != nullptr && *h.found_inf != 0.0f) return;  // uniform skip
-  const int t = tensor_of(tab.chunk_start, tab.count, (int)blockIdx.x);
-  const int64_t off = (int64_t)(blockIdx.x - tab.chunk_start[t]) * kUpdateChunk;
+  const int64_t block = (int64_t)blockIdx.y * kGridRow + blockIdx.x;
+  if (block >= tab.chunk_start[tab.count]) return;  // past the last row's end
+  const int t = tensor_of(tab.chunk_start, tab.count, (int)block);
+  const int64_t off = (block - tab.chunk_start[t]) * kUpdateChunk;
   const int64_t end = off + kUpdateChunk < tab.n[t] ? off + kUpdateChunk : tab.n[t];
   float* p = tab.p[t];
   const float* g = tab.g[t];
@@ -408,7 +413,9 @@ int rv_adamw_step_clipped(int count, float* const* params, const float* const* g
   h.found_inf = found_inf;
   h.inv_scale = inv_scale;
   h.clip = clip_coef;
-  const dim3 grid((unsigned)chunks), block(kThreads);
+  const dim3 grid((unsigned)(chunks < kGridRow ? chunks : kGridRow),
+                  (unsigned)((chunks + (int64_t)kGridRow - 1) / kGridRow));
+  const dim3 block(kThreads);
   const hipStream_t s = (hipStream_t)stream;
   if (bytes > kStreamStoreBytes)
     hipLaunchKernelGGL((adamw_k<true, true>), grid, block, 0, s, tab, h);

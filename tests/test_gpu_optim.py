@@ -238,3 +238,18 @@ def test_update_by_size_of_the_arrays(cuda_device, numel):
         assert _close(b.detach(), a.detach())
     sa, sb = ta.state[a], fb.state[b]
     assert _close(sb["exp_avg"], sa["exp_avg"]) and _close(sb["exp_avg_sq"], sa["exp_avg_sq"])
+
+
+@pytest.mark.parametrize("numel", [(1 << 34) - 1024, (1 << 34) + 1, 19_000_000_000])
+def test_update_past_one_grid_row(cuda_device, numel):
+    """Parameters enough for more workgroups than one launch dimension holds are
+    accepted: a step whose overflow flag is set, in which no workgroup touches
+    memory (the pointers are never read)."""
+    import ctypes
+    from reversability_amd._hip import _stream, library
+    flag, step = torch.ones(1, device=cuda_device), torch.ones(1, device=cuda_device)
+    fake = (ctypes.c_void_p * 1)(4096)
+    sizes = (ctypes.c_int64 * 1)(numel)
+    assert library().rv_adamw_step(1, fake, fake, fake, fake, sizes, 1e-3, 0.9, 0.95, 1e-8, 0.1,
+                                   step.data_ptr(), flag.data_ptr(), None, _stream(flag)) == 0
+    torch.cuda.synchronize()
