@@ -32,9 +32,9 @@ constexpr int kMaxTensors = 48;
 constexpr int64_t kChunk = 16384;
 // Elements per workgroup of the update: one pass, so that consecutive
 // workgroups, and the HBM pages they touch in the seven streams, stay close
-// together (update alone, us, 103.9 M / 2.0 M parameters: 65536 elements 589 / -,
-// 16384 551 / 20, 4096 519 / 12, 1024 545 / 15 with two double pow per thread, 470 /
-// 16.5 with one exp2 each).
+// together (update alone, nothing evicted, us, 103.9 M / 2.0 M parameters: 65536
+// elements 589 / -, 16384 551 / 20, 4096 519 / 12, 1024 545 / 15 with two double pow per
+// thread, 480 / 10.9 with one exp2 each).
 constexpr int64_t kUpdateChunk = kThreads * 4;
 // Update workgroups per grid row: a launch dimension holds fewer than 2^32
 // threads, which one row of 2^24 workgroups (17.2 G parameters) would pass.
@@ -158,7 +158,7 @@ void adamw_k(TensorTable tab, Hyper h) {
 }
 
 // Gradient-norm pass of GradScaler.unscale_ + clip_grad_norm_(p, max_norm, 2):
-// per chunk of one tensor (same table and chunking as the update) the fp32 sum
+// per chunk of kChunk elements of one tensor the fp32 sum
 // of squares of the unscaled gradient g * inv (the value unscale_ would write)
 // and whether any unscaled element is non-finite.  Fixed summation order:
 // each thread its elements in order, then a wave butterfly, then the waves in
@@ -290,13 +290,15 @@ void grad_clip_k(const float* __restrict__ part, const float* __restrict__ flag,
 }
 
 // Cache hints by the bytes of the four arrays (16 per parameter), against the
-// 256 MB Infinity Cache.  Norm pass and update, us, with everything else evicted
-// before each call, at 16384 elements per workgroup (plain / streamed loads /
-// loads and stores; 32 MB also with nothing evicted): 32 MB 36 / 32 / 32 (24 / 26 /
-// 28), 325 MB 122 / 109 / 120, 430 MB 118 / 106 / 113, 1.66 GB 652 / 624 / 605 (656 /
-// 646 / 568: the gradients then stay cached between the two passes).
+// 256 MB Infinity Cache.  Norm pass and update, us, plain / streamed loads / loads
+// and stores, with everything else evicted before each call (with nothing
+// evicted): 31 MB 22.6 / 20.7 / 20.0 (15.2 / 15.7 / 15.8), 122 MB 59.0 / 56.0 / 53.2 (43.2 /
+// 43.4 / 45.0), 310 MB 131 / 129 / 121 (105 / 102 / 101), 504 MB 209 / 204 / 190 (193 / 177 /
+// 154), 1.6 GB 625 / 598 / 603 (614 / 589 / 548).  Streamed stores cost 4% where the
+// arrays would have stayed cached, so they start where these no longer fit;
+// streamed loads cost 1% there and save 5% where they would not have.
 constexpr int64_t kStreamLoadBytes = int64_t(64) << 20;
-constexpr int64_t kStreamStoreBytes = int64_t(512) << 20;
+constexpr int64_t kStreamStoreBytes = int64_t(256) << 20;
 
 __global__ void adamw_advance_k(float* step, const float* found_inf) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {

@@ -216,7 +216,7 @@ def test_clip_without_scaler(cuda_device):
 
 @pytest.mark.parametrize("numel", [1023, 16384 * 3 + 5, 5_000_003, 36_000_001])
 def test_update_by_size_of_the_arrays(cuda_device, numel):
-    """Tensors on both sides of the update's streaming thresholds (64 MB and 512
+    """Tensors on both sides of the update's streaming thresholds (64 MB and 256
     MB of the four arrays) and off the vector and chunk lengths: two steps of
     unscale_clip_ + step equal torch's clip and AdamW to the bar above, and
     the norm to 1e-6."""
