@@ -44,6 +44,8 @@ def cast_f16(t: torch.Tensor) -> torch.Tensor:
     if t.dtype != torch.float32 or not t.is_contiguous():
         raise ValueError("cast_f16 needs a contiguous fp32 or fp16 CUDA (ROCm device) tensor")
     out = torch.empty(t.shape, device=t.device, dtype=torch.float16)
+    if not t.numel():  # no memory to point at
+        return out
     _check(library().rv_cast_f32_f16(t.data_ptr(), out.data_ptr(), t.numel(), _stream(t)),
            "rv_cast_f32_f16")
     return out

@@ -177,7 +177,9 @@ class TiledMLP(torch.autograd.Function):
                 x16, (up16, down16) = mlp.cast_f16(flat.contiguous()), cast
             else:  # the forward computed nothing (need_output=False)
                 x16, up16, down16 = mlp.cast_operands(flat.contiguous(), up, down)
-            dup, ddown = torch.empty_like(up), torch.empty_like(down)
+            # written by the first tile; without rows there is none
+            new = torch.empty_like if flat.shape[0] else torch.zeros_like
+            dup, ddown = new(up), new(down)
             tiles, ctx.tiles = ctx.tiles, None
             whole = flat.shape[0] <= ctx.tokens  # one tile: no slices
             for i, start in enumerate(range(0, flat.shape[0], ctx.tokens)):

@@ -386,3 +386,19 @@ def test_first_call_times_at_most_30_launches(cuda_device):
     first = launches()
     assert launches() == 1  # the profiler sees the library's kernels
     assert 2 <= first <= 31
+
+
+@pytest.mark.parametrize("xdtype", [torch.float16, torch.float32])
+def test_tiled_mlp_without_rows(cuda_device, xdtype):
+    """No tokens: an empty output and zero weight gradients, whatever the
+    allocator's memory held."""
+    from reversability_amd.optimized_v3 import TiledMLP
+    up, down = (w.requires_grad_(True) for w in weights(128, 256, cuda_device))
+    x = torch.empty(2, 0, 128, device=cuda_device, dtype=xdtype, requires_grad=True)
+    used = [torch.full_like(w, float("nan")) for w in (up, down)]
+    del used
+    with torch.autocast("cuda", dtype=torch.float16):
+        y = TiledMLP.apply(x, up, down, 64, True)
+    dx, dup, ddown = torch.autograd.grad(y, (x, up, down), torch.empty_like(y))
+    assert y.shape == dx.shape == x.shape
+    assert not dup.any() and not ddown.any()
