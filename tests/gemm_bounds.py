@@ -13,6 +13,10 @@ from __future__ import annotations
 
 import torch
 
+# Output columns of each tile shape that rv_gemm_force_shape takes: a product whose
+# width they do not divide is refused (RV_ERR_UNSUPPORTED, 3).
+TILE_WIDTHS = (256, 256, 128, 128, 256, 128, 128)
+
 
 def fp16_ulp(t: torch.Tensor) -> torch.Tensor:
     """Spacing of fp16 at |t| (2^-24 below the normal range), on t's device."""

@@ -103,7 +103,7 @@ def test_rejects_cpu_and_bad_inputs(cuda_device):
 
 
 @pytest.mark.parametrize("rows,d,vocab", [(1000, 256, 50257), (333, 128, 1001), (64, 256, 64),
-                                           (64, 64, 70001),
+                                           (64, 64, 70001), (64, 128, 70001),
                                            # the routes of head_routes (own logits, own gradients)
                                            (5100, 1024, 4001),   # no, yes
                                            (8200, 384, 1001)])   # yes, no
@@ -122,6 +122,10 @@ def test_tied_head_ce_matches_autograd(cuda_device, rows, d, vocab):
     grad = torch.tensor([0.37], device=cuda_device)
     head16 = padded_head(w)
     assert head16.shape[0] % 64 == 0 and torch.equal(head16[vocab:], torch.zeros_like(head16[vocab:]))
+    # memory that the call's buffers take over (the logits' pad columns among them)
+    used = [torch.full((rows, head16.shape[0]), float("nan"), device=cuda_device,
+                       dtype=torch.float16) for _ in range(2)]
+    del used
     loss, dx16, dw16 = tied_head_ce(x16, head16, vocab, labels, grad)
     xr = x16.clone().requires_grad_(True)
     hr = w.half().requires_grad_(True)
@@ -253,9 +257,10 @@ def test_head_products(cuda_device, rows, d, vocab):
     multiple of the tiles: the fp64 bound, identical bits on every tile shape,
     pad columns zero also for a row of infinities, dW as fp16, widened, and
     accumulated, from one workspace."""
-    from gemm_bounds import within_gemm_bound
+    from gemm_bounds import TILE_WIDTHS, within_gemm_bound
     from reversability_amd._hip import RV_F16, RV_F32, _stream, library
     lib = library()
+    assert lib.rv_gemm_num_shapes() == len(TILE_WIDTHS)
     padded = -(-vocab // 64) * 64
     g = torch.Generator().manual_seed(19)
     x = torch.randn(rows, d, generator=g).half().to(cuda_device)
@@ -280,10 +285,10 @@ def test_head_products(cuda_device, rows, d, vocab):
                                       st) == 0
             rc = lib.rv_head_dx(grad.data_ptr(), head.data_ptr(), *size, dx.data_ptr(),
                                 ws.data_ptr(), nbytes, st)
-            if rc == 3 and shape >= 0:  # d does not divide this tile
+            fits = shape < 0 or d % TILE_WIDTHS[shape] == 0
+            assert rc == (0 if fits else 3), shape
+            if not fits:  # refused: only the logits are compared
                 dx = first[1]
-            else:
-                assert rc == 0
             if first is None:
                 first = (logits, dx)
                 assert within_gemm_bound(logits, x, head, d)
@@ -432,3 +437,28 @@ def test_tied_head_records_the_sides_taken(cuda_device):
     assert record(5100, 1024, 4001) == ["fused-ce+hipblaslt/mfma"]
     off = torch.empty(100 * 128 + 1, device=cuda_device)[1:].view(100, 128)
     assert record(32, 128, 100, dw_out=off) == ["fused-ce+mfma/hipblaslt"]
+
+
+@pytest.mark.parametrize("offset", [0, 1])  # floats: the kernels' route, and torch's off 16 bytes
+def test_tied_head_ce_accumulates_over_chunks(cuda_device, offset):
+    """Two chunks whose dW is written, then added, into one fp32 tensor: each
+    chunk's own fp16 gradient widened, and their sum."""
+    from reversability_amd.kernels import padded_head, tied_head_ce
+    rows, d, vocab = 300, 128, 1001
+    g = torch.Generator().manual_seed(13)
+    x16 = torch.randn(rows, d, generator=g).half().to(cuda_device)
+    head16 = padded_head((0.05 * torch.randn(vocab, d, generator=g)).to(cuda_device))
+    labels = torch.randint(0, vocab, (rows,), generator=g).to(cuda_device)
+    grad = torch.tensor([0.37], device=cuda_device)
+    out = torch.full((vocab * d + 4,), float("nan"), device=cuda_device)
+    dw = out[offset:offset + vocab * d].view(vocab, d)
+    total = None
+    for i, part in enumerate((slice(0, 170), slice(170, rows))):
+        args = (x16[part], head16, vocab, labels[part], grad)
+        *_, alone = tied_head_ce(*args, dw_out=torch.empty(out.shape, device=cuda_device)[
+            offset:offset + vocab * d].view(vocab, d))
+        *_, got = tied_head_ce(*args, dw_out=dw, accumulate=i > 0)
+        total = alone if total is None else total + alone
+        assert got is dw and torch.equal(alone, alone.half().float())
+        assert torch.equal(dw, total)
+    assert torch.isnan(out[:offset]).all() and torch.isnan(out[offset + vocab * d:]).all()

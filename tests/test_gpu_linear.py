@@ -11,7 +11,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from gemm_bounds import rel_l2, within_gemm_bound
+from gemm_bounds import TILE_WIDTHS, rel_l2, within_gemm_bound
 from reversability_amd import mlp
 from reversability_amd._hip import RV_F16, RV_F32, _check, _stream, library
 from reversability_amd.linear import FusedLinear, enable_linear, linear, supported
@@ -131,8 +131,8 @@ def test_split_reduction(cuda_device, rows, in_f, out_f):
             for dx, code in ((d16, RV_F16), (d32, RV_F32)):
                 codes.append(lib.rv_linear_dx_ws(x.data_ptr(), wt.data_ptr(), rows, out_f, in_f,
                                                  dx.data_ptr(), code, *args))
-            if shape >= 0 and codes[0] == 3:  # the width does not divide this tile
-                assert codes == [3, 3, 3]
+            if shape >= 0 and out_f % TILE_WIDTHS[shape]:
+                assert codes == [3, 3, 3], shape
                 continue
             assert codes == [0, 0, 0], shape
             if first is None:
