@@ -80,7 +80,10 @@ class AttentionLayer(torch.autograd.Function):
     autograd node: the same kernels on the same values as ``FusedLinear``,
     ``CausalAttention`` and ``FusedLinear`` in turn, with one launch for the
     operand casts and one for the two weight gradients (reduced over the
-    rows in another fixed order than each alone)."""
+    rows in another fixed order than each alone).  The weights' fp16 casts live
+    from forward to backward (2 bytes per weight), and qkv, its log-sum-exp and the
+    attention output to the end of the backward, where three nodes free them one
+    after the other (8 bytes per token and column more at the input gradient)."""
 
     @staticmethod
     def forward(ctx, x, w_qkv, w_proj, heads):

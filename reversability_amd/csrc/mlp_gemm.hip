@@ -212,8 +212,8 @@ struct Dma {
     }
   }
   // A KC row's last stage holds `valid` < BK values of the reduction: chunks
-  // at or past it are sent out of the resource's range (2 GiB > the largest
-  // operand the entry points accept) and read as zero.
+  // at or past it are sent out of the resource's range and read as zero (stage()
+  // gives it at most INT32_MAX bytes, whatever the operand's size).
   __device__ __forceinline__ void cut_kc(int valid, int wave, int lane) {
 #pragma unroll
     for (int it = 0; it < kPerWave; ++it) {
