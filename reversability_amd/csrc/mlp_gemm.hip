@@ -1433,16 +1433,17 @@ int64_t head_dx_bytes(int64_t rows, int64_t d, int64_t k) {
 // row count may change from call to call, and a sweep of both made the first
 // call at a row count 60 ms (16896 x 256 over 50257) where a call takes 2.1.  The
 // lines (kShapes' indices) are from all shapes timed at widths 128 .. 2048, 64 .. 32768
-// rows and vocabularies 1000 .. 50257, the operands evicted before each product:
+// rows and vocabularies 1000 .. 50257, with the operands evicted before each
+// product (figures marked c: still cached):
 //   logits  4 (eight waves) is the fastest or within 5% of it once its tiles fill
 //           the CUs four times (16896 x 256 over 50257: 619 us, the others 670-999);
 //           1 at d = 128, where two workgroups per CU hide the epilogues of a
 //           short k loop, and below that number of tiles if 8 divides its own
-//           (tile_of: 24000 x 256 over 3000 49 against 57, but 1500 x 512 over 32000 87
-//           against 70); 2 and 3 below one and a half rounds, as pick_act
+//           (tile_of: c 24000 x 256 over 3000 49 against 57, but 1500 x 512 over 32000
+//           87 against 70); 2 and 3 below one and a half rounds, as pick_act
 //   dx      where act_splits splits, 3 as long as its workgroups fill one round of
-//           the CUs (1000 x 512 over 50257: 81 us, 5 takes 116) and 5 past it (300 x
-//           768: 67, 3 takes 99); 0 (2 at odd multiples of 128) over a long
+//           the CUs (c 1000 x 512 over 50257: 81 us, 5 takes 116) and 5 past it (c 300
+//           x 768: 67, 3 takes 99); 0 (2 at odd multiples of 128) over a long
 //           reduction, else as pick_act with 3 below one round
 int head_logits_shape(int64_t rows, int64_t d, int64_t padded) {
   const auto tiles = [&](int i) {
