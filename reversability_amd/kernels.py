@@ -77,15 +77,15 @@ def tied_head_ce(x16: torch.Tensor, head16: torch.Tensor, vocab: int, labels: to
     gradient ``grad`` (a device fp32 scalar): logits = fp16(x16 W^T); loss and
     dlogits from one pass of rv_ce_fused over each logits row (the two-pass
     rv_ce_fwd / rv_ce_bwd above FUSED_CE_MAX_COLS, same bits); dx = dlogits W and
-    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The
-    logits and the two gradients run on the MFMA kernels or on torch's GEMMs
-    (``head_routes``, and operands off a 16-byte boundary; ``paths.report()`` has
-    the sides taken, "mfma", "hipblaslt" or "logits'/gradients'").  ``head16`` is the fp16 head with its rows padded to a
-    multiple of VOCAB_ALIGN (the pad rows zero), so every logits row starts
-    16-byte aligned.  Returns (loss sum, dx16, dW16 [vocab, d]);
-    dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when given, and
-    dW -- the same fp16 values widened -- into ``dw_out`` (contiguous fp32 [vocab,
-    d]; added to it with ``accumulate``), which is then returned for dW16.
+    dW = dlogits^T x16 (fp16, as autocast's linear produces them).  The logits and
+    the two gradients run on the MFMA kernels or on torch's GEMMs (``head_routes``,
+    and operands off a 16-byte boundary; ``paths.report()`` has the sides taken,
+    "mfma", "hipblaslt" or the logits' and the gradients').  ``head16`` is the fp16
+    head with its rows padded to a multiple of VOCAB_ALIGN (as ``padded_head`` makes
+    it), so every logits row starts 16-byte aligned.  Returns (loss sum, dx16, dW16
+    [vocab, d]); dx16 is written into ``dx_out`` (contiguous fp16 [rows, d]) when
+    given, and dW -- the same fp16 values widened -- into ``dw_out`` (contiguous fp32
+    [vocab, d]; added to it with ``accumulate``), which is then returned for dW16.
     """
     rows, d = x16.shape
     padded = head16.shape[0]
