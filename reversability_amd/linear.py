@@ -11,6 +11,8 @@ fp16 product widened to the input's dtype, ``dW`` as the fp16 product widened
 to fp32 -- with the gfx950 GEMM kernels of ``csrc/mlp_gemm.hip``
 (``rv_linear_fwd``, ``rv_linear_dx``, ``rv_linear_dw``; the weight gradient
 reduces over all tokens in a fixed order, split-K when the output is small).
+The weight's fp16 cast is made in the forward and kept for the backward (2 bytes
+per weight while the graph lives).
 
 ``enable_linear(model)`` patches every block's ``attn.qkv`` and ``attn.proj``;
 calls the kernels do not cover (no fp16 autocast, a bias, widths that are not
